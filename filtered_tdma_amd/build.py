@@ -20,8 +20,8 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libftdma.so")
 SOURCES = [os.path.join(CSRC, "ftdma_kernels.hip"), os.path.join(CSRC, "ftdma_api.cpp"),
-           os.path.join(CSRC, "ftdma_heat.hip"), os.path.join(CSRC, "ftdma_batched.hip"),
-           os.path.join(CSRC, "ftdma_poisson.hip")]
+           os.path.join(CSRC, "ftdma_lines.hip"), os.path.join(CSRC, "ftdma_heat.hip"),
+           os.path.join(CSRC, "ftdma_batched.hip"), os.path.join(CSRC, "ftdma_poisson.hip")]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 

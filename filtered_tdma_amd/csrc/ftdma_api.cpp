@@ -166,33 +166,59 @@ bool shape_for(int M, int T, int Q, int n_row, int forced_S, FusedShape& out) {
     return true;
 }
 
-bool pick_pascal(const ftd_handle* h, int n_row, int cyclic, FusedShape& out, int csh = 0) {
+// (M, T) in order of preference, fastest first at 262144 x 512
+constexpr int kMs[] = {64, 32, 32, 16, 8};
+constexpr int kTs[] = {256, 512, 256, 512, 512};
+
+// the shape that keeps the caller's P > 1 partitions (smallest M that holds
+// them, at least 16 systems per workgroup)
+bool caller_shape(const ftd_handle* h, int n_row, FusedShape& out) {
+    const int P = h->P;
+    if (P < 2) return false;
+    int s_, m_max;
+    part_of(n_row, P, 0, s_, m_max);
+    bool found = false;
+    for (int k = 0; k < 5; ++k) {
+        FusedShape fs;
+        if (kMs[k] >= m_max && (!found || kMs[k] < out.M) &&
+            shape_for(kMs[k], kTs[k], P, n_row, 0, fs) && fs.S >= 16) {
+            out = fs;
+            found = true;
+        }
+    }
+    return found;
+}
+
+// the fused shape of `Q` partitions, whatever its systems per workgroup
+bool fused_of(int Q, int n_row, FusedShape& out) {
+    for (int k = 4; k >= 0; --k)
+        if (shape_for(kMs[k], kTs[k], Q, n_row, 0, out)) return true;
+    return false;
+}
+
+// Partitions and tile of a real exact solve whose partitions the engine
+// chooses, above 512 rows; out.M == 0: the long-system streamed kernel (Q and
+// S set). Both sides of each line in us:
+//  * above 512 rows the streamed long-system kernel (66049 x 768: 562 against
+//    609; 131104 x 1024: 1081 against 1125); with fewer than two 16-system
+//    tiles per CU and up to 1024 rows, 32-row lanes (2048 x 768: 23.3 against
+//    26.7).
+bool own_shape(int n_sys, int n_row, FusedShape& out) {
+    if (n_row <= 512) return false;
+    const int S = ftd::lines_systems(n_sys, n_row);
+    if (n_row <= 1024 && n_sys < 8192)
+        return shape_for(32, 512, (n_row + 31) / 32, n_row, 16, out);
+    if (!S) return false;
+    out = FusedShape{0, 0, S, 256 / S};
+    return true;
+}
+
+bool pick_pascal(const ftd_handle* h, int n_row, FusedShape& out, int csh = 0) {
     if (h->t_M) {
         int Q = h->t_Q ? h->t_Q : std::max(2, (n_row + h->t_M - 1) / h->t_M);
         return shape_for(h->t_M, h->t_T ? h->t_T : 256, Q, n_row, h->t_S, out);
     }
-    // (M, T) in order of preference, fastest first at 262144 x 512
-    static const int Ms[] = {64, 32, 32, 16, 8};
-    static const int Ts[] = {256, 512, 256, 512, 512};
-    const int P = h->P;
-    if (P > 1) {
-        int s_, m_max;
-        part_of(n_row, P, 0, s_, m_max);
-        for (int k = 0; k < 5; ++k) {
-            if (Ms[k] < m_max) continue;
-            FusedShape fs;
-            if (shape_for(Ms[k], Ts[k], P, n_row, 0, fs) && fs.S >= 16) {
-                // smallest M that holds the partitions
-                out = fs;
-                for (int k2 = 0; k2 < 5; ++k2)
-                    if (Ms[k2] >= m_max && Ms[k2] < out.M && shape_for(Ms[k2], Ts[k2], P, n_row, 0, fs) &&
-                        fs.S >= 16)
-                        out = fs;
-                return true;
-            }
-        }
-    }
-    (void)cyclic;
+    if (caller_shape(h, n_row, out)) return true;
     if (csh || n_row > 8 * 64) {
         // complex right-hand sides, one caller partition: 32-row partitions
         // in 512-thread workgroups measured fastest (16384 x 129 and
@@ -208,9 +234,9 @@ bool pick_pascal(const ftd_handle* h, int n_row, int cyclic, FusedShape& out, in
         }
     }
     for (int k = 0; k < 5; ++k) {
-        const int Q = std::max(2, (n_row + Ms[k] - 1) / Ms[k]);
+        const int Q = std::max(2, (n_row + kMs[k] - 1) / kMs[k]);
         FusedShape fs;
-        if (shape_for(Ms[k], Ts[k], Q, n_row, 0, fs) && fs.S >= 16) {
+        if (shape_for(kMs[k], kTs[k], Q, n_row, 0, fs) && fs.S >= 16) {
             out = fs;
             return true;
         }
@@ -238,12 +264,26 @@ ftd_status solve_exact(ftd_handle* h, double* A, double* B, double* C, double* D
         }
         return FTD_OK;
     }
-    if (!h->force_general && n_row >= 3 && pick_pascal(h, n_row, cyclic, fs, csh)) {
+    // Real systems whose partitions the engine chooses (one caller partition,
+    // or more rows in one than a lane holds). Without the streamed kernels
+    // (set_tuning -2) the fused kernel runs the same partitions.
+    const bool own = !h->force_general && !h->t_M && !csh && n_row >= 3 &&
+                     !caller_shape(h, n_row, fs) && own_shape(n_sys, n_row, fs);
+    const int Sl = own && !fs.M ? fs.S : 0;
+    if (Sl && !h->no_stream) {
+        std::snprintf(h->path, sizeof h->path, "pascal_stream M=64 Q=%d R=4 S=%d", fs.Q, Sl);
+        FTD_LAUNCH(ftd::launch_pascal_lines(Sl, A, B, C, D, n_sys, n_row, cyclic, st));
+        return FTD_OK;
+    }
+    if (Sl) fused_of(256 / Sl, n_row, fs);
+    if (!h->force_general && n_row >= 3 && (own || pick_pascal(h, n_row, fs, csh))) {
         // the streamed kernel runs the same partitioning (bit-identical
         // results) where a variant holds it and the arrays allow its DMA
         int s_, m_max;
         part_of(n_row, fs.Q, 0, s_, m_max);
-        const int Ms = (h->t_M || h->no_stream || csh) ? 0 : ftd::stream_rows(m_max, fs.Q);
+        const int Ms = (h->t_M || h->no_stream || csh || (own && fs.M < 64))
+                           ? 0
+                           : ftd::stream_rows(m_max, fs.Q);
         if (Ms && ftd::stream_eligible(n_sys, A, B, C, D)) {
             std::snprintf(h->path, sizeof h->path, "pascal_stream M=%d Q=%d R=%d", Ms, fs.Q,
                           ftd::stream_ring_depth(Ms, fs.Q));
@@ -848,7 +888,7 @@ static ftd_status solve_f32_common(ftd_handle* h, const float* A, const float* B
         return fail(FTD_ERR_UNSUPPORTED, "FP32 storage is available for the exact (PaScaL) solve");
     if (h->n_sys == 0) return FTD_OK;
     FusedShape fs;
-    if (h->n_row < 6 || !pick_pascal(h, h->n_row, 0, fs))
+    if (h->n_row < 6 || !pick_pascal(h, h->n_row, fs))
         return fail(FTD_ERR_UNSUPPORTED, "no fused kernel holds this system for FP32 storage");
     if (h->profiling) FTD_HIP(hipEventRecord(h->ev0, h->stream));
     // FP32 A, B, C, D: the streamed kernel runs the same partitions (same
@@ -903,7 +943,7 @@ ftd_status ftd_solve_f32_refine(ftd_handle* h, const float* A, const float* B, c
         return fail(FTD_ERR_UNSUPPORTED, "FP32 storage is available for the exact (PaScaL) solve");
     if (h->n_sys == 0) return FTD_OK;
     FusedShape fs;
-    if (h->n_row < 6 || !pick_pascal(h, h->n_row, 0, fs))
+    if (h->n_row < 6 || !pick_pascal(h, h->n_row, fs))
         return fail(FTD_ERR_UNSUPPORTED, "no fused kernel holds this system for FP32 storage");
     if (h->profiling) FTD_HIP(hipEventRecord(h->ev0, h->stream));
     std::snprintf(h->path, sizeof h->path, "pascal_ir M=%d T=%d S=%d Q=%d sweeps=%d", fs.M, fs.T,

@@ -68,6 +68,18 @@ hipError_t launch_filtered_stream(int M, int Q, int version, int pass, const dou
                                   double* partial, double eps_value, int eps_direct, int* Jsys,
                                   int guard, hipStream_t st);
 
+// Workgroups of `kernel` resident on the whole device at once, at most
+// n_tiles: the grid of the persistent kernels
+int resident_grid(const void* kernel, int threads, int n_tiles);
+
+// Streamed exact solve of 513 to 4096 rows over the engine's own 256 / S
+// partitions, S = 16, 8 or 4 systems per tile: the S for these sizes, 0
+// where none holds them (n_sys >= 2). The arrays need no more than their
+// elements' alignment.
+int lines_systems(int n_sys, int n_row);
+hipError_t launch_pascal_lines(int S, const double* A, const double* B, const double* C, double* D,
+                               int n_sys, int n_row, int cyclic, hipStream_t st);
+
 // uneven batches: one lane per chunk of <= 64 rows of a system, 64 lanes per
 // work item (a wave); kind 0 = single-chunk systems (plain Thomas), kind 1 =
 // chunked systems (PaScaL with P = Q inside the wave)

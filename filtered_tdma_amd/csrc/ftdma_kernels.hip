@@ -40,17 +40,11 @@
 #include <mutex>
 #include <utility>
 
+#include "ftdma_device.h"
 #include "ftdma_kernels.h"
 #include "ftdma_mlpj_weights.h"
 
 namespace ftd {
-
-// para_range over [0, n) in P parts (libs/pascal_tdma/cpu/para_range.cpp:4-9)
-__host__ __device__ inline void part_of(int n, int P, int p, int& s, int& m) {
-    int base = n / P, rem = n % P;
-    s = p * base + (p < rem ? p : rem);
-    m = base + (p < rem ? 1 : 0);
-}
 
 // float -> int truncation that saturates instead of being undefined, NaN -> 0
 __device__ inline long long trunc_sat(double x) {
@@ -314,60 +308,6 @@ __global__ __launch_bounds__(256) void k_thomas_cyclic_fused(const double* __res
 #pragma unroll
     for (int j = 1; j < M; ++j)
         if (j < cnt) FTD_ST(d[j] + x0 * e[j], D + base + (size_t)j * ld);
-}
-
-// Reduced system of NR rows (B == 1) in LDS, row k of this lane's system at
-// index k * S, solved by Thomas in place (x to Dr). 4 rows at a time: their
-// values are read into registers first and c', d' are carried in registers,
-// so the serial chain is the arithmetic, not an LDS round trip per row.
-__device__ __forceinline__ void reduced_thomas_lds(double* Ar, double* Cr, double* Dr, int NR,
-                                                   int S) {
-    double cp = Cr[0], dp = Dr[0];
-    int k = 1;
-    for (; k + 4 <= NR; k += 4) {
-        double ak[4], ck[4], dk[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            ak[u] = Ar[(k + u) * S];
-            ck[u] = Cr[(k + u) * S];
-            dk[u] = Dr[(k + u) * S];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const double inv = 1.0 / (1.0 - ak[u] * cp);
-            dp = inv * (dk[u] - ak[u] * dp);
-            cp = inv * ck[u];
-            Dr[(k + u) * S] = dp;
-            Cr[(k + u) * S] = cp;
-        }
-    }
-    for (; k < NR; ++k) {
-        const double ak = Ar[k * S];
-        const double inv = 1.0 / (1.0 - ak * cp);
-        dp = inv * (Dr[k * S] - ak * dp);
-        cp = inv * Cr[k * S];
-        Dr[k * S] = dp;
-        Cr[k * S] = cp;
-    }
-    double dn = dp;
-    k = NR - 2;
-    for (; k >= 3; k -= 4) {
-        double ck[4], dk[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            ck[u] = Cr[(k - u) * S];
-            dk[u] = Dr[(k - u) * S];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            dn = dk[u] - ck[u] * dn;
-            Dr[(k - u) * S] = dn;
-        }
-    }
-    for (; k >= 0; --k) {
-        dn = Dr[k * S] - Cr[k * S] * dn;
-        Dr[k * S] = dn;
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -691,14 +631,6 @@ __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE))) voi
 // The last tile re-fetches its own rows into consumed slots so that the
 // pattern stays uniform; the kernel drains vmcnt before it ends.
 // ---------------------------------------------------------------------------
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-    static_assert(N >= 0 && N <= 63, "vmcnt range");
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-typedef const __attribute__((address_space(3))) double* lds_cdptr_t;
 typedef double ftd_dbl2 __attribute__((ext_vector_type(2)));
 
 // The four operands of one row-step from a ring slot (a, b at bytes 0 and
@@ -735,12 +667,6 @@ __device__ __forceinline__ void xin_read(lds_cdptr_t p, double& x0, double& xN) 
         : "memory");
     x0 = v.x;
     xN = v.y;
-}
-
-// workgroup barrier for LDS traffic only: the LDS writes are complete, the
-// DMAs in flight are left alone (__syncthreads would wait for them as well)
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
 #ifndef FTD_DMA_AUX
@@ -2766,7 +2692,7 @@ bool stream_eligible(int n_sys, const void* A, const void* B, const void* C, con
 
 // Workgroups of `kernel` resident on the whole device at once: the
 // persistent grid. Cached per (kernel, device).
-static int resident_grid(const void* kernel, int threads, int n_tiles) {
+int resident_grid(const void* kernel, int threads, int n_tiles) {
     static std::mutex mu;
     static std::map<std::pair<const void*, int>, int> cache;
     int dev = 0;

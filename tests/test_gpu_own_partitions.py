@@ -1,0 +1,96 @@
+"""Exact solves over partitions the engine chooses (one caller partition, or
+more rows in one than a lane holds): every kernel and tile shape the choice
+has, at the sizes where it changes, with rows on and off the 128-byte lines
+and last tiles of one system. Bit for bit the oracle's PaScaL of the
+partition count the path names, and within 1e-13 of serial Thomas."""
+import sys
+
+import numpy as np
+import pytest
+
+import oracle as O
+from filtered_tdma_amd import Kind, TdmaBackendGPU, cases
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+def note(msg):
+    print(f"[gpu-case] {msg}", flush=True)
+    sys.stdout.flush()
+
+
+def path_Q(path):
+    return int(path.split("Q=")[1].split()[0])
+
+
+def solve(A, B, C, D, P=1, cyclic=False, tuning=None, shift=0):
+    """x, path and the coefficients after the solve; shift: elements by which
+    the arrays start off their allocation."""
+    n_row, n_sys = D.shape
+
+    def place(x):
+        flat = torch.empty(x.size + shift, dtype=torch.float64, device="cuda")
+        flat[shift:].copy_(torch.from_numpy(np.ascontiguousarray(x).reshape(-1)))
+        return flat[shift:].view(n_row, n_sys)
+
+    be = TdmaBackendGPU(Kind.PASCAL, n_sys, n_row, P)
+    try:
+        if tuning is not None:
+            be.set_tuning(*tuning)
+        t = [place(x) for x in (A, B, C, D)]
+        (be.solve_cyclic if cyclic else be.solve)(*t)
+        torch.cuda.synchronize()
+        return t[3].cpu().numpy(), be.last_path(), [v.cpu().numpy() for v in t[:3]]
+    finally:
+        be.close()
+
+
+def check(n_sys, n_row, P=1, cyclic=False, shift=0):
+    A, B, C, D = cases.general_batch(n_sys, n_row, seed=n_sys + n_row)
+    x, path, after = solve(A, B, C, D, P, cyclic, shift=shift)
+    note(f"own partitions n_sys={n_sys} n_row={n_row} P={P} cyclic={cyclic} shift={shift}: {path}")
+    ref = O.pascal(A, B, C, D, path_Q(path), sem=O.SEM_GPU, cyclic=cyclic)
+    np.testing.assert_array_equal(x, ref, err_msg=path)
+    for v, w in zip(after, (A, B, C)):
+        np.testing.assert_array_equal(v, w, err_msg=path)
+    th = O.thomas(A, B, C, D, sem=O.SEM_GPU, cyclic=cyclic)
+    assert np.max(np.max(np.abs(x - th), 0) / np.max(np.abs(th), 0)) <= 1e-13, path
+    return A, B, C, D, x, path
+
+
+@pytest.mark.parametrize("cyclic", [False, True])
+@pytest.mark.parametrize("n_sys,n_row", [
+    (8192, 513), (8193, 1024),             # 16 systems per tile, last tile of 1
+    (2, 1025), (9, 1025), (2051, 1500), (24, 2048),   # 8 per tile
+    (3, 2049), (5, 3000), (1030, 4095), (4, 4096),    # 4 per tile
+])
+def test_long_systems_bitwise(n_sys, n_row, cyclic):
+    A, B, C, D, x, path = check(n_sys, n_row, cyclic=cyclic)
+    assert path.startswith("pascal_stream"), path
+    # the same partitions without the streamed kernels
+    xf, pathf, _ = solve(A, B, C, D, cyclic=cyclic, tuning=(-2, 0, 0, 0))
+    assert pathf.startswith("pascal_fused") and path_Q(pathf) == path_Q(path), pathf
+    np.testing.assert_array_equal(xf, x)
+
+
+@pytest.mark.parametrize("n_sys,n_row,P", [(100, 1500, 2), (33, 1030, 8), (5000, 200, 2)])
+def test_caller_partitions_longer_than_a_lane(n_sys, n_row, P):
+    check(n_sys, n_row, P=P)
+
+
+@pytest.mark.parametrize("n_sys,n_row", [(2048, 100), (512, 300), (33, 1100), (2048, 2100)])
+def test_own_partitions_at_element_alignment(n_sys, n_row):
+    check(n_sys, n_row, shift=1)
+
+
+def test_beyond_the_long_system_kernel():
+    """Above 4096 rows, and a single system above 512 rows in a batch the
+    other shapes do not hold: the lane-per-system Thomas, as before."""
+    for n_sys, n_row in ((3, 4097), (1, 1025)):
+        A, B, C, D = cases.general_batch(n_sys, n_row, seed=3)
+        note(f"general n_sys={n_sys} n_row={n_row}")
+        x, path, _ = solve(A, B, C, D)
+        assert path == "thomas_general", path
+        np.testing.assert_array_equal(x, O.thomas(A, B, C, D, sem=O.SEM_GPU))
