@@ -197,20 +197,48 @@ bool fused_of(int Q, int n_row, FusedShape& out) {
 }
 
 // Partitions and tile of a real exact solve whose partitions the engine
-// chooses, above 512 rows; out.M == 0: the long-system streamed kernel (Q and
-// S set). Both sides of each line in us:
+// chooses; out.M == 0: the long-system streamed kernel (Q and S set). Lines
+// drawn from a sweep over 512..131104 systems of 65..1024 rows; both sides of
+// each in us:
+//  * up to 512 rows, 32-row lanes, two waves per SIMD: the register prefetch
+//    of 8 waves covers the latency that 64-row lanes (one wave per SIMD)
+//    expose (16384 x 96: 14 against 18; 66049 x 257: 170 against 210).
+//  * up to 256 rows, while 32-system tiles do not fill the CUs once (8192
+//    systems): 16-row lanes, the shorter chain (2048 x 80: 7.4 against 8.6;
+//    8192 x 96: 8.7 against 9.9); 16-system tiles up to half of that.
+//  * 64-system tiles for up to 256 rows where rows are whole lines and the
+//    lanes fill whole waves (32768 x 256: 66 against 88); not at 5 or 6
+//    partitions, which leave a third of the waves unused (66049 x 160: 104
+//    against 120). A batch of one round of 64-system tiles takes them always
+//    (10000 x 200: 17 against 20).
+//  * above, 32-system tiles where rows are whole lines and the tiles fill the
+//    CUs (32768 x 512: 146 against 163), else 16 (66049 x 257: 170 against
+//    193; 2048 x 300: 12.7 against 15.8).
+//  * 449..512 rows of whole 32-system tiles keep 8 partitions, which the
+//    streamed kernel runs (262144 x 512: 980 against 1018).
 //  * above 512 rows the streamed long-system kernel (66049 x 768: 562 against
 //    609; 131104 x 1024: 1081 against 1125); with fewer than two 16-system
 //    tiles per CU and up to 1024 rows, 32-row lanes (2048 x 768: 23.3 against
 //    26.7).
 bool own_shape(int n_sys, int n_row, FusedShape& out) {
-    if (n_row <= 512) return false;
-    const int S = ftd::lines_systems(n_sys, n_row);
-    if (n_row <= 1024 && n_sys < 8192)
-        return shape_for(32, 512, (n_row + 31) / 32, n_row, 16, out);
-    if (!S) return false;
-    out = FusedShape{0, 0, S, 256 / S};
-    return true;
+    if (n_row < 65) return false;  // caller: Thomas, or the general choice
+    const bool lines = n_sys % 16 == 0;
+    if (n_row > 512) {
+        const int S = ftd::lines_systems(n_sys, n_row);
+        if (n_row <= 1024 && n_sys < 8192) return shape_for(32, 512, (n_row + 31) / 32, n_row, 16, out);
+        if (!S) return false;
+        out = FusedShape{0, 0, S, 256 / S};
+        return true;
+    }
+    if (n_row > 448 && n_sys % 32 == 0) return shape_for(64, 256, 8, n_row, 32, out);
+    if (n_row <= 256 && n_sys <= 8192)
+        return shape_for(16, 512, (n_row + 15) / 16, n_row, n_sys <= 4096 ? 16 : 32, out);
+    const int Q = (n_row + 31) / 32;
+    const int S = n_row > 256         ? (lines && n_sys >= 8192 ? 32 : 16)
+                  : n_sys <= 16384    ? 64
+                  : lines && Q != 5 && Q != 6 ? 64
+                                      : 32;
+    return shape_for(32, 512, Q, n_row, S, out);
 }
 
 bool pick_pascal(const ftd_handle* h, int n_row, FusedShape& out, int csh = 0) {

@@ -43,6 +43,7 @@
 #include "ftdma_device.h"
 #include "ftdma_kernels.h"
 #include "ftdma_mlpj_weights.h"
+#include "ftdma_xcd.h"
 
 namespace ftd {
 
@@ -185,16 +186,22 @@ __global__ __launch_bounds__(256) void k_compute_J(const double* __restrict__ pa
 #define FTD_ST(v, p) (*(p) = (v))
 #endif
 
-#define FTD_LOAD_ROW(j)                                                      \
+template <bool NT, typename T>
+__device__ __forceinline__ double load_row(const T* p) {
+    return (double)(NT ? FTD_LD(p) : *p);
+}
+
+#define FTD_LOAD_ROW_(j, nt)                                                 \
     do {                                                                     \
         const int jj_ = (j) < cnt ? (j) : cnt - 1;                           \
         const size_t o_ = base + (size_t)jj_ * ld;                           \
         const size_t oc_ = cbase + (size_t)jj_ * cld;                        \
-        ra[(j)] = (double)FTD_LD(A + oc_);                                   \
-        rb[(j)] = (double)FTD_LD(B + oc_);                                   \
-        rc[(j)] = (double)FTD_LD(C + oc_);                                   \
-        rd[(j)] = (double)FTD_LD(Din + o_);                                  \
+        ra[(j)] = load_row<nt>(A + oc_);                                     \
+        rb[(j)] = load_row<nt>(B + oc_);                                     \
+        rc[(j)] = load_row<nt>(C + oc_);                                     \
+        rd[(j)] = load_row<nt>(Din + o_);                                    \
     } while (0)
+#define FTD_LOAD_ROW(j) FTD_LOAD_ROW_(j, true)
 
 // ---------------------------------------------------------------------------
 // plain Thomas with the whole system in registers (n_row <= M): the
@@ -319,7 +326,12 @@ __global__ __launch_bounds__(256) void k_thomas_cyclic_fused(const double* __res
 // ---------------------------------------------------------------------------
 // TC: storage type of A, B, C; TD: of the right-hand side Din. The solution
 // goes to X (float64), which may be Din itself when TD is double.
-template <int M, int MAXT, bool CYCLIC, int PF, int WPE, typename TC, typename TD, int CSH = 0>
+// NT: row loads and stores marked nontemporal. Adjacent tiles run on one XCD
+// (xcd_tile), so a 128-byte line that two tiles share (rows that do not
+// start on lines, tiles under 16 systems) is fetched once, into that XCD's
+// L2, if both leave it there (NT = false). Measured at the launcher.
+template <int M, int MAXT, bool CYCLIC, int PF, int WPE, typename TC, typename TD, int CSH = 0,
+          bool NT = true>
 __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE))) void k_pascal_fused(
     const TC* __restrict__ A, const TC* __restrict__ B, const TC* __restrict__ C, const TD* Din,
     double* X, int n_sys, int n_row, int Q, int lgS) {
@@ -328,7 +340,7 @@ __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE))) voi
     const int t = threadIdx.x;
     const int sl = t & (S - 1);
     const int q = t >> lgS;
-    const int i_raw = blockIdx.x * S + sl;
+    const int i_raw = xcd_tile(blockIdx.x, gridDim.x) * S + sl;
     const bool live = i_raw < n_sys;
     // dead lanes shadow the last system (of their parity when CSH = 1)
     const int i = live ? i_raw : n_sys - (1 << CSH) + (i_raw & ((1 << CSH) - 1));
@@ -344,12 +356,12 @@ __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE))) voi
     double aN = 0.0, cN = 0.0, dN = 0.0;
 
 #pragma unroll
-    for (int j = 0; j < PF && j < M; ++j) FTD_LOAD_ROW(j);
+    for (int j = 0; j < PF && j < M; ++j) FTD_LOAD_ROW_(j, NT);
 
     // forward sweep: rows 0,1 divided by b, then modified elimination
 #pragma unroll
     for (int j = 0; j < M; ++j) {
-        if (j + PF < M) FTD_LOAD_ROW(j + PF);
+        if (j + PF < M) FTD_LOAD_ROW_(j + PF, NT);
         if (j < cnt) {
             const double aj = ra[j], bj = rb[j], cj = rc[j], dj = rd[j];
             if (j < 2) {
@@ -446,7 +458,10 @@ __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE))) voi
                     x = xN;
                 else
                     x = d[j] - (a[j] * x0 + c[j] * xN);
-                FTD_ST(x, X + base + (size_t)j * ld);
+                if (NT)
+                    FTD_ST(x, X + base + (size_t)j * ld);
+                else
+                    X[base + (size_t)j * ld] = x;
             }
         }
     }
@@ -2479,7 +2494,7 @@ size_t pascal_fused_lds(int Q, int S, int cyclic) {
     return sizeof(double) * (size_t)(cyclic ? 4 : 3) * (size_t)(2 * Q) * (size_t)S;
 }
 
-template <typename TC, typename TD>
+template <typename TC, typename TD, bool NT>
 static hipError_t launch_pascal_fused_t(int M, int maxt, const TC* A, const TC* B, const TC* C,
                                         const TD* Din, double* Xout, int n_sys, int n_row, int Q,
                                         int S, int cyclic, int csh, hipStream_t st) {
@@ -2489,13 +2504,13 @@ static hipError_t launch_pascal_fused_t(int M, int maxt, const TC* A, const TC* 
 #define X(m_, t_, pf_, w_)                                                                  \
     if (M == m_ && maxt == t_) {                                                            \
         if (cyclic)                                                                         \
-            hipLaunchKernelGGL((k_pascal_fused<m_, t_, true, pf_, w_, TC, TD>), grid, block, \
-                               lds, st, A, B, C, Din, Xout, n_sys, n_row, Q, lgS);          \
+            hipLaunchKernelGGL((k_pascal_fused<m_, t_, true, pf_, w_, TC, TD, 0, NT>), grid, \
+                               block, lds, st, A, B, C, Din, Xout, n_sys, n_row, Q, lgS);   \
         else if (csh)                                                                       \
             hipLaunchKernelGGL((k_pascal_fused<m_, t_, false, pf_, w_, TC, TD, 1>), grid,   \
                                block, lds, st, A, B, C, Din, Xout, n_sys, n_row, Q, lgS);   \
         else                                                                                \
-            hipLaunchKernelGGL((k_pascal_fused<m_, t_, false, pf_, w_, TC, TD>), grid,      \
+            hipLaunchKernelGGL((k_pascal_fused<m_, t_, false, pf_, w_, TC, TD, 0, NT>), grid, \
                                block, lds, st, A, B, C, Din, Xout, n_sys, n_row, Q, lgS);   \
         return hipGetLastError();                                                           \
     }
@@ -2508,21 +2523,28 @@ hipError_t launch_pascal_fused(int M, int maxt, const double* A, const double* B
                                double* D, int n_sys, int n_row, int Q, int S, int cyclic, int csh,
                                hipStream_t st) {
     if (csh && cyclic) return hipErrorInvalidValue;
-    return launch_pascal_fused_t<double, double>(M, maxt, A, B, C, D, D, n_sys, n_row, Q, S,
-                                                 cyclic, csh, st);
+    // rows that start off the 128-byte lines share lines with the neighbouring
+    // tiles: those stay cached (66049 x 257, M = 32, S = 16: 172 against 264 us;
+    // where rows are whole lines nontemporal is faster, 65536 x 512, S = 32:
+    // 280 against 345 us)
+    if (csh || n_sys % 16 == 0)
+        return launch_pascal_fused_t<double, double, true>(M, maxt, A, B, C, D, D, n_sys, n_row, Q,
+                                                           S, cyclic, csh, st);
+    return launch_pascal_fused_t<double, double, false>(M, maxt, A, B, C, D, D, n_sys, n_row, Q, S,
+                                                        cyclic, csh, st);
 }
 
 hipError_t launch_pascal_fused_f32c(int M, int maxt, const float* A, const float* B,
                                     const float* C, double* D, int n_sys, int n_row, int Q, int S,
                                     int cyclic, hipStream_t st) {
-    return launch_pascal_fused_t<float, double>(M, maxt, A, B, C, D, D, n_sys, n_row, Q, S,
+    return launch_pascal_fused_t<float, double, true>(M, maxt, A, B, C, D, D, n_sys, n_row, Q, S,
                                                 cyclic, 0, st);
 }
 
 hipError_t launch_pascal_fused_f32(int M, int maxt, const float* A, const float* B, const float* C,
                                    const float* D, double* X, int n_sys, int n_row, int Q, int S,
                                    int cyclic, hipStream_t st) {
-    return launch_pascal_fused_t<float, float>(M, maxt, A, B, C, D, X, n_sys, n_row, Q, S, cyclic,
+    return launch_pascal_fused_t<float, float, true>(M, maxt, A, B, C, D, X, n_sys, n_row, Q, S, cyclic,
                                                0, st);
 }
 

@@ -62,6 +62,18 @@ def check(n_sys, n_row, P=1, cyclic=False, shift=0):
 
 @pytest.mark.parametrize("cyclic", [False, True])
 @pytest.mark.parametrize("n_sys,n_row", [
+    (1, 65), (4096, 80), (4097, 256),      # 16-row lanes, 16- and 32-system tiles
+    (8193, 100), (16385, 130),             # 64-system tiles; 32 off the lines
+    (16400, 150), (16400, 256),            # 5 partitions (32) and 8 (64) on the lines
+    (8208, 300), (8209, 300), (40, 448),   # above 256 rows: 32 on the lines, else 16
+    (64, 449), (8224, 512), (65, 512),     # 8 streamed partitions, and off whole tiles
+])
+def test_own_partitions_bitwise(n_sys, n_row, cyclic):
+    check(n_sys, n_row, cyclic=cyclic)
+
+
+@pytest.mark.parametrize("cyclic", [False, True])
+@pytest.mark.parametrize("n_sys,n_row", [
     (8192, 513), (8193, 1024),             # 16 systems per tile, last tile of 1
     (2, 1025), (9, 1025), (2051, 1500), (24, 2048),   # 8 per tile
     (3, 2049), (5, 3000), (1030, 4095), (4, 4096),    # 4 per tile
