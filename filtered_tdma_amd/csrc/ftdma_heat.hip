@@ -107,6 +107,25 @@ __global__ void k_periodic(double* __restrict__ th, Dims g, int face) {
     }
 }
 
+// Lines of the field (pitch px) from or to the packed host layout (pitch
+// nx + 2), so that the field crosses to the host in one linear copy: a pitched
+// 2-D copy to pageable memory goes line by line (100 steps and the field:
+// 35.3 against 6.0 ms at 64^3, 485 against 37.6 at 256^3). One workgroup per
+// line; the pack itself is a copy of the field on the device.
+template <bool PACK>
+__global__ __launch_bounds__(128) void k_lines(double* __restrict__ field,
+                                               double* __restrict__ packed, Dims g) {
+    const size_t line = blockIdx.x;
+    double* const f = field + kOrigin + line * g.px;
+    double* const p = packed + line * g.nx1;
+    for (int i = threadIdx.x; i < g.nx1; i += 128) {
+        if (PACK)
+            p[i] = f[i];
+        else
+            f[i] = p[i];
+    }
+}
+
 struct Stencil {
     double xa, xb, xc, ya, yb, yc, za, zb, zc, c0;
 };
@@ -1410,8 +1429,12 @@ ftd_status ftd_heat_init(ftd_heat* h) {
                 f[((size_t)k * ny1 + j) * nx1 + i] =
                     h->sx_[i] * h->sy_[j] * h->sz_[k] + h->cx_[i] * h->cy_[j] * h->cz_[k];
     const Dims g = h->g;
-    HH(hipMemcpy2DAsync(h->th + kOrigin, sizeof(double) * g.px, f.data(), sizeof(double) * nx1,
-                        sizeof(double) * nx1, (size_t)ny1 * nz1, hipMemcpyHostToDevice, h->stream));
+    // rhs is free between steps: every step writes its cells before reading them
+    HH(hipMemcpyAsync(h->rhs, f.data(), sizeof(double) * f.size(), hipMemcpyHostToDevice,
+                      h->stream));
+    hipLaunchKernelGGL((k_lines<false>), dim3((unsigned)(ny1 * nz1)), dim3(128), 0, h->stream,
+                       h->th, h->rhs, g);
+    HH(hipGetLastError());
     const dim3 b2(16, 16);
     for (int d = 0; d < 3; ++d) {
         if (!h->periodic[d]) continue;
@@ -1506,9 +1529,13 @@ ftd_status ftd_heat_set_fused(ftd_heat* h, int enable) {
 ftd_status ftd_heat_field(ftd_heat* h, double* host_out) {
     if (!h || !host_out) return herr(FTD_ERR_INVALID, "null argument");
     const Dims& g = h->g;
-    HH(hipMemcpy2DAsync(host_out, sizeof(double) * g.nx1, h->th + kOrigin, sizeof(double) * g.px,
-                        sizeof(double) * g.nx1, (size_t)g.ny1 * (h->nz + 2),
-                        hipMemcpyDeviceToHost, h->stream));
+    // packed into rhs (free between steps), then one linear copy
+    const size_t lines = (size_t)g.ny1 * (h->nz + 2);
+    hipLaunchKernelGGL((k_lines<true>), dim3((unsigned)lines), dim3(128), 0, h->stream, h->th,
+                       h->rhs, g);
+    HH(hipGetLastError());
+    HH(hipMemcpyAsync(host_out, h->rhs, sizeof(double) * lines * g.nx1, hipMemcpyDeviceToHost,
+                      h->stream));
     HH(hipStreamSynchronize(h->stream));
     return FTD_OK;
 }
