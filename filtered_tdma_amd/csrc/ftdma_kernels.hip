@@ -2008,18 +2008,33 @@ __global__ __launch_bounds__(256) void k_gen_pascal_update(const double* __restr
 // sweeps): the network's features are taken from the raw rows as the
 // forward pass reads them; its J of this (system, partition), clamped to
 // [0, m-1], goes to Jsys[p][i] for k_gen_filtered_check.
+//
+// A lane walks its whole partition, so what bounds a batch that does not fill
+// the chip is the latency of each row's loads: rows are read kGenU at a time,
+// a block ahead of the one being worked on and before its stores (the
+// compiler cannot move them there: same pointers, and it cannot rule out
+// ld == 0), and a workgroup is one wave, so that few systems still reach
+// every CU. 16641 x 512 in 2 partitions: one row ahead in 256-lane groups
+// 230 us, now 159 (4096 x 1024: the solve 0.65 to 0.16 ms). A large batch is
+// bound by the bytes of the state (a', c', d' written and read back).
+constexpr int kGenU = 8;
+
 template <int VERSION, bool FEAT>
-__global__ __launch_bounds__(256) void k_gen_filtered_sweep(double* __restrict__ A,
-                                                            const double* __restrict__ B,
-                                                            double* __restrict__ C,
-                                                            double* __restrict__ D, int n_sys,
-                                                            int n_row, int P,
-                                                            const int* __restrict__ Jp,
-                                                            double eps_value, int eps_direct,
-                                                            int* __restrict__ Jsys) {
+__global__ __launch_bounds__(64) void k_gen_filtered_sweep(double* __restrict__ A,
+                                                           const double* __restrict__ B,
+                                                           double* __restrict__ C,
+                                                           double* __restrict__ D, int n_sys,
+                                                           int n_row, int P,
+                                                           const int* __restrict__ Jp,
+                                                           double eps_value, int eps_direct,
+                                                           int* __restrict__ Jsys) {
     static_assert(!FEAT || VERSION == 1, "the learned J runs the v1 sweeps");
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int p = blockIdx.y;
+    constexpr int U = kGenU;
+    // neighbouring systems' waves on one XCD: they share the lines their rows
+    // end on
+    const int T = xcd_tile(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+    const int i = T % (int)gridDim.x * 64 + threadIdx.x;
+    const int p = T / (int)gridDim.x;
     if (i >= n_sys) return;
     int s, m;
     part_of(n_row, P, p, s, m);
@@ -2032,6 +2047,19 @@ __global__ __launch_bounds__(256) void k_gen_filtered_sweep(double* __restrict__
     // features: max |a/b|, |c/b| over rows 1..m-1, raw d of rows 0 and m-1,
     // max |d| (as k_filtered_fused takes them)
     double f_rho = 0.0, f_d0 = 0.0, f_dN = 0.0, f_dmax = 0.0;
+    // rows j .. j + U - 1 (past the partition: its last row, unused)
+    double ra[U], rb[U], rc[U], rd[U];
+    auto fetch = [&](int j) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const size_t o = (size_t)(j + u < m ? j + u : m - 1) * ld;
+            ra[u] = Ap[o];
+            rb[u] = Bp[o];
+            rc[u] = Cp[o];
+            rd[u] = Dp[o];
+        }
+    };
+    fetch(2);
     for (int j = 0; j < 2; ++j) {
         const size_t o = (size_t)j * ld;
         if (FEAT) {
@@ -2046,34 +2074,47 @@ __global__ __launch_bounds__(256) void k_gen_filtered_sweep(double* __restrict__
         Dp[o] *= r0;
     }
     double am = Ap[ld], cm = Cp[ld], dm = Dp[ld];
-    // Row j + 1's loads are issued before row j's stores: the compiler cannot
-    // move them there itself (the same pointers one row apart, and it cannot
-    // rule out ld == 0), and a lane then waits for every row's loads in turn.
-    // The next row is clamped to the partition's last row (a reload, unused).
-    int j = 2;
-    const int j2 = 2 < m ? 2 : m - 1;
-    double na = Ap[(size_t)j2 * ld], nb = Bp[(size_t)j2 * ld], nc = Cp[(size_t)j2 * ld],
-           nd = Dp[(size_t)j2 * ld];
-    for (; j <= J && j < m; ++j) {
-        const size_t o = (size_t)j * ld;
-        const double aj = na, bj = nb, cj = nc, dj = nd;
-        const size_t on = (size_t)(j + 1 < m ? j + 1 : m - 1) * ld;
-        na = Ap[on];
-        nb = Bp[on];
-        nc = Cp[on];
-        nd = Dp[on];
-        if (FEAT) {
-            f_rho = fmax(f_rho, fmax(fabs(aj), fabs(cj)) / fabs(bj));
-            if (j == m - 1) f_dN = dj;
-            f_dmax = fmax(f_dmax, fabs(dj));
+    if (VERSION == 2 && J == 0) {
+        // k_fwd_pass_v2 with J == 0 starts its skip-A loop at row 1 and
+        // eliminates the normalised row 1 against itself
+        const double inv = 1.0 / (Bp[ld] - am * cm);
+        dm = inv * (dm - am * dm);
+        cm = inv * cm;
+        Cp[ld] = cm;
+        Dp[ld] = dm;
+    }
+    for (int j0 = 2; j0 < m; j0 += U) {
+        double va[U], vb[U], vc[U], vd[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            va[u] = ra[u];
+            vb[u] = rb[u];
+            vc[u] = rc[u];
+            vd[u] = rd[u];
         }
-        const double inv = 1.0 / (bj - aj * cm);
-        dm = inv * (dj - aj * dm);
-        cm = inv * cj;
-        am = -inv * aj * am;
-        Ap[o] = am;
-        Cp[o] = cm;
-        Dp[o] = dm;
+        fetch(j0 + U);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int j = j0 + u;
+            if (j < m) {
+                const size_t o = (size_t)j * ld;
+                const double aj = va[u], bj = vb[u], cj = vc[u], dj = vd[u];
+                if (FEAT) {
+                    f_rho = fmax(f_rho, fmax(fabs(aj), fabs(cj)) / fabs(bj));
+                    if (j == m - 1) f_dN = dj;
+                    f_dmax = fmax(f_dmax, fabs(dj));
+                }
+                const double inv = 1.0 / (bj - aj * cm);
+                dm = inv * (dj - aj * dm);
+                cm = inv * cj;
+                if (VERSION == 1 || j <= J) {  // v2 leaves the later rows' A raw
+                    am = -inv * aj * am;
+                    Ap[o] = am;
+                }
+                Cp[o] = cm;
+                Dp[o] = dm;
+            }
+        }
     }
     if (FEAT) {
         const double Nl = (double)(m * P);
@@ -2082,61 +2123,50 @@ __global__ __launch_bounds__(256) void k_gen_filtered_sweep(double* __restrict__
                        lg_feature(f_dmax), lg_feature(eps));
         Jsys[(size_t)p * ld + i] = Jl < 0 ? 0 : (Jl > m - 1 ? m - 1 : Jl);
     }
-    if (VERSION == 2) {
-        // the skip-A rows, loads one row ahead as above
-        j = J + 1 > 1 ? J + 1 : 1;
-        if (j < m) {
-            na = Ap[(size_t)j * ld];
-            nb = Bp[(size_t)j * ld];
-            nc = Cp[(size_t)j * ld];
-            nd = Dp[(size_t)j * ld];
-        }
-        for (; j < m; ++j) {
-            const size_t o = (size_t)j * ld;
-            const double aj = na, bj = nb, cj = nc, dj = nd;
-            const size_t on = (size_t)(j + 1 < m ? j + 1 : m - 1) * ld;
-            na = Ap[on];
-            nb = Bp[on];
-            nc = Cp[on];
-            nd = Dp[on];
-            const double inv = 1.0 / (bj - aj * cm);
-            dm = inv * (dj - aj * dm);
-            cm = inv * cj;
-            Cp[o] = cm;
-            Dp[o] = dm;
-        }
-    }
-    // backward, row j - 1's loads issued before row j's stores
+    // backward: rows j, j - 1, .., j - U + 1, a block ahead as above (before
+    // the partition: row 1, unused). v2 reads a row's A only where it updates
+    // a, rows below J: J is the partition's, so the test is uniform.
     const size_t onm2 = (size_t)(m - 2) * ld;
     double dn = Dp[onm2], cn = Cp[onm2];
     double an = (VERSION == 1) ? Ap[onm2] : (J >= 2 ? Ap[(size_t)J * ld] : 0.0);
     const int lo = (m - 2) - J;
-    // (v2 reads a row's A only where it updates a, rows below J: J is the
-    // partition's, so the test is uniform across the wave)
-    j = m - 3;
-    double pa = 0.0, pc = 0.0, pd = 0.0;
-    if (j >= 1) {
-        if (VERSION == 1 || (J >= 2 && j < J)) pa = Ap[(size_t)j * ld];
-        pc = Cp[(size_t)j * ld];
-        pd = Dp[(size_t)j * ld];
-    }
-    for (; j >= 1; --j) {
-        const size_t o = (size_t)j * ld;
-        const double aj = pa, cj = pc, dj = pd;
-        const int jp = j > 1 ? j - 1 : 1;
-        const size_t op = (size_t)jp * ld;
-        if (VERSION == 1 || (J >= 2 && jp < J)) pa = Ap[op];
-        pc = Cp[op];
-        pd = Dp[op];
-        dn = dj - cj * dn;
-        Dp[o] = dn;
-        if (VERSION == 1 || (J >= 2 && j < J)) {
-            an = aj - cj * an;
-            Ap[o] = an;
+    auto fetch_back = [&](int j) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int jj = j - u > 1 ? j - u : 1;
+            const size_t o = (size_t)jj * ld;
+            if (VERSION == 1 || (J >= 2 && jj < J)) ra[u] = Ap[o];
+            rc[u] = Cp[o];
+            rd[u] = Dp[o];
         }
-        if (VERSION == 1 || j > lo) {
-            cn = -cj * cn;
-            Cp[o] = cn;
+    };
+    fetch_back(m - 3);
+    for (int j0 = m - 3; j0 >= 1; j0 -= U) {
+        double va[U], vc[U], vd[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            va[u] = ra[u];
+            vc[u] = rc[u];
+            vd[u] = rd[u];
+        }
+        if (j0 - U >= 1) fetch_back(j0 - U);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int j = j0 - u;
+            if (j >= 1) {
+                const size_t o = (size_t)j * ld;
+                const double cj = vc[u];
+                dn = vd[u] - cj * dn;
+                Dp[o] = dn;
+                if (VERSION == 1 || (J >= 2 && j < J)) {
+                    an = va[u] - cj * an;
+                    Ap[o] = an;
+                }
+                if (VERSION == 1 || j > lo) {
+                    cn = -cj * cn;
+                    Cp[o] = cn;
+                }
+            }
         }
     }
     const double A1 = Ap[ld], C0 = Cp[0], D1 = Dp[ld];
@@ -2360,24 +2390,16 @@ __global__ __launch_bounds__(256) void k_gen_filtered_check(
     }
 }
 
-__device__ inline int wave_max_i(int v) {
-    for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, 64));
-    return v;
-}
-__device__ inline int wave_min_i(int v) {
-    for (int off = 32; off > 0; off >>= 1) v = min(v, __shfl_xor(v, off, 64));
-    return v;
-}
-
 // truncated final correction (k_final_pass, filtered_tdma_kernels.cuh:196-218);
 // J per partition from Jp, or per (partition, system) from Jsys (low 16
-// bits) where the general path's check kernel ran.
-// One J per partition: the left rows 1..jL, then the right rows jR..m-2.
-// A J per system: one walk over the rows, each read and written once, the
-// two corrections predicated per lane ((d - a x0) - c xN where both apply,
-// as the two walks give), and the rows no lane of the wave corrects skipped
-// at once. A lane that falls back to J = m-1 then costs its wave one walk
-// over the partition instead of two.
+// bits) where the general path's check kernel ran. Each row stands by itself
+// (d - a x0 on the rows 1..jL, then - c xN on jR..m-2), so the rows are spread
+// over the grid: block z takes kFinalRows of them, and the blocks whose rows
+// no lane corrects (the middle of the partition) end at once. All of a
+// thread's loads are in flight together. One lane walking the whole
+// partition took 87 us at 16641 x 512 in 2 partitions, now 33 us.
+constexpr int kFinalRows = 8;
+
 __global__ __launch_bounds__(256) void k_gen_filtered_final(const double* __restrict__ A,
                                                             const double* __restrict__ C,
                                                             double* __restrict__ D, int n_sys,
@@ -2385,53 +2407,51 @@ __global__ __launch_bounds__(256) void k_gen_filtered_final(const double* __rest
                                                             const int* __restrict__ Jp,
                                                             const double* __restrict__ xbuf,
                                                             const int* __restrict__ Jsys) {
-    const int i_raw = blockIdx.x * blockDim.x + threadIdx.x;
-    const int p = blockIdx.y;
-    const bool live = i_raw < n_sys;
-    if (!Jsys && !live) return;
-    const int i = live ? i_raw : n_sys - 1;
+    const int T = xcd_tile(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+    const int i = T % (int)gridDim.x * 256 + threadIdx.x;
+    const int p = T / (int)gridDim.x;
+    if (i >= n_sys) return;
     int s, m;
     part_of(n_row, P, p, s, m);
     const size_t ld = (size_t)n_sys;
-    const double x0 = xbuf[(size_t)(2 * p) * ld + i];
-    const double xN = xbuf[(size_t)(2 * p + 1) * ld + i];
+    const int J = Jsys ? (Jsys[(size_t)p * ld + i] & 0xFFFF) : Jp[p];
+    const int jL = J < m - 2 ? J : m - 2;
+    const int jR = (m - 1) - J > 1 ? (m - 1) - J : 1;
     double* Dp = D + (size_t)s * ld + i;
     const double* Ap = A + (size_t)s * ld + i;
     const double* Cp = C + (size_t)s * ld + i;
-    const int J = Jsys ? (Jsys[(size_t)p * ld + i] & 0xFFFF) : Jp[p];
-    int jL = J < m - 2 ? J : m - 2;
-    int jR = (m - 1) - J > 1 ? (m - 1) - J : 1;
-    if (!Jsys) {
-        Dp[0] = x0;
-        Dp[(size_t)(m - 1) * ld] = xN;
-        for (int j = 1; j <= jL; ++j) {
+    // (a grid of more blocks than z holds comes round again)
+    for (int j0 = (int)blockIdx.z * kFinalRows; j0 < m; j0 += (int)gridDim.z * kFinalRows) {
+        if (j0 > jL && j0 + kFinalRows <= jR) continue;  // no row in 0..jL or jR..m-1
+        const double x0 = xbuf[(size_t)(2 * p) * ld + i];
+        const double xN = xbuf[(size_t)(2 * p + 1) * ld + i];
+        double x[kFinalRows], a[kFinalRows], c[kFinalRows];
+#pragma unroll
+        for (int u = 0; u < kFinalRows; ++u) {
+            const int j = j0 + u;
             const size_t o = (size_t)j * ld;
-            Dp[o] = Dp[o] - Ap[o] * x0;
+            const bool in = j >= 1 && j <= m - 2;
+            const bool l = in && j <= jL, r = in && j >= jR;
+            x[u] = a[u] = c[u] = 0.0;
+            if (l || r) x[u] = Dp[o];
+            if (l) a[u] = Ap[o];
+            if (r) c[u] = Cp[o];
         }
-        for (int j = jR; j < m - 1; ++j) {
+#pragma unroll
+        for (int u = 0; u < kFinalRows; ++u) {
+            const int j = j0 + u;
             const size_t o = (size_t)j * ld;
-            Dp[o] = Dp[o] - Cp[o] * xN;
-        }
-        return;
-    }
-    if (live) {
-        Dp[0] = x0;
-        Dp[(size_t)(m - 1) * ld] = xN;
-    } else {
-        jL = 0;  // no row
-        jR = m - 1;
-    }
-    const int wjL = wave_max_i(jL), wjR = wave_min_i(jR);
-    for (int j = 1; j <= m - 2; ++j) {
-        if (j > wjL && j < wjR) j = wjR;  // wave-uniform: no lane corrects rows wjL+1..wjR-1
-        if (j > m - 2) break;
-        const bool l = j <= jL, r = j >= jR;
-        if (l || r) {
-            const size_t o = (size_t)j * ld;
-            double x = Dp[o];
-            if (l) x = x - Ap[o] * x0;
-            if (r) x = x - Cp[o] * xN;
-            Dp[o] = x;
+            if (j == 0) {
+                Dp[o] = x0;
+            } else if (j == m - 1) {
+                Dp[o] = xN;
+            } else if (j < m - 1) {
+                const bool l = j <= jL, r = j >= jR;
+                double v = x[u];
+                if (l) v = v - a[u] * x0;
+                if (r) v = v - c[u] * xN;
+                if (l || r) Dp[o] = v;
+            }
         }
     }
 }
@@ -2882,16 +2902,16 @@ hipError_t launch_gen_pascal(double* A, const double* B, double* C, double* D, i
 hipError_t launch_gen_filtered_sweep(int version, double* A, const double* B, double* C, double* D,
                                      int n_sys, int n_row, int P, const int* Jp, int learned,
                                      double eps_value, int eps_direct, int* Jsys, hipStream_t st) {
-    const dim3 g2((n_sys + 255) / 256, P);
+    const dim3 g2((n_sys + 63) / 64, P);
     if (learned && version != 1) return hipErrorInvalidValue;
     if (version == 2)
-        hipLaunchKernelGGL((k_gen_filtered_sweep<2, false>), g2, dim3(256), 0, st, A, B, C, D,
+        hipLaunchKernelGGL((k_gen_filtered_sweep<2, false>), g2, dim3(64), 0, st, A, B, C, D,
                            n_sys, n_row, P, Jp, eps_value, eps_direct, Jsys);
     else if (learned)
-        hipLaunchKernelGGL((k_gen_filtered_sweep<1, true>), g2, dim3(256), 0, st, A, B, C, D,
+        hipLaunchKernelGGL((k_gen_filtered_sweep<1, true>), g2, dim3(64), 0, st, A, B, C, D,
                            n_sys, n_row, P, Jp, eps_value, eps_direct, Jsys);
     else
-        hipLaunchKernelGGL((k_gen_filtered_sweep<1, false>), g2, dim3(256), 0, st, A, B, C, D,
+        hipLaunchKernelGGL((k_gen_filtered_sweep<1, false>), g2, dim3(64), 0, st, A, B, C, D,
                            n_sys, n_row, P, Jp, eps_value, eps_direct, Jsys);
     return hipGetLastError();
 }
@@ -2929,7 +2949,9 @@ hipError_t launch_gen_filtered_iface(const double* A, const double* C, const dou
 hipError_t launch_gen_filtered_final(const double* A, const double* C, double* D, int n_sys,
                                      int n_row, int P, const int* Jp, const double* xbuf,
                                      const int* Jsys, hipStream_t st) {
-    const dim3 g2((n_sys + 255) / 256, P);
+    const int m_max = (n_row + P - 1) / P;
+    const int blocks = (m_max + kFinalRows - 1) / kFinalRows;
+    const dim3 g2((n_sys + 255) / 256, P, blocks < 65535 ? blocks : 65535);
     hipLaunchKernelGGL(k_gen_filtered_final, g2, dim3(256), 0, st, A, C, D, n_sys, n_row, P, Jp,
                        xbuf, Jsys);
     return hipGetLastError();
