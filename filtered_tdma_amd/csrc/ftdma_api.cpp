@@ -78,6 +78,7 @@ struct ftd_handle {
     char path[96] = "none";
     int t_M = 0, t_T = 0, t_S = 0, t_Q = 0;  // forced tuning (0 = automatic)
     int force_general = 0;                   // use the general kernels only
+    int keep_thomas = 0;                     // one partition of up to 64 rows: always Thomas
     int no_stream = 0;                       // automatic choice without the streamed kernels
     int j_mode = 0;                          // 0: cal_J (reference), 1: learned J per system
     int guard = 0;                           // filtered kinds: exact solve where terms exceed eps_/4
@@ -200,6 +201,8 @@ bool fused_of(int Q, int n_row, FusedShape& out) {
 // chooses; out.M == 0: the long-system streamed kernel (Q and S set). Lines
 // drawn from a sweep over 512..131104 systems of 65..1024 rows; both sides of
 // each in us:
+//  * 33 to 64 rows: 16-row lanes; 64-system tiles once 32-system ones fill the
+//    CUs twice (66049 x 48: 25.1 against 28.6 us; 4096 x 64: 8.3 against 8.9).
 //  * up to 512 rows, 32-row lanes, two waves per SIMD: the register prefetch
 //    of 8 waves covers the latency that 64-row lanes (one wave per SIMD)
 //    expose (16384 x 96: 14 against 18; 66049 x 257: 170 against 210).
@@ -221,7 +224,9 @@ bool fused_of(int Q, int n_row, FusedShape& out) {
 //    tiles per CU and up to 1024 rows, 32-row lanes (2048 x 768: 23.3 against
 //    26.7).
 bool own_shape(int n_sys, int n_row, FusedShape& out) {
-    if (n_row < 65) return false;  // caller: Thomas, or the general choice
+    if (n_row < 33) return false;  // caller: Thomas, or the general choice
+    if (n_row <= 64)
+        return shape_for(16, 512, (n_row + 15) / 16, n_row, n_sys <= 16384 ? 32 : 64, out);
     const bool lines = n_sys % 16 == 0;
     if (n_row > 512) {
         const int S = ftd::lines_systems(n_sys, n_row);
@@ -279,9 +284,14 @@ ftd_status solve_exact(ftd_handle* h, double* A, double* B, double* C, double* D
     hipStream_t st = h->stream;
     if (cyclic && n_row < 3) return fail(FTD_ERR_UNSUPPORTED, "periodic solve needs n_row >= 3");
     FusedShape fs;
-    if (!h->force_general && !h->t_M && h->P == 1 && n_row >= 3 && ftd::thomas_fused_rows(n_row)) {
+    if (!h->force_general && !h->t_M && h->P == 1 && n_row >= 3 && ftd::thomas_fused_rows(n_row) &&
+        (csh || cyclic || h->keep_thomas || n_row <= 32 || n_sys >= 131072)) {
         // one partition that fits a lane: plain (or Sherman-Morrison periodic)
-        // Thomas in registers, the reference's single-rank path
+        // Thomas in registers, the reference's single-rank path. Above 32 rows
+        // (not periodic) only where the batch fills the chip many times over (262144 x 64: 115
+        // against 123 us); a smaller one waits for the chain of its rows, and
+        // 16-row partitions shorten it (4096 x 64: 15.0 to 8.1 us, 66049 x 48:
+        // 38.5 to 25.1, 1024 x 48: 11.1 to 8.0)
         if (cyclic) {
             std::snprintf(h->path, sizeof h->path, "thomas_cyclic_fused M=%d",
                           ftd::thomas_fused_rows(n_row));
@@ -916,7 +926,11 @@ static ftd_status solve_f32_common(ftd_handle* h, const float* A, const float* B
         return fail(FTD_ERR_UNSUPPORTED, "FP32 storage is available for the exact (PaScaL) solve");
     if (h->n_sys == 0) return FTD_OK;
     FusedShape fs;
-    if (h->n_row < 6 || !pick_pascal(h, h->n_row, fs))
+    // the shapes of own_shape hold for FP32 storage as well (131072 x 256: 174
+    // against 193 us with 64-row lanes, 131104 x 80: 58 against 78)
+    const bool own = !h->t_M && h->n_row >= 6 && !caller_shape(h, h->n_row, fs) &&
+                     own_shape(h->n_sys, h->n_row, fs) && fs.M;
+    if (h->n_row < 6 || !(own || pick_pascal(h, h->n_row, fs)))
         return fail(FTD_ERR_UNSUPPORTED, "no fused kernel holds this system for FP32 storage");
     if (h->profiling) FTD_HIP(hipEventRecord(h->ev0, h->stream));
     // FP32 A, B, C, D: the streamed kernel runs the same partitions (same
@@ -924,7 +938,9 @@ static ftd_status solve_f32_common(ftd_handle* h, const float* A, const float* B
     int s_, m_max;
     part_of(h->n_row, fs.Q, 0, s_, m_max);
     const int Ms =
-        (d_is_float && !h->t_M && !h->no_stream) ? ftd::stream_rows_f32(m_max, fs.Q) : 0;
+        (d_is_float && !h->t_M && !h->no_stream && !(own && fs.M < 64))
+            ? ftd::stream_rows_f32(m_max, fs.Q)
+            : 0;
     const bool streamed =
         Ms && ftd::stream_eligible(h->n_sys, A, B, C, D) && !((uintptr_t)X & 15u);
     if (streamed) {
@@ -1330,6 +1346,8 @@ const char* ftd_last_error_string(void) { return g_err.c_str(); }
 }  // extern "C"
 
 namespace ftd {
+void handle_keep_thomas(ftd_handle* h) { h->keep_thomas = 1; }
+
 int handle_filtered_state(ftd_handle* h, int** J, const double** rho, double* eps_value,
                           int* eps_direct) {
     if (!h || h->kind == FTD_KIND_PASCAL || h->P < 2 || !h->J || !h->rho)

@@ -1392,7 +1392,10 @@ ftd_status ftd_heat_create(ftd_heat** out, int nx, int ny, int nz, const int* pa
     }
     for (int d = 0; d < 3; ++d) {
         ftd_status st = ftd_create(&h->solver[d], kind, ns[d], nr[d], h->parts[d], dt, h->stream);
-        if (st == FTD_OK) st = sync_solver_plan(h, d);
+        if (st == FTD_OK) {
+            ftd::handle_keep_thomas(h->solver[d]);
+            st = sync_solver_plan(h, d);
+        }
         if (st != FTD_OK) {
             std::string m = ftd_last_error_string();
             ftd_heat_destroy(h);

@@ -170,6 +170,9 @@ hipError_t launch_gen_filtered_final(const double* A, const double* C, double* D
 // the guard switched on (those run on the handle's own solve).
 struct ftd_handle;
 namespace ftd {
+// one partition of up to 64 rows solved by plain Thomas at every batch size
+// (the heat step, whose fused sweeps are the same Thomas)
+void handle_keep_thomas(ftd_handle* h);
 int handle_filtered_state(ftd_handle* h, int** J, const double** rho, double* eps_value,
                           int* eps_direct);
 }  // namespace ftd

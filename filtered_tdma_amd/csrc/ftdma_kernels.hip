@@ -2554,18 +2554,25 @@ hipError_t launch_pascal_fused(int M, int maxt, const double* A, const double* B
                                                         cyclic, csh, st);
 }
 
+// (float rows are whole lines from 32 systems on)
 hipError_t launch_pascal_fused_f32c(int M, int maxt, const float* A, const float* B,
                                     const float* C, double* D, int n_sys, int n_row, int Q, int S,
                                     int cyclic, hipStream_t st) {
-    return launch_pascal_fused_t<float, double, true>(M, maxt, A, B, C, D, D, n_sys, n_row, Q, S,
-                                                cyclic, 0, st);
+    return n_sys % 32 == 0
+               ? launch_pascal_fused_t<float, double, true>(M, maxt, A, B, C, D, D, n_sys, n_row,
+                                                            Q, S, cyclic, 0, st)
+               : launch_pascal_fused_t<float, double, false>(M, maxt, A, B, C, D, D, n_sys, n_row,
+                                                             Q, S, cyclic, 0, st);
 }
 
 hipError_t launch_pascal_fused_f32(int M, int maxt, const float* A, const float* B, const float* C,
                                    const float* D, double* X, int n_sys, int n_row, int Q, int S,
                                    int cyclic, hipStream_t st) {
-    return launch_pascal_fused_t<float, float, true>(M, maxt, A, B, C, D, X, n_sys, n_row, Q, S, cyclic,
-                                               0, st);
+    return n_sys % 32 == 0
+               ? launch_pascal_fused_t<float, float, true>(M, maxt, A, B, C, D, X, n_sys, n_row,
+                                                           Q, S, cyclic, 0, st)
+               : launch_pascal_fused_t<float, float, false>(M, maxt, A, B, C, D, X, n_sys, n_row,
+                                                            Q, S, cyclic, 0, st);
 }
 
 hipError_t launch_pascal_ir(int M, int maxt, const float* A, const float* B, const float* C,

@@ -75,7 +75,8 @@ ftd_status ftd_destroy(ftd_handle* h);
 
 /* TdmaBackendGPU::solve (tdma_backend_gpu.cu:35-46):
  * FILTERED -> solve_filtered_v1, FILTERED_V2 -> solve_filtered_v2,
- * PASCAL -> PaScaLTDMACUDA::solve; partitions == 1 -> plain Thomas. */
+ * PASCAL -> PaScaLTDMACUDA::solve; partitions == 1 -> plain Thomas, or above
+ * 32 rows PaScaL over the engine's own partitions (exact to rounding). */
 ftd_status ftd_solve(ftd_handle* h, double* A, double* B, double* C, double* D);
 
 /* PaScaLTDMACUDA::solve(A, B, C, D, n_sys, n_row) (pascal_tdma_cuda.hpp:28-29):

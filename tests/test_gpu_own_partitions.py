@@ -72,6 +72,18 @@ def test_own_partitions_bitwise(n_sys, n_row, cyclic):
     check(n_sys, n_row, cyclic=cyclic)
 
 
+@pytest.mark.parametrize("n_sys,n_row", [(1, 33), (1000, 48), (16385, 64)])
+def test_short_rows_of_a_small_batch(n_sys, n_row):
+    """33 to 64 rows below 131072 systems: 16-row partitions; the periodic
+    solve stays Sherman-Morrison Thomas."""
+    path = check(n_sys, n_row)[5]
+    assert path.startswith("pascal_fused M=16"), path
+    A, B, C, D = cases.general_batch(n_sys, n_row, seed=2)
+    x, path, _ = solve(A, B, C, D, cyclic=True)
+    assert path.startswith("thomas_cyclic"), path
+    np.testing.assert_array_equal(x, O.thomas(A, B, C, D, sem=O.SEM_GPU, cyclic=True))
+
+
 @pytest.mark.parametrize("cyclic", [False, True])
 @pytest.mark.parametrize("n_sys,n_row", [
     (8192, 513), (8193, 1024),             # 16 systems per tile, last tile of 1
@@ -95,6 +107,41 @@ def test_caller_partitions_longer_than_a_lane(n_sys, n_row, P):
 @pytest.mark.parametrize("n_sys,n_row", [(2048, 100), (512, 300), (33, 1100), (2048, 2100)])
 def test_own_partitions_at_element_alignment(n_sys, n_row):
     check(n_sys, n_row, shift=1)
+
+
+@pytest.mark.parametrize("cyclic", [False, True])
+@pytest.mark.parametrize("n_sys,n_row", [(131072, 33), (33, 32), (5, 3)])
+def test_thomas_where_it_stays(n_sys, n_row, cyclic):
+    A, B, C, D = cases.general_batch(n_sys, n_row, seed=9)
+    note(f"thomas n_sys={n_sys} n_row={n_row} cyclic={cyclic}")
+    x, path, _ = solve(A, B, C, D, cyclic=cyclic)
+    assert path.startswith("thomas"), path
+    np.testing.assert_array_equal(x, O.thomas(A, B, C, D, sem=O.SEM_GPU, cyclic=cyclic))
+
+
+@pytest.mark.parametrize("d32", [False, True])
+@pytest.mark.parametrize("n_sys,n_row", [(100, 40), (2048, 100), (16400, 256), (16416, 256),
+                                         (8200, 300), (9000, 600)])
+def test_f32_storage_own_partitions(n_sys, n_row, d32):
+    A, B, C, D, _ = cases.toeplitz_batch(n_sys, n_row, 5.0, 500.0, seed=4)
+    f = [v.astype(np.float32) for v in (A, B, C)]
+    D32 = D.astype(np.float32) if d32 else D
+    note(f"f32 own partitions n_sys={n_sys} n_row={n_row} d32={d32}")
+    be = TdmaBackendGPU(Kind.PASCAL, n_sys, n_row, 1)
+    try:
+        t = [torch.from_numpy(v).cuda() for v in f]
+        tD = torch.from_numpy(D32.copy()).cuda()
+        X = torch.empty((n_row, n_sys), dtype=torch.float64, device="cuda") if d32 else tD
+        if d32:
+            be.solve_f32(*t, tD, X)
+        else:
+            be.solve_f32c(*t, X)
+        torch.cuda.synchronize()
+        x, path = X.cpu().numpy(), be.last_path()
+    finally:
+        be.close()
+    w = [v.astype(np.float64) for v in f] + [D32.astype(np.float64)]
+    np.testing.assert_array_equal(x, O.pascal(*w, path_Q(path), sem=O.SEM_GPU), err_msg=path)
 
 
 def test_beyond_the_long_system_kernel():
