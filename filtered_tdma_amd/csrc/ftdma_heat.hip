@@ -266,88 +266,212 @@ __device__ __forceinline__ void adi_row(bool first, bool last, double sa, double
     }
 }
 
-// d of row j of one partition (rows past the partition repeat its last
-// row, so the load carries no branch and can be issued ahead of its use)
+// A cell of a lane as a base that is the same for the whole wave (the first
+// lane's cell) and the lane's byte offset from it: with a uniform row index the
+// row's address is then scalar arithmetic, and the load takes the offset from
+// one register (the lanes of a wave hold consecutive systems, a few lines or
+// planes at most, so 32 bits hold it).
+template <typename T>
+struct LaneCell {
+    T* base;
+    uint32_t off;
+    __device__ __forceinline__ LaneCell(T* field, size_t at) {
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)at);
+        const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(at >> 32));
+        const size_t first = ((size_t)hi << 32) | lo;
+        base = field + first;
+        off = (uint32_t)((at - first) * sizeof(T));
+    }
+    __device__ __forceinline__ T& operator[](ptrdiff_t o) const {
+        return *(T*)((char*)(base + o) + off);
+    }
+    __device__ __forceinline__ LaneCell& operator+=(ptrdiff_t o) {
+        base += o;
+        return *this;
+    }
+};
+
+// d of row j of one partition, asked for in order (j = 0, 1, ...): p points at
+// the next row (rows past the partition repeat its last row, so the load carries
+// no branch and can be issued ahead of its use)
+template <typename P>
 struct RowAt {
-    const double* p;
-    size_t rs;
+    P p;
+    ptrdiff_t rs;
     int cnt;
-    __device__ __forceinline__ double operator()(int j) const {
-        const int jj = j < cnt ? j : cnt - 1;
-        return p[(size_t)jj * rs];
+    __device__ __forceinline__ double operator()(int j) {
+        const double v = p[0];
+        p += j + 1 < cnt ? rs : 0;
+        return v;
     }
 };
 
 // d of row j of one z partition formed from th as k_rhs_z forms it (the
-// z sweep then needs no rhs pass): c0 is the cell of the partition's first
-// row, k0 its z index; rows past the partition repeat its last row
-// Rows are formed in order (j = 0, 1, ...), so th at z - 1, z, z + 1 rolls
-// through zm, z0, zp: one z load per row instead of three. Rows past the
+// z sweep then needs no rhs pass): c is the cell of the next row, cz the
+// table at its z; rows past the partition repeat its last row. Rows are formed
+// in order (j = 0, 1, ...), so th at z - 1, z, z + 1
+// rolls through zm, z0, zp: one z load per row instead of three. Rows past the
 // partition (j >= cnt) repeat its last row, as the clamped index does; the
 // roll is by selects, not a branch (the lanes of a wave may hold partitions
 // of different lengths).
+template <typename P>
 struct RowRhsZ {
-    const double* th;
+    P c;
     const double* cz;
-    size_t c0, sy, sz;
-    int cnt, k0;
+    ptrdiff_t sy, sz;
+    int cnt;
     double xa, xc, ya, yc, za, zc, diag, cxy;
     double zm = 0.0, z0 = 0.0, zp = 0.0;
     __device__ __forceinline__ double operator()(int j) {
-        const int jj = j < cnt ? j : cnt - 1;
-        const size_t c = c0 + (size_t)jj * sz;
         if (j == 0) {
-            zm = th[c - sz];
-            z0 = th[c];
-            zp = th[c + sz];
+            zm = c[-sz];
+            z0 = c[0];
+            zp = c[sz];
         } else {
             const bool adv = j < cnt;
-            const double nzp = th[c + sz];
+            const double nzp = c[sz];
             zm = adv ? z0 : zm;
             z0 = adv ? zp : z0;
             zp = adv ? nzp : zp;
         }
-        return (xc * th[c + 1] + xa * th[c - 1]) + (yc * th[c + sy] + ya * th[c - sy]) +
-               (zc * zp + za * zm) + diag * z0 + cxy * cz[k0 + jj];
+        const double v = (xc * c[1] + xa * c[-1]) + (yc * c[sy] + ya * c[-sy]) +
+                         (zc * zp + za * zm) + diag * z0 + cxy * cz[0];
+        const bool more = j + 1 < cnt;
+        c += more ? sz : 0;
+        cz += more ? 1 : 0;
+        return v;
     }
 };
 
-// One lane per (system, partition) with the partition's rows in registers.
-// rows(j) returns d of local row j (clamped to the partition), Store(j, x)
-// writes x of local row j. The d loads run PF rows ahead of their use. Restates k_thomas_fused (Q == 1) and
-// k_pascal_fused (Q >= 2, non-cyclic): rows 0, 1 of a partition divided by
-// b, modified elimination, 2Q-row reduced system in LDS, interior update.
-template <int M, int PF, bool THOMAS, typename Rows, typename Store>
-__device__ __forceinline__ void adi_solve_lane(int N, int Q, int q, int r0, int cnt, int S, int sl,
-                                               double sa, double sb, double sc,
-                                               const double* __restrict__ th, size_t lo,
+// The elimination of a sweep's rows is the same for every system: the
+// coefficients are the stencil's constants, with the wall rows' b. Its factors
+// are therefore formed once, when the sweep is planned (adi_table, on the
+// host, by the statements the solve would run per system: the same bits), and a
+// lane carries only d. That takes the divisions and two thirds of the
+// registers out of the sweeps: a whole partition's loads fit in flight, four
+// waves per SIMD. At 256^3 the y sweep went from 58.7 to 50.9 us (5.3 TB/s), the
+// z sweep from 92.6 to 88 (its five stencil loads a row), at 64^3 y from 12.0 to
+// 9.2 and x from 17.6 to 14.5 (one wave's instructions on a part of the CUs); the
+// 256^3 x sweep stays at 77 (its LDS tile's copy-in, solve and copy-out).
+//
+// Row j of partition q at tab[q * M + j]:
+//   inv   1 / (b - a c'_{j-1}); the rows that are divided by b (0 and 1 of a
+//         partition; only 0 in the plain Thomas): b itself
+//   cf    c' of the forward sweep
+//   a, c  a', c' after the backward sweep; row 0: a = 1 / (1 - a'_1 c'_0)
+// then the 2Q rows of the reduced system: inv, a, and c' (in cf).
+struct AdiRow {
+    double inv, cf, a, c;
+};
+
+// value v of lane `lane` (uniform), as a scalar
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// A wave's part of the table. With S >= 64 systems per workgroup a wave holds
+// one partition (SPAN 1): lane l keeps row l and the rows reach the others by
+// v_readlane, with no load in the chain of rows (scalar loads there cost a
+// round trip per few rows). At S = 32 and up to 32 rows it holds two (SPAN 2):
+// rows of the lower in lanes 0..31, of the upper in 32..63, each lane takes its
+// own. Else (SPAN 0) each lane loads its own rows. Made with every lane of the
+// wave active, in workgroups of whole waves for SPAN 1.
+template <int M, int SPAN>
+struct AdiTable {
+    AdiRow own;        // SPAN 1, 2: this lane's row
+    AdiRow red;        // SPAN 1, 2: row l of the reduced system
+    const AdiRow* p;   // SPAN 0: the partition's rows
+    const AdiRow* rp;  // SPAN 0: the reduced rows
+    bool upper;
+    __device__ __forceinline__ AdiTable(const AdiRow* __restrict__ tab, int q, int Q) {
+        const int l = threadIdx.x & 63;
+        if (SPAN == 0) {
+            p = tab + q * M;
+            rp = tab + Q * M;
+            upper = false;
+        } else {
+            const int q0 = __builtin_amdgcn_readfirstlane(q);
+            const int part = SPAN == 2 && l >= 32 && q0 + 1 < Q ? q0 + 1 : q0;
+            const int row = SPAN == 2 ? l & 31 : l;
+            own = tab[part * M + (row < M ? row : M - 1)];
+            red = tab[Q * M + (l < 2 * Q ? l : 0)];
+            upper = SPAN == 2 && l >= 32;
+            // every lane's rows are here now: the loads must not sink into a
+            // branch that some lanes skip
+            asm volatile("" : "+v"(own.inv), "+v"(own.cf), "+v"(own.a), "+v"(own.c));
+            asm volatile("" : "+v"(red.inv), "+v"(red.cf), "+v"(red.a));
+        }
+    }
+    __device__ __forceinline__ double get(double AdiRow::* f, int j) const {
+        if (SPAN == 0) return p[j].*f;
+        const double lo = lane_value(own.*f, j);
+        if (SPAN == 1) return lo;
+        const double hi = lane_value(own.*f, 32 + (j & 31));
+        return upper ? hi : lo;
+    }
+    __device__ __forceinline__ double inv(int j) const { return get(&AdiRow::inv, j); }
+    __device__ __forceinline__ double cf(int j) const { return get(&AdiRow::cf, j); }
+    __device__ __forceinline__ double a(int j) const { return get(&AdiRow::a, j); }
+    __device__ __forceinline__ double c(int j) const { return get(&AdiRow::c, j); }
+    __device__ __forceinline__ double rget(double AdiRow::* f, int k) const {
+        return SPAN == 0 ? rp[k].*f : lane_value(red.*f, k);
+    }
+    __device__ __forceinline__ double rinv(int k) const { return rget(&AdiRow::inv, k); }
+    __device__ __forceinline__ double ra(int k) const { return rget(&AdiRow::a, k); }
+    __device__ __forceinline__ double rcf(int k) const { return rget(&AdiRow::cf, k); }
+};
+
+// One lane per (system, partition) with d of the partition's rows in
+// registers. rows(j) returns d of local row j (clamped to the partition),
+// store(j, x) writes x of local row j. The d loads run PF rows ahead of their
+// use (by value: a reference kept a row source's rolling state in scratch).
+// Restates k_thomas_fused (Q == 1) and k_pascal_fused (Q >= 2, non-cyclic):
+// rows 0, 1 of a partition divided by b, modified elimination,
+// 2Q-row reduced system in LDS, interior update.
+// where a wave's lanes have one row count (SPAN 1), the row tests are scalar
+// branches; the statement keeps the compiler from turning them into selects
+#define FTD_ADI_BRANCH \
+    if (SPAN == 1) asm volatile("")
+template <int M, int PF, bool THOMAS, int SPAN, typename Rows, typename Store>
+__device__ __forceinline__ void adi_solve_lane(int Q, int q, int cnt, int S, int sl, double sa,
+                                               double sc, const double* __restrict__ th, size_t lo,
                                                size_t hi, size_t rs, bool live, double* lds,
-                                               Rows& rows, Store store) {
-    double rd[M];
-#define FTD_ADI_LOAD(j) rd[(j)] = rows(j)
+                                               const AdiTable<M, SPAN>& T, Rows rows,
+                                               Store store) {
+    const double aj = -sa;
+    double d[M];
+    // the wall fold-in of the system's first and last rows
+    const double wl = (THOMAS || q == 0) ? sa * (th[lo - rs] + th[lo]) : 0.0;
+    const double wh = (THOMAS || q == Q - 1) ? sc * (th[hi + rs] + th[hi]) : 0.0;
 #pragma unroll
-    for (int j = 0; j < PF && j < M; ++j) FTD_ADI_LOAD(j);
+    for (int j = 0; j < PF && j < M; ++j) d[j] = rows(j);
+    double dN = 0.0;
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+        if (j + PF < M) d[j + PF] = rows(j + PF);
+        const double k = T.inv(j);  // (taken where every lane is active)
+        if (j < cnt) {
+            FTD_ADI_BRANCH;
+            double dj = d[j];
+            if (j == 0) dj = q == 0 ? dj + wl : dj;
+            if (j >= 2) dj = (j == cnt - 1 && q == Q - 1) ? dj + wh : dj;
+            if (j < (THOMAS ? 1 : 2))
+                d[j] = dj / k;
+            else
+                d[j] = k * (dj - aj * d[j >= 1 ? j - 1 : 0]);
+            if (!THOMAS && j == cnt - 1) dN = d[j];
+        }
+    }
     if (THOMAS) {
-        double c[M], d[M];
 #pragma unroll
-        for (int j = 0; j < M; ++j) {
-            if (j + PF < M) FTD_ADI_LOAD(j + PF);
-            if (j < cnt) {
-                double aj, bj, cj, dj;
-                adi_row(j == 0, j == cnt - 1, sa, sb, sc, rd[j], th, lo, hi, rs, aj, bj, cj, dj);
-                if (j == 0) {
-                    d[0] = dj / bj;
-                    c[0] = cj / bj;
-                } else {
-                    const double r = 1.0 / (bj - aj * c[j - 1]);
-                    d[j] = r * (dj - aj * d[j - 1]);
-                    c[j] = r * cj;
-                }
+        for (int j = M - 2; j >= 0; --j) {
+            const double k = T.cf(j);
+            if (j <= cnt - 2) {
+                FTD_ADI_BRANCH;
+                d[j] = d[j] - k * d[j + 1];
             }
         }
-#pragma unroll
-        for (int j = M - 2; j >= 0; --j)
-            if (j <= cnt - 2) d[j] = d[j] - c[j] * d[j + 1];
         if (live) {
 #pragma unroll
             for (int j = 0; j < M; ++j)
@@ -355,142 +479,90 @@ __device__ __forceinline__ void adi_solve_lane(int N, int Q, int q, int r0, int 
         }
         return;
     }
-    double a[M], c[M], d[M];
-    double aN = 0.0, cN = 0.0, dN = 0.0;
-#pragma unroll
-    for (int j = 0; j < M; ++j) {
-        if (j + PF < M) FTD_ADI_LOAD(j + PF);
-        if (j < cnt) {
-            double aj, bj, cj, dj;
-            // the system's first row is row 0 of partition 0, its last row the
-            // last row of partition Q-1
-            adi_row(j == 0 && q == 0, j == cnt - 1 && q == Q - 1, sa, sb, sc, rd[j], th, lo, hi,
-                    rs, aj, bj, cj, dj);
-            if (j < 2) {
-                a[j] = aj / bj;
-                c[j] = cj / bj;
-                d[j] = dj / bj;
-            } else {
-                const double inv = 1.0 / (bj - aj * c[j - 1]);
-                d[j] = inv * (dj - aj * d[j - 1]);
-                c[j] = inv * cj;
-                a[j] = -inv * aj * a[j - 1];
-            }
-            if (j == cnt - 1) {
-                aN = a[j];
-                cN = c[j];
-                dN = d[j];
-            }
-        }
-    }
 #pragma unroll
     for (int j = M - 3; j >= 1; --j) {
+        const double k = T.cf(j);
         if (j <= cnt - 3) {
-            const double cj = c[j];
-            d[j] = d[j] - cj * d[j + 1];
-            a[j] = a[j] - cj * a[j + 1];
-            c[j] = -cj * c[j + 1];
+            FTD_ADI_BRANCH;
+            d[j] = d[j] - k * d[j + 1];
         }
     }
-    const double r = 1.0 / (1.0 - a[1] * c[0]);
-    const double d0 = r * (d[0] - c[0] * d[1]);
-    const double a0 = r * a[0];
-    const double c0 = -r * c[0] * c[1];
+    const double d0 = T.a(0) * (d[0] - T.cf(0) * d[1]);
     const int NR = 2 * Q;
-    double* rA = lds;
-    double* rC = rA + NR * S;
-    double* rD = rC + NR * S;
-    rA[(2 * q) * S + sl] = a0;
-    rC[(2 * q) * S + sl] = c0;
-    rD[(2 * q) * S + sl] = d0;
-    rA[(2 * q + 1) * S + sl] = aN;
-    rC[(2 * q + 1) * S + sl] = cN;
-    rD[(2 * q + 1) * S + sl] = dN;
+    lds[(2 * q) * S + sl] = d0;
+    lds[(2 * q + 1) * S + sl] = dN;
     __syncthreads();
     if (q == 0) {
         // the reduced rows 4 at a time: their values are read into registers
-        // first and c', d' are carried in registers, so the serial chain is
-        // the arithmetic, not a round trip through LDS per row
-        double* Ar = rA + sl;
-        double* Cr = rC + sl;
-        double* Dr = rD + sl;
-        double cp = Cr[0], dp = Dr[0];
+        // first, so the serial chain is the arithmetic, not a round trip
+        // through LDS per row
+        double* Dr = lds + sl;
+        double dp = Dr[0];
         int k = 1;
         for (; k + 4 <= NR; k += 4) {
-            double ak[4], ck[4], dk[4];
+            double dk[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) dk[u] = Dr[(k + u) * S];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                ak[u] = Ar[(k + u) * S];
-                ck[u] = Cr[(k + u) * S];
-                dk[u] = Dr[(k + u) * S];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const double inv = 1.0 / (1.0 - ak[u] * cp);
-                dp = inv * (dk[u] - ak[u] * dp);
-                cp = inv * ck[u];
+                dp = T.rinv(k + u) * (dk[u] - T.ra(k + u) * dp);
                 Dr[(k + u) * S] = dp;
-                Cr[(k + u) * S] = cp;
             }
         }
         for (; k < NR; ++k) {
-            const double ak = Ar[k * S];
-            const double inv = 1.0 / (1.0 - ak * cp);
-            dp = inv * (Dr[k * S] - ak * dp);
-            cp = inv * Cr[k * S];
+            dp = T.rinv(k) * (Dr[k * S] - T.ra(k) * dp);
             Dr[k * S] = dp;
-            Cr[k * S] = cp;
         }
         double dn = dp;
         k = NR - 2;
         for (; k >= 3; k -= 4) {
-            double ck[4], dk[4];
+            double dk[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) dk[u] = Dr[(k - u) * S];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                ck[u] = Cr[(k - u) * S];
-                dk[u] = Dr[(k - u) * S];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                dn = dk[u] - ck[u] * dn;
+                dn = dk[u] - T.rcf(k - u) * dn;
                 Dr[(k - u) * S] = dn;
             }
         }
         for (; k >= 0; --k) {
-            dn = Dr[k * S] - Cr[k * S] * dn;
+            dn = Dr[k * S] - T.rcf(k) * dn;
             Dr[k * S] = dn;
         }
     }
     __syncthreads();
-    const double x0 = rD[(2 * q) * S + sl];
-    const double xN = rD[(2 * q + 1) * S + sl];
-    if (live) {
+    const double x0 = lds[(2 * q) * S + sl];
+    const double xN = lds[(2 * q + 1) * S + sl];
 #pragma unroll
-        for (int j = 0; j < M; ++j) {
-            if (j < cnt) {
-                double x;
-                if (j == 0)
-                    x = x0;
-                else if (j == cnt - 1)
-                    x = xN;
-                else
-                    x = d[j] - (a[j] * x0 + c[j] * xN);
-                store(j, x);
-            }
+    for (int j = 0; j < M; ++j) {
+        const double ka = T.a(j), kc = T.c(j);
+        if (live && j < cnt) {
+            double x;
+            if (j == 0)
+                x = x0;
+            else if (j == cnt - 1)
+                x = xN;
+            else
+                x = d[j] - (ka * x0 + kc * xN);
+            store(j, x);
         }
     }
-#undef FTD_ADI_LOAD
 }
+
+// threads of a y or z sweep's workgroup at most: 16- and 32-row lanes that read
+// d fit 16 waves a CU (128 registers), 64-row ones and those that form it 8
+constexpr int adi_threads(int M, bool rhsz) { return M >= 64 || rhsz ? 512 : 1024; }
 
 // Z (dir 2) and Y (dir 1) sweeps: systems consecutive in x, so a wave's row
 // loads are contiguous; rows strided by a plane (Z) or a line (Y). The
 // solution goes back into rhs. RHSZ (the z sweep, first of the step): d is
 // formed from th by the explicit stencil (RowRhsZ) instead of read from rhs,
 // so the step has no separate rhs pass; th is not written until the x sweep.
-template <int M, bool THOMAS, bool RHSZ>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(M >= 64 ? 1 : 2))) void k_adi_yz(const double* __restrict__ th, double* rhs, Dims g,
-                                                int nz, int dir, double sa, double sb, double sc,
-                                                int Q, int lgS, Stencil st,
+template <int M, bool THOMAS, bool RHSZ, int SPAN>
+__global__ __launch_bounds__(adi_threads(M, RHSZ)) void k_adi_yz(const double* __restrict__ th, double* rhs, Dims g,
+                                                int nz, int dir, double sa, double sc, int Q,
+                                                int lgS, Stencil st,
+                                                const AdiRow* __restrict__ tab,
                                                 const double* __restrict__ cx,
                                                 const double* __restrict__ cy,
                                                 const double* __restrict__ cz) {
@@ -498,7 +570,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(M >= 64 ? 1
     const int S = 1 << lgS;
     const int t = threadIdx.x;
     const int sl = t & (S - 1);
-    const int q = t >> lgS;
+    // SPAN 1: the wave's one partition, so its rows' bounds are scalar
+    const int q = SPAN == 1 ? __builtin_amdgcn_readfirstlane(t >> lgS) : t >> lgS;
     const int n_sys = g.nx * (dir == 2 ? g.ny : nz);
     const int N = dir == 2 ? nz : g.ny;
     // RHSZ reads th at x +- 1 and y +- 1: each XCD takes a contiguous run of
@@ -517,19 +590,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(M >= 64 ? 1
         r0 = q * base + (q < rem ? q : rem);
         cnt = base + (q < rem ? 1 : 0);
     }
-    double* const pbase = rhs + here0 + (size_t)r0 * rs;
+    LaneCell<double> first(rhs, here0);
+    first += (ptrdiff_t)((size_t)r0 * rs);
+    // x of row j, rows stored in order
+    LaneCell<double> out = first;
+    auto store = [&](int, double x) {
+        out[0] = x;
+        out += (ptrdiff_t)rs;
+    };
+    const AdiTable<M, SPAN> T(tab, q, Q);
     if (RHSZ) {
-        RowRhsZ rows{th, cz, here0 + (size_t)r0 * rs, (size_t)g.px, rs, cnt, r0 + 1,
+        LaneCell<const double> c0(th, here0);
+        c0 += (ptrdiff_t)((size_t)r0 * rs);
+        RowRhsZ<LaneCell<const double>> rows{c0, cz + r0 + 1, (ptrdiff_t)g.px, (ptrdiff_t)rs, cnt,
                      st.xa, st.xc, st.ya, st.yc, st.za, st.zc, 1.0 + st.xb + st.yb + st.zb,
                      st.c0 * cx[ii] * cy[oo]};
-        adi_solve_lane<M, (M >= 32 ? 2 : 4), THOMAS>(N, Q, q, r0, cnt, S, sl, sa, sb, sc, th, here0,
-                                     here0 + (size_t)(N - 1) * rs, rs, live, lds, rows,
-                                     [&](int j, double x) { pbase[(size_t)j * rs] = x; });
+        adi_solve_lane<M, 4, THOMAS, SPAN>(Q, q, cnt, S, sl, sa, sc, th, here0,
+                                           here0 + (size_t)(N - 1) * rs, rs, live, lds, T, rows,
+                                           store);
     } else {
-        RowAt rows{pbase, rs, cnt};
-        adi_solve_lane<M, (M == 16 ? 16 : M == 32 ? 8 : 4), THOMAS>(
-            N, Q, q, r0, cnt, S, sl, sa, sb, sc, th, here0, here0 + (size_t)(N - 1) * rs, rs,
-            live, lds, rows, [&](int j, double x) { pbase[(size_t)j * rs] = x; });
+        RowAt<LaneCell<double>> rows{first, (ptrdiff_t)rs, cnt};
+        adi_solve_lane<M, M, THOMAS, SPAN>(
+            Q, q, cnt, S, sl, sa, sc, th, here0, here0 + (size_t)(N - 1) * rs, rs, live, lds, T,
+            rows, store);
     }
 }
 
@@ -718,13 +801,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(M >= 64 ? 1
     const size_t lo = here0, hi = here0 + (size_t)(N - 1) * rs;
     double* const pbase = rhs + here0 + (size_t)r0 * rs;
     if constexpr (DIR == 2) {
-        RowRhsZ rows{th, cz, here0 + (size_t)r0 * rs, (size_t)g.px, rs, m, r0 + 1,
+        RowRhsZ<const double*> rows{th + here0 + (size_t)r0 * rs, cz + r0 + 1, (ptrdiff_t)g.px,
+                                    (ptrdiff_t)rs, m,
                      st.xa, st.xc, st.ya, st.yc, st.za, st.zc, 1.0 + st.xb + st.yb + st.zb,
                      st.c0 * cx[ii] * cy[oo]};
         filt_lane<M, VERSION, PASS>(rows, th, Q, q, S, sl, m, n_sys, s, live, sa, sb, sc, lo, hi,
                                     rs, pbase, Jp, xbuf, partial, blk, lds);
     } else {
-        RowAt rows{pbase, rs, m};
+        RowAt<const double*> rows{pbase, (ptrdiff_t)rs, m};
         filt_lane<M, VERSION, PASS>(rows, th, Q, q, S, sl, m, n_sys, s, live, sa, sb, sc, lo, hi,
                                     rs, pbase, Jp, xbuf, partial, blk, lds);
     }
@@ -791,14 +875,14 @@ __host__ __device__ inline int x_tile_stride(int N) { return N + 2 - (N & 1); }
 // workgroup first copies its S lines of rhs into an LDS tile (coalesced,
 // line stride x_tile_stride(N)), solves from the tile, writes x back into the tile and copies the tile to
 // theta (coalesced).
-template <int M, bool THOMAS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(M >= 64 ? 1 : 2))) void k_adi_x(double* th, const double* __restrict__ rhs, Dims g,
-                                               int nz, double sa, double sb, double sc, int Q,
-                                               int lgS) {
+template <int M, bool THOMAS, int SPAN>
+__global__ __launch_bounds__(256) void k_adi_x(double* th, const double* __restrict__ rhs, Dims g,
+                                               int nz, double sa, double sc, int Q, int lgS,
+                                               const AdiRow* __restrict__ tab) {
     extern __shared__ double lds[];
     const int S = 1 << lgS;
     const int t = threadIdx.x;
-    const int T = blockDim.x;
+    const int nt = blockDim.x;
     const int sl = t & (S - 1);
     const int q = t >> lgS;
     const int n_sys = g.ny * nz;
@@ -815,7 +899,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(M >= 64 ? 1
     // cells start on 128-byte boundaries, tile lines on 16-byte ones), so
     // every line of the tile is in flight at once with no register staging
     // and a wave's DMAs stay under the count of operations it can track.
-    const int step = T < 64 ? T : 64, nw = T / step, w = t / step, lane = t - w * step;
+    const int step = nt < 64 ? nt : 64, nw = nt / step, w = t / step, lane = t - w * step;
     const int nu = N >> 1;  // 16-byte units per line; an odd N leaves 8 bytes
     for (int l = w < nw ? w : nl; l < nl; l += nw) {
         const int s = first + l;
@@ -834,26 +918,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(M >= 64 ? 1
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    // threads past S * Q (a Thomas tile of fewer than 64 lines is launched as
-    // one full wave, so that its copies use 64 lanes) only copy: the Thomas
-    // solve has no barrier
-    if (q < Q) {
+    const AdiTable<M, SPAN> T(tab, THOMAS ? 0 : q, Q);
+    {
+        // threads past S * Q (a Thomas tile of fewer than 64 lines is launched
+        // as one full wave, so that its copies use 64 lanes and hold the
+        // factor table) solve a line along, as dead lanes do
         const int s_raw = first + sl;
-        const bool live = s_raw < n_sys;
+        const bool live = s_raw < n_sys && q < Q;
         const int s = live ? s_raw : n_sys - 1;
+        const int qq = THOMAS ? 0 : SPAN == 1 ? __builtin_amdgcn_readfirstlane(q) : q;
         const size_t here0 = cell(g, 1, s % g.ny + 1, s / g.ny + 1);
         int r0, cnt;
         {
             const int base = N / Q, rem = N % Q;
-            r0 = q * base + (q < rem ? q : rem);
-            cnt = base + (q < rem ? 1 : 0);
+            r0 = qq * base + (qq < rem ? qq : rem);
+            cnt = base + (qq < rem ? 1 : 0);
         }
         const int lt = live ? sl : 0;  // dead lanes read a loaded line
         double* myline = tile + (size_t)lt * LS + r0;
-        RowAt rows{myline, 1, cnt};
-        adi_solve_lane<M, 2, THOMAS>(
-            N, Q, q, r0, cnt, S, sl, sa, sb, sc, th, here0, here0 + (size_t)(N - 1), 1, live, red,
-            rows, [&](int j, double x) { myline[j] = x; });
+        RowAt<const double*> rows{myline, 1, cnt};
+        adi_solve_lane<M, (M < 32 ? M : 32), THOMAS, SPAN>(
+            Q, qq, cnt, S, sl, sa, sc, th, here0, here0 + (size_t)(N - 1), 1, live, red, T, rows,
+            [&](int j, double x) { myline[j] = x; });
     }
     __syncthreads();
     for (int l = w < nw ? w : nl; l < nl; l += nw) {
@@ -941,6 +1027,7 @@ struct ftd_heat {
         int on = 0, M = 0, thomas = 0, Q = 0, lgS = 0;
         size_t lds = 0;
     } fused[3];
+    AdiRow* coef[3] = {nullptr, nullptr, nullptr};  // elimination factors of the fused sweeps
     // fused y, z sweeps of the filtered kinds over the caller's partitions
     // (k_adi_filt): enabled, rows per lane, partitions, log2 systems per
     // workgroup, dynamic LDS bytes of the exchange (x stays materialized)
@@ -954,6 +1041,79 @@ struct ftd_heat {
 };
 
 namespace {
+
+// entries of a sweep's factor table at most: 16 partitions of 64 rows, the
+// reduced rows, and the rows a wave's upper half may read past the last
+constexpr size_t kCoefRows = 16 * 64 + 2 * 16 + 64;
+
+// The elimination factors of a planned sweep (AdiRow), by the statements
+// that k_thomas_fused and k_pascal_fused run on its rows.
+void adi_table(int N, int Q, int M, bool thomas, double sa, double sb, double sc,
+               std::vector<AdiRow>& tab) {
+    tab.assign((size_t)Q * M + 2 * Q, AdiRow{1.0, 0.0, 0.0, 0.0});
+    std::vector<double> a(M), c(M), ra(2 * Q), rc(2 * Q);
+    for (int q = 0; q < Q; ++q) {
+        const int base = N / Q, rem = N % Q, cnt = base + (q < rem ? 1 : 0);
+        AdiRow* const t = &tab[(size_t)q * M];
+        for (int j = 0; j < cnt; ++j) {
+            const double aj = -sa, cj = -sc;
+            double bj = 1.0 - sb;
+            if (j == 0 && q == 0) bj += sa;
+            if (j == cnt - 1 && q == Q - 1) bj += sc;
+            if (j < (thomas ? 1 : 2)) {
+                t[j].inv = bj;
+                a[j] = aj / bj;
+                c[j] = cj / bj;
+            } else {
+                const double inv = 1.0 / (bj - aj * c[j - 1]);
+                t[j].inv = inv;
+                c[j] = inv * cj;
+                a[j] = -inv * aj * a[j - 1];
+            }
+            t[j].cf = c[j];
+        }
+        if (thomas) continue;
+        ra[2 * q + 1] = a[cnt - 1];
+        rc[2 * q + 1] = c[cnt - 1];
+        for (int j = cnt - 3; j >= 1; --j) {
+            const double cj = c[j];
+            a[j] = a[j] - cj * a[j + 1];
+            c[j] = -cj * c[j + 1];
+        }
+        const double r = 1.0 / (1.0 - a[1] * c[0]);
+        ra[2 * q] = r * a[0];
+        rc[2 * q] = -r * c[0] * c[1];
+        for (int j = 1; j < cnt; ++j) {
+            t[j].a = a[j];
+            t[j].c = c[j];
+        }
+        t[0].a = r;
+    }
+    if (thomas) return;
+    AdiRow* const t = &tab[(size_t)Q * M];
+    double cp = rc[0];
+    t[0].cf = cp;
+    for (int k = 1; k < 2 * Q; ++k) {
+        const double inv = 1.0 / (1.0 - ra[k] * cp);
+        cp = inv * rc[k];
+        t[k].inv = inv;
+        t[k].a = ra[k];
+        t[k].cf = cp;
+    }
+}
+
+// forms and uploads the factors of direction d's fused sweep (no step is in
+// flight: steps are waited for)
+hipError_t upload_table(ftd_heat* h, int d) {
+    const ftd_heat::Fused& f = h->fused[d];
+    if (!f.on) return hipSuccess;
+    const int N[3] = {h->g.nx, h->g.ny, h->nz};
+    const double sa[3] = {h->s.xa, h->s.ya, h->s.za}, sb[3] = {h->s.xb, h->s.yb, h->s.zb},
+                 sc[3] = {h->s.xc, h->s.yc, h->s.zc};
+    std::vector<AdiRow> tab;
+    adi_table(N[d], f.Q, f.M, f.thomas != 0, sa[d], sb[d], sc[d], tab);
+    return hipMemcpy(h->coef[d], tab.data(), sizeof(AdiRow) * tab.size(), hipMemcpyHostToDevice);
+}
 
 // The partition count the sweep's solver picks for (N rows, P partitions):
 // P == 1 -> plain Thomas when N <= 64, else ceil(N / 64) internal
@@ -1011,7 +1171,7 @@ void plan_fused(ftd_heat* h, int d, int N, int n_sys, int rows_per_lane = 0,
     f.thomas = Q == 1;
     f.M = rows_per_lane ? rows_per_lane : m_max <= 16 ? 16 : m_max <= 32 ? 32 : 64;
     int S = systems_per_tile ? systems_per_tile : 64;
-    while (S * Q > 256) S >>= 1;
+    while (S * Q > (d == 0 ? 256 : adi_threads(f.M, d == 2))) S >>= 1;
     // x tiles: each workgroup copies its lines in, solves and copies them out
     // in one pass, so a grid of fewer tiles than CUs leaves CUs idle. Halve
     // the tile down to 16 lines until the grid covers the CUs (64^3: 256
@@ -1022,7 +1182,7 @@ void plan_fused(ftd_heat* h, int d, int N, int n_sys, int rows_per_lane = 0,
         while (S > 16 && (n_sys + S - 1) / S < cus) S >>= 1;
     }
     auto lds_of = [&](int S_) {
-        const size_t red = f.thomas ? 0 : (size_t)3 * 2 * Q * S_;
+        const size_t red = f.thomas ? 0 : (size_t)2 * Q * S_;
         const size_t tile = d == 0 ? (size_t)S_ * x_tile_stride(N) : 0;
         return sizeof(double) * (red + tile);
     };
@@ -1133,7 +1293,7 @@ hipError_t launch_filt(ftd_heat* h, int d, hipStream_t st) {
     return hipErrorInvalidValue;
 }
 
-template <int M, bool TH>
+template <int M, bool TH, int SPAN>
 hipError_t launch_adi_t(ftd_heat* h, int d, hipStream_t st) {
     const ftd_heat::Fused& f = h->fused[d];
     const Dims g = h->g;
@@ -1143,54 +1303,57 @@ hipError_t launch_adi_t(ftd_heat* h, int d, hipStream_t st) {
     // wave: the extra threads take part in the copies only
     const int T = d == 0 && TH && S * f.Q < 64 ? 64 : S * f.Q;
     const dim3 grid((n_sys + S - 1) / S), block(T);
-    const double sa[3] = {h->s.xa, h->s.ya, h->s.za}, sb[3] = {h->s.xb, h->s.yb, h->s.zb},
-                 sc[3] = {h->s.xc, h->s.yc, h->s.zc};
+    const double sa[3] = {h->s.xa, h->s.ya, h->s.za}, sc[3] = {h->s.xc, h->s.yc, h->s.zc};
     if (d == 0) {
-        hipLaunchKernelGGL((k_adi_x<M, TH>), grid, block, f.lds, st, h->th, h->rhs, g, h->nz,
-                           sa[0], sb[0], sc[0], f.Q, f.lgS);
+        hipLaunchKernelGGL((k_adi_x<M, TH, SPAN>), grid, block, f.lds, st, h->th, h->rhs, g, h->nz,
+                           sa[0], sc[0], f.Q, f.lgS, h->coef[0]);
     } else if (d == 2 && h->fuse_rhs) {
-        hipLaunchKernelGGL((k_adi_yz<M, TH, true>), grid, block, f.lds, st, h->th, h->rhs, g,
-                           h->nz, d, sa[d], sb[d], sc[d], f.Q, f.lgS, h->s, h->cx, h->cy, h->cz);
+        hipLaunchKernelGGL((k_adi_yz<M, TH, true, SPAN>), grid, block, f.lds, st, h->th, h->rhs, g,
+                           h->nz, d, sa[d], sc[d], f.Q, f.lgS, h->s, h->coef[d], h->cx, h->cy,
+                           h->cz);
     } else {
-        hipLaunchKernelGGL((k_adi_yz<M, TH, false>), grid, block, f.lds, st, h->th, h->rhs, g,
-                           h->nz, d, sa[d], sb[d], sc[d], f.Q, f.lgS, h->s, h->cx, h->cy, h->cz);
+        hipLaunchKernelGGL((k_adi_yz<M, TH, false, SPAN>), grid, block, f.lds, st, h->th, h->rhs,
+                           g, h->nz, d, sa[d], sc[d], f.Q, f.lgS, h->s, h->coef[d], h->cx, h->cy,
+                           h->cz);
     }
     return hipGetLastError();
 }
 
+// F<M, THOMAS, SPAN>: how a wave holds the factor table (AdiTable). Thomas x
+// tiles are launched as whole waves; y and z ones are where S >= 64.
+#define FTD_ADI_DISPATCH(F, f, ...)                                            \
+    do {                                                                       \
+        if ((f).M == 16) FTD_ADI_CASE(F, 16, f, __VA_ARGS__)                   \
+        if ((f).M == 32) FTD_ADI_CASE(F, 32, f, __VA_ARGS__)                   \
+        if ((f).M == 64) FTD_ADI_CASE(F, 64, f, __VA_ARGS__)                   \
+        return hipErrorInvalidValue;                                           \
+    } while (0)
+#define FTD_ADI_CASE(F, m_, f, ...)                                            \
+    return (f).thomas && (d == 0 || (f).lgS >= 6) ? F<m_, true, 1>(__VA_ARGS__) \
+           : (f).thomas                            ? F<m_, true, 0>(__VA_ARGS__) \
+           : (f).lgS >= 6                          ? F<m_, false, 1>(__VA_ARGS__) \
+           : (f).lgS == 5 && m_ <= 32 ? F<m_, false, m_ <= 32 ? 2 : 0>(__VA_ARGS__) \
+                                      : F<m_, false, 0>(__VA_ARGS__);
+
 hipError_t launch_adi(ftd_heat* h, int d, hipStream_t st) {
-    const ftd_heat::Fused& f = h->fused[d];
-#define FTD_ADI_CASE(m_)                                                              \
-    if (f.M == m_) return f.thomas ? launch_adi_t<m_, true>(h, d, st)                   \
-                                   : launch_adi_t<m_, false>(h, d, st);
-    FTD_ADI_CASE(16)
-    FTD_ADI_CASE(32)
-    FTD_ADI_CASE(64)
-#undef FTD_ADI_CASE
-    return hipErrorInvalidValue;
+    FTD_ADI_DISPATCH(launch_adi_t, h->fused[d], h, d, st);
 }
 
 // dynamic LDS above the default limit must be declared for the kernel
-template <int M, bool TH>
+template <int M, bool TH, int SPAN>
 hipError_t allow_lds_t(int d, size_t bytes) {
     if (d == 0)
-        return hipFuncSetAttribute((const void*)k_adi_x<M, TH>,
+        return hipFuncSetAttribute((const void*)k_adi_x<M, TH, SPAN>,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-    const hipError_t e = hipFuncSetAttribute((const void*)k_adi_yz<M, TH, false>,
+    const hipError_t e = hipFuncSetAttribute((const void*)k_adi_yz<M, TH, false, SPAN>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     if (e != hipSuccess || d != 2) return e;
-    return hipFuncSetAttribute((const void*)k_adi_yz<M, TH, true>,
+    return hipFuncSetAttribute((const void*)k_adi_yz<M, TH, true, SPAN>,
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
 hipError_t allow_lds(const ftd_heat::Fused& f, int d) {
-#define FTD_ADI_CASE(m_)                                                                     \
-    if (f.M == m_) return f.thomas ? allow_lds_t<m_, true>(d, f.lds) : allow_lds_t<m_, false>(d, f.lds);
-    FTD_ADI_CASE(16)
-    FTD_ADI_CASE(32)
-    FTD_ADI_CASE(64)
-#undef FTD_ADI_CASE
-    return hipErrorInvalidValue;
+    FTD_ADI_DISPATCH(allow_lds_t, f, d, f.lds);
 }
 
 // Dirichlet ghosts of every non-periodic face, one launch (grid z = face)
@@ -1300,7 +1463,9 @@ ftd_status sync_solver_plan(ftd_heat* h, int d) {
     const ftd_heat::Fused& f = h->fused[d];
     if (f.on && !f.thomas && h->parts[d] == 1) {
         const int T = f.M == 64 ? 256 : 512;
-        if (ftd_set_tuning(h->solver[d], f.M, T, 1 << f.lgS, f.Q) != FTD_OK)
+        int S = 1 << f.lgS;  // (the bits do not depend on the tile)
+        while (S > 64 || S * f.Q > T) S >>= 1;
+        if (ftd_set_tuning(h->solver[d], f.M, T, S, f.Q) != FTD_OK)
             return herr(FTD_ERR_UNSUPPORTED, std::string("sweep solver: ") + ftd_last_error_string());
         return FTD_OK;
     }
@@ -1365,6 +1530,8 @@ ftd_status ftd_heat_create(ftd_heat** out, int nx, int ny, int nz, const int* pa
     double** ins[] = {&h->A, &h->B, &h->C, &h->D};
     for (double** b : ins)
         if (e == hipSuccess) e = hipMalloc(b, nin * sizeof(double));
+    for (AdiRow** b : {&h->coef[0], &h->coef[1], &h->coef[2]})
+        if (e == hipSuccess) e = hipMalloc(b, kCoefRows * sizeof(AdiRow));
     if (e == hipSuccess) e = hipMalloc(&h->cx, (nx + 2) * sizeof(double));
     if (e == hipSuccess) e = hipMalloc(&h->cy, (ny + 2) * sizeof(double));
     if (e == hipSuccess) e = hipMalloc(&h->cz, (nz + 2) * sizeof(double));
@@ -1372,6 +1539,8 @@ ftd_status ftd_heat_create(ftd_heat** out, int nx, int ny, int nz, const int* pa
     if (e == hipSuccess) e = hipMemcpy(h->cy, h->cy_.data(), (ny + 2) * sizeof(double), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(h->cz, h->cz_.data(), (nz + 2) * sizeof(double), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemset(h->rhs, 0, ncell * sizeof(double));
+    for (AdiRow* b : h->coef)
+        if (e == hipSuccess) e = hipMemset(b, 0, kCoefRows * sizeof(AdiRow));
     if (e == hipSuccess) e = hipEventCreate(&h->e0);
     if (e == hipSuccess) e = hipEventCreate(&h->e1);
     if (e != hipSuccess) {
@@ -1388,6 +1557,10 @@ ftd_status ftd_heat_create(ftd_heat** out, int nx, int ny, int nz, const int* pa
         if (h->fused[d].on && h->fused[d].lds > 64 * 1024) {
             hipError_t ea = allow_lds(h->fused[d], d);
             if (ea != hipSuccess) h->fused[d].on = 0;
+        }
+        if ((e = upload_table(h, d)) != hipSuccess) {
+            ftd_heat_destroy(h);
+            return herr(FTD_ERR_HIP, std::string("ftd_heat_create: ") + hipGetErrorString(e));
         }
     }
     for (int d = 0; d < 3; ++d) {
@@ -1412,6 +1585,8 @@ ftd_status ftd_heat_destroy(ftd_heat* h) {
     if (h->graph) hipGraphDestroy(h->graph);
     for (ftd_handle* s : h->solver) ftd_destroy(s);
     for (double* p : {h->th, h->rhs, h->A, h->B, h->C, h->D, h->cx, h->cy, h->cz})
+        if (p) hipFree(p);
+    for (AdiRow* p : h->coef)
         if (p) hipFree(p);
     if (h->e0) hipEventDestroy(h->e0);
     if (h->e1) hipEventDestroy(h->e1);
@@ -1508,6 +1683,8 @@ ftd_status ftd_heat_set_plan(ftd_heat* h, int dir, int rows_per_lane, int system
     if (f.on && f.lds > 64 * 1024 && allow_lds(f, dir) != hipSuccess) f.on = 0;
     if ((rows_per_lane || systems_per_tile) && !f.on)
         return herr(FTD_ERR_UNSUPPORTED, "no fused sweep with this plan for this direction");
+    HH(hipStreamSynchronize(h->stream));
+    HH(upload_table(h, dir));
     ftd_status st = sync_solver_plan(h, dir);
     if (st != FTD_OK) return st;
     return ftd_heat_set_fused(h, h->use_fused);  // drops a captured step
