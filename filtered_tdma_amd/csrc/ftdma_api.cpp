@@ -1348,6 +1348,15 @@ const char* ftd_last_error_string(void) { return g_err.c_str(); }
 namespace ftd {
 void handle_keep_thomas(ftd_handle* h) { h->keep_thomas = 1; }
 
+bool handle_is_plain(const ftd_handle* h, hipStream_t st) {
+    return h->P == 1 && h->stream == st && !h->t_M && !h->force_general && !h->no_stream &&
+           !h->profiling;
+}
+
+void handle_note_path(ftd_handle* h, const char* path) {
+    std::snprintf(h->path, sizeof h->path, "%s", path);
+}
+
 int handle_filtered_state(ftd_handle* h, int** J, const double** rho, double* eps_value,
                           int* eps_direct) {
     if (!h || h->kind == FTD_KIND_PASCAL || h->P < 2 || !h->J || !h->rho)

@@ -11,31 +11,41 @@
 //   divergence   compute_rhs_ (:193-212)
 //   FFT x, y     plan_fwd_x_, plan_fwd_y_ (:110-135) as one 2-D D2Z
 //   z solve      solve_tdma_z_ (:400-464): a, c from the z metrics, the
-//                modified wavenumbers of :72-78, the (0, 0) mode pinned
+//                modified wavenumbers of :72-78, the (0, 0) mode pinned. With
+//                one caller partition k_mode_solve forms the coefficients as
+//                it solves (a, c of a row are the same for every mode), and the
+//                spectra's lines start on 128-byte boundaries
 //   inverse FFT  plan_bwd_y_, plan_bwd_x_ as one 2-D Z2D, scale 1/(nx ny)
 //   projection   project_ (:470-490) with dp's ghosts (Neumann in z,
 //                periodic in x and y, :512-526) read by index
 #include <hip/hip_runtime.h>
 #include <hipfft/hipfft.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <string>
 #include <vector>
 
 #include "../../include/ftdma.h"
+#include "ftdma_device.h"
+#include "ftdma_kernels.h"
 #include "ftdma_xcd.h"
 
 struct ftd_poisson {
     int nx = 0, ny = 0, nz = 0, nxh = 0, nm = 0;
+    int pitch = 0;  // modes from one line of the spectra to the next (0: no k_mode_solve)
     hipStream_t stream = nullptr;  // the caller's
-    hipfftHandle fwd = 0, bwd = 0;
-    int have_fwd = 0, have_bwd = 0;
+    // plans of lines of nxh modes back to back (ftd_solve_complex's layout) and
+    // of lines of `pitch` modes where that is another layout
+    hipfftHandle fwd[2] = {0, 0}, bwd[2] = {0, 0};
+    int have_fwd[2] = {0, 0}, have_bwd[2] = {0, 0};
     double* A = nullptr;    // [nz][nm] coefficients, built once
     double* B = nullptr;
     double* C = nullptr;
     double* rhs = nullptr;  // [nz][ny][nx]: divergence, then dp (unscaled)
-    double* hat = nullptr;  // [nz][ny][nxh] complex, interleaved (re, im)
+    double* coef = nullptr; // k_mode_solve: a, c, -(a + c) per row, kx2, ky2
+    double* hat = nullptr;  // [nz][ny][nxh or pitch] complex, interleaved (re, im)
     double* met = nullptr;  // dx, dmx [nx+2]; dy, dmy [ny+2]; dz, dmz [nz+2]
     ftd_handle* solver = nullptr;
     double scale = 1.0;
@@ -158,13 +168,241 @@ __global__ void k_unpack_dp(const double* __restrict__ raw, double* __restrict__
     if (t < n) dp[t] = 0.0 + raw[t] * scale;
 }
 
+// ---------------------------------------------------------------------------
+// The wall-normal solves of every mode, coefficients formed in the kernel:
+// row k of mode (i, j) is a_k, b = -(a_k + c_k) - (kx2_i + ky2_j), c_k, the
+// (0, 0) mode's wall row pinned (a = c = 0, b = 1, right-hand side 0): the values
+// of the arrays that ftd_solve_complex reads, by the same expressions.
+//
+// PaScaL over ceil(nz / 16) partitions of up to 16 rows, one lane per (mode,
+// partition): a', c' once for both parts of the right-hand side, which come in
+// and go out 16 bytes per lane. A mode costs 32 B per row where the solve on
+// arrays reads A, B, C as well (56), and half the divisions: 34816 modes of 256
+// rows (286 MB) in 58 us, 4.9 TB/s, where that solve took 125 and the pin's
+// launch 5 more.
+//
+// Bound by the loads in flight: all rows of a lane are requested at once, and
+// three waves per SIMD pay for 80 B of spills (67 us with two and none).
+// Workgroups of 256 lanes, three to a CU, so that one solves its 2Q-row system
+// while the others load: 86 us with 512, 64 with 128; partitions of 8 rows 85,
+// of 32 (one wave per SIMD) 80.
+// ---------------------------------------------------------------------------
+constexpr int kModeRows = 16;
+constexpr int kModeThreads = 256;
+typedef double mode_dbl2 __attribute__((ext_vector_type(2)));
+
+// the modes' shape: Q partitions, S modes per workgroup (0: nz is outside what
+// the kernel holds, up to 512 rows, and the solve on arrays takes them; below 17
+// rows one partition is left)
+void mode_shape(int nz, int& Q, int& S) {
+    Q = (nz + kModeRows - 1) / kModeRows;
+    S = 0;
+    if (Q < 2 || Q > 32 || nz / Q < 3) return;
+    S = 64;
+    while (S * Q > kModeThreads) S >>= 1;
+}
+
+size_t mode_lds(int nz, int Q, int S) {
+    return sizeof(double) * ((size_t)8 * Q * S + 3 * (size_t)nz);
+}
+
+__global__ __launch_bounds__(kModeThreads, 3) void k_mode_solve(double* __restrict__ hat, int nxh,
+                                                             int pitch, int ny, int nz, int Q,
+                                                             int lgS,
+                                                             const double* __restrict__ coef) {
+    constexpr int M = kModeRows;
+    extern __shared__ double lds[];
+    const int S = 1 << lgS;
+    const int t = threadIdx.x;
+    const int sl = t & (S - 1);
+    const int q = t >> lgS;
+    const int n = ny * pitch;
+    const int s_raw = ftd::xcd_tile(blockIdx.x, gridDim.x) * S + sl;
+    const int s = s_raw < n ? s_raw : n - 1;
+    const int jy = s / pitch, ix = s - jy * pitch;
+    const bool live = s_raw < n && ix < nxh;
+    int r0, cnt;
+    ftd::part_of(nz, Q, q, r0, cnt);
+    // a, c, -(a + c) of every row to LDS
+    double* const ta = lds + 8 * Q * S;
+    for (int k = t; k < 3 * nz; k += S * Q) ta[k] = coef[k];
+    const double* const tc = ta + nz;
+    const double* const tb = tc + nz;
+    // (modes in the padding have no wavenumber: the last one's)
+    const double lam = coef[3 * nz + (ix < nxh ? ix : nxh - 1)] + coef[3 * nz + nxh + jy];
+    const bool pin = s == 0 && q == 0;
+
+    mode_dbl2* const z = (mode_dbl2*)hat + (size_t)r0 * n + s;
+    mode_dbl2 d[M];
+#pragma unroll
+    for (int j = 0; j < M; ++j) d[j] = z[(size_t)(j < cnt ? j : cnt - 1) * n];
+    __syncthreads();
+    double a[M], c[M];
+    double aN = 0.0, cN = 0.0;
+    mode_dbl2 dN = {0.0, 0.0};
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+        if (j < cnt) {
+            double aj = ta[r0 + j], cj = tc[r0 + j], bj = tb[r0 + j] - lam;
+            if (j == 0) {
+                aj = pin ? 0.0 : aj;
+                cj = pin ? 0.0 : cj;
+                bj = pin ? 1.0 : bj;
+                d[0].x = pin ? 0.0 : d[0].x;
+                d[0].y = pin ? 0.0 : d[0].y;
+            }
+            if (j < 2) {
+                a[j] = aj / bj;
+                c[j] = cj / bj;
+                d[j].x = d[j].x / bj;
+                d[j].y = d[j].y / bj;
+            } else {
+                const double inv = 1.0 / (bj - aj * c[j - 1]);
+                d[j].x = inv * (d[j].x - aj * d[j - 1].x);
+                d[j].y = inv * (d[j].y - aj * d[j - 1].y);
+                c[j] = inv * cj;
+                a[j] = -inv * aj * a[j - 1];
+            }
+            if (j == cnt - 1) {
+                aN = a[j];
+                cN = c[j];
+                dN = d[j];
+            }
+        }
+    }
+#pragma unroll
+    for (int j = M - 3; j >= 1; --j) {
+        if (j <= cnt - 3) {
+            const double cj = c[j];
+            d[j].x = d[j].x - cj * d[j + 1].x;
+            d[j].y = d[j].y - cj * d[j + 1].y;
+            a[j] = a[j] - cj * a[j + 1];
+            c[j] = -cj * c[j + 1];
+        }
+    }
+    const double r = 1.0 / (1.0 - a[1] * c[0]);
+    const int NR = 2 * Q;
+    double* const rA = lds;
+    double* const rC = rA + NR * S;
+    double* const rX = rC + NR * S;
+    double* const rY = rX + NR * S;
+    const int o0 = 2 * q * S + sl, oN = o0 + S;
+    rA[o0] = r * a[0];
+    rC[o0] = -r * c[0] * c[1];
+    rX[o0] = r * (d[0].x - c[0] * d[1].x);
+    rY[o0] = r * (d[0].y - c[0] * d[1].y);
+    rA[oN] = aN;
+    rC[oN] = cN;
+    rX[oN] = dN.x;
+    rY[oN] = dN.y;
+    __syncthreads();
+    if (q == 0) {
+        // Thomas on the 2Q rows (b == 1) of both parts, 4 rows read at a time
+        double cp = rC[sl], xp = rX[sl], yp = rY[sl];
+        int k = 1;
+        for (; k + 4 <= NR; k += 4) {
+            double ak[4], ck[4], xk[4], yk[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int o = (k + u) * S + sl;
+                ak[u] = rA[o];
+                ck[u] = rC[o];
+                xk[u] = rX[o];
+                yk[u] = rY[o];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int o = (k + u) * S + sl;
+                const double inv = 1.0 / (1.0 - ak[u] * cp);
+                xp = inv * (xk[u] - ak[u] * xp);
+                yp = inv * (yk[u] - ak[u] * yp);
+                cp = inv * ck[u];
+                rX[o] = xp;
+                rY[o] = yp;
+                rC[o] = cp;
+            }
+        }
+        for (; k < NR; ++k) {
+            const int o = k * S + sl;
+            const double ak = rA[o];
+            const double inv = 1.0 / (1.0 - ak * cp);
+            xp = inv * (rX[o] - ak * xp);
+            yp = inv * (rY[o] - ak * yp);
+            cp = inv * rC[o];
+            rX[o] = xp;
+            rY[o] = yp;
+            rC[o] = cp;
+        }
+        for (k = NR - 2; k >= 0; --k) {
+            const int o = k * S + sl;
+            const double ck = rC[o];
+            xp = rX[o] - ck * xp;
+            yp = rY[o] - ck * yp;
+            rX[o] = xp;
+            rY[o] = yp;
+        }
+    }
+    __syncthreads();
+    const double x0 = rX[o0], y0 = rY[o0], xN = rX[oN], yN = rY[oN];
+    if (live) {
+#pragma unroll
+        for (int j = 0; j < M; ++j) {
+            if (j < cnt) {
+                mode_dbl2 x;
+                x.x = j == 0 ? x0 : j == cnt - 1 ? xN : d[j].x - (a[j] * x0 + c[j] * xN);
+                x.y = j == 0 ? y0 : j == cnt - 1 ? yN : d[j].y - (a[j] * y0 + c[j] * yN);
+                z[(size_t)j * n] = x;
+            }
+        }
+    }
+}
+
+// the FFT plans of layout k: lines of nxh modes (0) or of p->pitch (1)
+ftd_status fft_plans(ftd_poisson* p, int k) {
+    const int w = k ? p->pitch : p->nxh;
+    int n2[2] = {p->ny, p->nx}, real[2] = {p->ny, p->nx}, modes[2] = {p->ny, w};
+    const int dr = p->nx * p->ny, dm = w * p->ny;
+    if (hipfftPlanMany(&p->fwd[k], 2, n2, real, 1, dr, modes, 1, dm, HIPFFT_D2Z, p->nz) !=
+        HIPFFT_SUCCESS)
+        return perr(FTD_ERR_HIP, "hipfftPlanMany (D2Z) failed");
+    p->have_fwd[k] = 1;
+    if (hipfftPlanMany(&p->bwd[k], 2, n2, modes, 1, dm, real, 1, dr, HIPFFT_Z2D, p->nz) !=
+        HIPFFT_SUCCESS)
+        return perr(FTD_ERR_HIP, "hipfftPlanMany (Z2D) failed");
+    p->have_bwd[k] = 1;
+    if (hipfftSetStream(p->fwd[k], p->stream) != HIPFFT_SUCCESS ||
+        hipfftSetStream(p->bwd[k], p->stream) != HIPFFT_SUCCESS)
+        return perr(FTD_ERR_HIP, "hipfftSetStream failed");
+    return FTD_OK;
+}
+
 ftd_status poisson_spectral(ftd_poisson* p) {
-    PF(hipfftExecD2Z(p->fwd, p->rhs, reinterpret_cast<hipfftDoubleComplex*>(p->hat)));
+    // the solver as it was made solves in k_mode_solve; one that the caller
+    // tuned, moved to another stream or times solves by itself
+    if (p->pitch && ftd::handle_is_plain(p->solver, p->stream)) {
+        int Q, S;
+        mode_shape(p->nz, Q, S);
+        const int k = p->pitch != p->nxh;
+        PF(hipfftExecD2Z(p->fwd[k], p->rhs, reinterpret_cast<hipfftDoubleComplex*>(p->hat)));
+        int lgS = 0;
+        while ((1 << lgS) < S) ++lgS;
+        const int n = p->ny * p->pitch;
+        char path[96];
+        std::snprintf(path, sizeof path, "pascal_modes M=%d T=%d S=%d Q=%d", kModeRows,
+                      kModeThreads, S, Q);
+        ftd::handle_note_path(p->solver, path);
+        hipLaunchKernelGGL(k_mode_solve, dim3((n + S - 1) / S), dim3(S * Q), mode_lds(p->nz, Q, S),
+                           p->stream, p->hat, p->nxh, p->pitch, p->ny, p->nz, Q, lgS, p->coef);
+        PH(hipGetLastError());
+        PF(hipfftExecZ2D(p->bwd[k], reinterpret_cast<hipfftDoubleComplex*>(p->hat), p->rhs));
+        return FTD_OK;
+    }
+    PF(hipfftExecD2Z(p->fwd[0], p->rhs, reinterpret_cast<hipfftDoubleComplex*>(p->hat)));
     hipLaunchKernelGGL(k_pin_zero_mode, dim3(1), dim3(64), 0, p->stream, p->hat);
     PH(hipGetLastError());
-    ftd_status s = ftd_solve_complex(p->solver, p->A, p->B, p->C, p->hat);
+    const ftd_status s = ftd_solve_complex(p->solver, p->A, p->B, p->C, p->hat);
     if (s != FTD_OK) return perr(s, std::string("z solve: ") + ftd_last_error_string());
-    PF(hipfftExecZ2D(p->bwd, reinterpret_cast<hipfftDoubleComplex*>(p->hat), p->rhs));
+    PF(hipfftExecZ2D(p->bwd[0], reinterpret_cast<hipfftDoubleComplex*>(p->hat), p->rhs));
     return FTD_OK;
 }
 
@@ -232,12 +470,35 @@ ftd_status ftd_poisson_create(ftd_poisson** out, int nx, int ny, int nz, double 
     hA[0] = 0.0;
     hB[0] = 1.0;
     hC[0] = 0.0;
+    // one caller partition: every kind solves exactly, over partitions of the
+    // engine's choice. Lines of the spectra padded to whole 128-byte lines (the
+    // FFTs of 256^3 in 90 + 86 us where lines of 129 modes took 125 + 127),
+    // unless the padding would be more than a fifth of them
+    int mq, ms;
+    mode_shape(nz, mq, ms);
+    const int padded = (nxh + 7) / 8 * 8;
+    if (partitions == 1 && ms) p->pitch = 5 * padded <= 6 * nxh ? padded : nxh;
+    std::vector<double> coef(3 * (size_t)nz + nxh + ny);
+    for (int k = 0; k < nz; ++k) {
+        const double a = k == 0 ? 0.0 : 1.0 / (dz[k + 1] * dmz[k + 1]);
+        const double c = k == nz - 1 ? 0.0 : 1.0 / (dz[k + 1] * dmz[k + 2]);
+        coef[k] = a;
+        coef[nz + k] = c;
+        coef[2 * (size_t)nz + k] = -(a + c);
+    }
+    for (int i = 0; i < nxh; ++i) coef[3 * (size_t)nz + i] = kx2[i];
+    for (int j = 0; j < ny; ++j) coef[3 * (size_t)nz + nxh + j] = ky2[j];
+    const size_t hb = 2 * sizeof(double) * (size_t)nz * ny * std::max(nxh, p->pitch);
     const size_t cb = sizeof(double) * (size_t)nz * nm;
     if (e == hipSuccess) e = hipMalloc(&p->A, cb);
     if (e == hipSuccess) e = hipMalloc(&p->B, cb);
     if (e == hipSuccess) e = hipMalloc(&p->C, cb);
     if (e == hipSuccess) e = hipMalloc(&p->rhs, sizeof(double) * cells);
-    if (e == hipSuccess) e = hipMalloc(&p->hat, 2 * cb);
+    if (e == hipSuccess) e = hipMalloc(&p->hat, hb);
+    if (e == hipSuccess) e = hipMemset(p->hat, 0, hb);  // (the padding is read)
+    if (e == hipSuccess) e = hipMalloc(&p->coef, sizeof(double) * coef.size());
+    if (e == hipSuccess)
+        e = hipMemcpy(p->coef, coef.data(), sizeof(double) * coef.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMalloc(&p->met, sizeof(double) * met.size());
     if (e == hipSuccess) e = hipMemcpy(p->A, hA.data(), cb, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(p->B, hB.data(), cb, hipMemcpyHostToDevice);
@@ -248,19 +509,10 @@ ftd_status ftd_poisson_create(ftd_poisson** out, int nx, int ny, int nz, double 
     if (e == hipSuccess) e = hipEventCreate(&p->e1);
     if (e != hipSuccess)
         return bail(perr(FTD_ERR_HIP, std::string("ftd_poisson_create: ") + hipGetErrorString(e)));
-    int n2[2] = {ny, nx};
-    if (hipfftPlanMany(&p->fwd, 2, n2, nullptr, 1, nx * ny, nullptr, 1, nm, HIPFFT_D2Z, nz) !=
-        HIPFFT_SUCCESS)
-        return bail(perr(FTD_ERR_HIP, "hipfftPlanMany (D2Z) failed"));
-    p->have_fwd = 1;
-    if (hipfftPlanMany(&p->bwd, 2, n2, nullptr, 1, nm, nullptr, 1, nx * ny, HIPFFT_Z2D, nz) !=
-        HIPFFT_SUCCESS)
-        return bail(perr(FTD_ERR_HIP, "hipfftPlanMany (Z2D) failed"));
-    p->have_bwd = 1;
-    if (hipfftSetStream(p->fwd, p->stream) != HIPFFT_SUCCESS ||
-        hipfftSetStream(p->bwd, p->stream) != HIPFFT_SUCCESS)
-        return bail(perr(FTD_ERR_HIP, "hipfftSetStream failed"));
-    ftd_status s = ftd_create(&p->solver, kind, nm, nz, partitions, eps_constant, p->stream);
+    ftd_status s = fft_plans(p, 0);
+    if (s == FTD_OK && p->pitch > nxh) s = fft_plans(p, 1);
+    if (s != FTD_OK) return bail(s);
+    s = ftd_create(&p->solver, kind, nm, nz, partitions, eps_constant, p->stream);
     if (s != FTD_OK) return bail(perr(s, std::string("z solver: ") + ftd_last_error_string()));
     *out = p;
     return FTD_OK;
@@ -268,10 +520,12 @@ ftd_status ftd_poisson_create(ftd_poisson** out, int nx, int ny, int nz, double 
 
 ftd_status ftd_poisson_destroy(ftd_poisson* p) {
     if (!p) return FTD_OK;
-    if (p->have_fwd) hipfftDestroy(p->fwd);
-    if (p->have_bwd) hipfftDestroy(p->bwd);
+    for (int k = 0; k < 2; ++k) {
+        if (p->have_fwd[k]) hipfftDestroy(p->fwd[k]);
+        if (p->have_bwd[k]) hipfftDestroy(p->bwd[k]);
+    }
     if (p->solver) ftd_destroy(p->solver);
-    for (double* b : {p->A, p->B, p->C, p->rhs, p->hat, p->met})
+    for (double* b : {p->A, p->B, p->C, p->rhs, p->hat, p->met, p->coef})
         if (b) hipFree(b);
     if (p->e0) hipEventDestroy(p->e0);
     if (p->e1) hipEventDestroy(p->e1);

@@ -389,7 +389,7 @@ const char* ftd_heat_last_plan(const ftd_heat* h);
 typedef struct ftd_poisson ftd_poisson;
 
 /* Metrics, modified wavenumbers and the wall-normal coefficients
- * (PressureSolver.cpp:36-104, 400-456) are built once; two hipFFT plans.
+ * (PressureSolver.cpp:36-104, 400-456) are built once; hipFFT plans.
  * nx even. `stream` is a hipStream_t (NULL = the null stream), as for
  * ftd_create. */
 ftd_status ftd_poisson_create(ftd_poisson** out, int nx, int ny, int nz, double Lx, double Ly,
@@ -398,7 +398,10 @@ ftd_status ftd_poisson_create(ftd_poisson** out, int nx, int ny, int nz, double 
 ftd_status ftd_poisson_destroy(ftd_poisson* p);
 
 /* The solver of the wall-normal systems (n_sys = (nx/2+1) ny complex, n_row
- * = nz), e.g. for ftd_set_j_mode or ftd_set_tuning. Owned by p. */
+ * = nz), e.g. for ftd_set_j_mode or ftd_set_tuning. Owned by p. With one
+ * partition and 17 to 512 rows the step solves the modes itself (ftd_last_path:
+ * "pascal_modes") as long as this handle is tuned, profiled and streamed as it
+ * was made. */
 ftd_handle* ftd_poisson_solver(ftd_poisson* p);
 
 /* One pressure step (solve, :493-533): rhs = div(u*)/dt, FFT, wall-normal
