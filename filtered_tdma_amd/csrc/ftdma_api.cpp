@@ -84,7 +84,7 @@ struct ftd_handle {
     int guard = 0;                           // filtered kinds: exact solve where terms exceed eps_/4
     DevBuf jsys;                             // learned mode: J (| fallback << 16) per lane
     size_t jsys_count = 0;
-    double* rho = nullptr;                   // A_rho[n_row+1] then C_rho[n_row+1]
+    double* rho = nullptr;                   // A_rho[n_row+1] then C_rho[n_row+1] (k_set_rho)
     int* J = nullptr;                        // J per partition
     DevBuf partial, xbuf, R, E;
     // uneven batches: the plan of the last layout (host copy of the layout
@@ -424,7 +424,7 @@ ftd_status solve_filtered(ftd_handle* h, double* A, double* B, double* C, double
                           P, R, gs);
             FTD_LAUNCH(ftd::launch_filtered_stream(Ms, P, 1, 3, A, B, C, D, n_sys, n_row, cyclic, Jp,
                                                    nullptr, nullptr, h->eps_value, h->eps_direct,
-                                                   Js, g, st));
+                                                   Js, g, nullptr, st));
             return FTD_OK;
         }
         if (version == 2) {
@@ -436,7 +436,8 @@ ftd_status solve_filtered(ftd_handle* h, double* A, double* B, double* C, double
             std::snprintf(h->path, sizeof h->path, "filtered_v2_stream M=%d Q=%d R=%d%s", Ms, P, R,
                           gs);
             FTD_LAUNCH(ftd::launch_filtered_stream(Ms, P, 2, 0, A, B, C, D, n_sys, n_row, cyclic, Jp,
-                                                   nullptr, nullptr, ev, ed, Js, g, st));
+                                                   nullptr, nullptr, ev, ed, Js, g, nullptr,
+                                                   st));
         } else {
             const int tiles = n_sys / 32;
             FTD_TRY(ensure(h, h->partial, sizeof(double) * (size_t)tiles * (P << csh)));
@@ -444,12 +445,14 @@ ftd_status solve_filtered(ftd_handle* h, double* A, double* B, double* C, double
             std::snprintf(h->path, sizeof h->path, "filtered_v1_stream M=%d Q=%d R=%d%s", Ms, P, R,
                           gs);
             FTD_LAUNCH(ftd::launch_filtered_stream(Ms, P, 1, 1, A, B, C, D, n_sys, n_row, cyclic, Jp,
-                                                   (double*)h->xbuf.p, (double*)h->partial.p, 0.0,
-                                                   0, nullptr, 0, st));
+                                                   (double*)h->xbuf.p, (double*)h->partial.p,
+                                                   h->eps_value, h->eps_direct, nullptr, 0,
+                                                   g ? nullptr : h->rho, st));
             FTD_LAUNCH(ftd::launch_compute_J((double*)h->partial.p, tiles, P, n_row, h->rho,
                                              h->eps_value, h->eps_direct, csh, Jp, st));
             FTD_LAUNCH(ftd::launch_filtered_stream(Ms, P, 1, 2, A, B, C, D, n_sys, n_row, cyclic, Jp,
-                                                   (double*)h->xbuf.p, nullptr, ev, ed, Js, g, st));
+                                                   (double*)h->xbuf.p, (double*)h->partial.p, ev,
+                                                   ed, Js, g, nullptr, st));
         }
         return FTD_OK;
     }
@@ -465,7 +468,7 @@ ftd_status solve_filtered(ftd_handle* h, double* A, double* B, double* C, double
                       fs.T, fs.S, gs);
         FTD_LAUNCH(ftd::launch_filtered_fused(fs.M, fs.T, 1, 3, A, B, C, D, n_sys, n_row, P, fs.S,
                                               cyclic, csh, Jp, nullptr, nullptr, h->eps_value,
-                                              h->eps_direct, (int*)h->jsys.p, g, st));
+                                              h->eps_direct, (int*)h->jsys.p, g, nullptr, st));
         return FTD_OK;
     }
     if (fs.M) {
@@ -481,7 +484,7 @@ ftd_status solve_filtered(ftd_handle* h, double* A, double* B, double* C, double
                           fs.S, gs);
             FTD_LAUNCH(ftd::launch_filtered_fused(fs.M, fs.T, 2, 0, A, B, C, D, n_sys, n_row, P, fs.S,
                                                   cyclic, csh, Jp, nullptr, nullptr, ev, ed, Js, g,
-                                                  st));
+                                                  nullptr, st));
         } else {
             FTD_TRY(ensure(h, h->partial, sizeof(double) * (size_t)tiles * (P << csh)));
             FTD_TRY(ensure(h, h->xbuf, xbytes));
@@ -489,12 +492,15 @@ ftd_status solve_filtered(ftd_handle* h, double* A, double* B, double* C, double
                           fs.S, gs);
             FTD_LAUNCH(ftd::launch_filtered_fused(fs.M, fs.T, 1, 1, A, B, C, D, n_sys, n_row, P, fs.S,
                                                   cyclic, csh, Jp, (double*)h->xbuf.p,
-                                                  (double*)h->partial.p, 0.0, 0, nullptr, 0, st));
+                                                  (double*)h->partial.p, h->eps_value,
+                                                  h->eps_direct, nullptr, 0, g ? nullptr : h->rho,
+                                                  st));
             FTD_LAUNCH(ftd::launch_compute_J((double*)h->partial.p, tiles, P, n_row, h->rho,
                                              h->eps_value, h->eps_direct, csh, Jp, st));
             FTD_LAUNCH(ftd::launch_filtered_fused(fs.M, fs.T, 1, 2, A, B, C, D, n_sys, n_row, P, fs.S,
-                                                  cyclic, csh, Jp, (double*)h->xbuf.p, nullptr, ev,
-                                                  ed, Js, g, st));
+                                                  cyclic, csh, Jp, (double*)h->xbuf.p,
+                                                  (double*)h->partial.p, ev, ed, Js, g, nullptr,
+                                                  st));
         }
         return FTD_OK;
     }
@@ -698,7 +704,7 @@ ftd_status ftd_set_rho(ftd_handle* h, const double* A, const double* B, const do
     if (h->kind == FTD_KIND_PASCAL) return FTD_OK;
     if (!A || !B || !C) return fail(FTD_ERR_INVALID, "null array pointer");
     if (h->n_sys == 0) return FTD_OK;
-    FTD_HIP(ftd::launch_set_rho(A, B, C, h->n_sys, h->n_row, h->rho, h->stream));
+    FTD_HIP(ftd::launch_set_rho(A, B, C, h->n_sys, h->n_row, h->P, h->rho, h->stream));
     return FTD_OK;
 }
 
@@ -1326,7 +1332,7 @@ ftd_status ftd_solve_static(int kind, int n_sys, int n_row, int partitions, doub
     // boundary values), so nothing needs clearing
     ftd_status st = FTD_OK;
     if (filtered) {
-        const hipError_t e = ftd::launch_set_rho(A, B, C, n_sys, n_row, h.rho, h.stream);
+        const hipError_t e = ftd::launch_set_rho(A, B, C, n_sys, n_row, partitions, h.rho, h.stream);
         if (e != hipSuccess) st = hip_fail(e, "set_rho");
     }
     if (st == FTD_OK)

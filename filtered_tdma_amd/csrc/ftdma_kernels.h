@@ -11,7 +11,7 @@
 namespace ftd {
 
 hipError_t launch_set_rho(const double* A, const double* B, const double* C, int n_sys, int n_row,
-                          double* rho, hipStream_t st);
+                          int P, double* rho, hipStream_t st);
 // csh = 1: complex right-hand sides stored as interleaved (re, im) columns
 // of n_sys = 2 x (complex systems) real columns; the coefficients have
 // n_sys / 2 columns, and J is kept per parity (J[p], J[P + p])
@@ -61,12 +61,14 @@ hipError_t launch_pascal_stream(int M, int Q, const double* A, const double* B, 
 // J records to Jsys [Q x n_sys]. guard = 1 (non-periodic; version 2 pass 0,
 // or version 1 pass 2 or 3): v1 sweeps, and the systems whose dropped terms
 // exceed eps_/4 solved exactly; records (J | fallback << 16 | guard << 17)
-// to Jsys
+// to Jsys. Version 1 without the guard: pass 1 given rho (the handle's column-0
+// bounds, k_set_rho) stores x of the tiles whose J it can tell and marks them in
+// partial for pass 2, which needs the same partial
 hipError_t launch_filtered_stream(int M, int Q, int version, int pass, const double* A,
                                   const double* B, const double* C, double* D, int n_sys,
                                   int n_row, int cyclic, const int* Jp, double* xbuf,
                                   double* partial, double eps_value, int eps_direct, int* Jsys,
-                                  int guard, hipStream_t st);
+                                  int guard, const double* rho, hipStream_t st);
 
 // Workgroups of `kernel` resident on the whole device at once, at most
 // n_tiles: the grid of the persistent kernels
@@ -127,12 +129,12 @@ hipError_t launch_thomas_cyclic_fused(const double* A, const double* B, const do
 
 int filtered_fused_supported(int M, int maxt);
 size_t filtered_fused_lds(int P, int S, int guard);
-// guard: as launch_filtered_stream
+// guard, rho: as launch_filtered_stream
 hipError_t launch_filtered_fused(int M, int maxt, int version, int pass, const double* A,
                                  const double* B, const double* C, double* D, int n_sys, int n_row,
                                  int P, int S, int cyclic, int csh, const int* Jp, double* xbuf,
                                  double* partial, double eps_value, int eps_direct, int* Jsys,
-                                 int guard, hipStream_t st);
+                                 int guard, const double* rho, hipStream_t st);
 
 hipError_t launch_gen_thomas(const double* A, const double* B, double* C, double* D, int n_sys,
                              int n_row, hipStream_t st);
@@ -165,7 +167,8 @@ hipError_t launch_gen_filtered_final(const double* A, const double* C, double* D
 // For a caller inside the library that runs a filtered kind's sweeps itself
 // (the heat step's fused filtered z sweep): the handle's J per partition
 // (device), its column-0 bounds as set by ftd_set_rho (device, A_rho then
-// C_rho, n_row + 1 each) and its eps_ setting. An error for a handle that is
+// C_rho, n_row + 1 each; A_rho of a partition's first row holds the partition's
+// full_J_scale) and its eps_ setting. An error for a handle that is
 // not a filtered kind over more than one partition, or that has learned J or
 // the guard switched on (those run on the handle's own solve).
 struct ftd_handle;

@@ -74,21 +74,67 @@ __device__ inline double group_max(double v, int width) {
     return v;
 }
 
+// From which boundary maximum v of any one tile on cal_J_gpu gives m - 1, the
+// full correction, for v and every larger one: eps / (B1 v) <= q^(m-2).
+// full_J_scale is B1 q^(m-2), which the column-0 bound alone settles (0: full
+// for every v, NaN: no v that can be told), full_J compares v with eps over
+// it, with 1e-9 to spare for the rounding of the logarithms.
+__device__ inline double full_J_scale(double rho, int m) {
+    if (rho == 0.0 || rho >= 0.5) return 0.0;
+    const double lambda_p = (1.0 + sqrt(1.0 - 4.0 * rho * rho)) * 0.5;
+    const double q = rho / lambda_p;
+    const double B1 = q * (2.0 + q) / ((1.0 - q) * (1.0 - 2.0 * rho));
+    const double T = B1 * exp((double)(m - 2) * log(q));
+    return T > 0.0 && T < __builtin_inf() ? T : __builtin_nan("");
+}
+
+// the v itself: -1 for every v, NaN for none
+__device__ inline double full_J_from(double scale, int m, int P, double eps_value,
+                                     int eps_direct) {
+    if (scale == 0.0) return -1.0;
+    const double Nl = (double)(m * P);
+    const double eps = eps_direct ? eps_value : eps_value / (Nl * Nl);
+    const double v = eps / scale * (1.0 + 1e-9);
+    return eps >= 0.0 && v < __builtin_inf() ? v : __builtin_nan("");
+}
+
+__device__ inline bool full_J(double from, double v) {
+    return from < 0.0 || (v > 0.0 && v >= from);
+}
+
 // ---------------------------------------------------------------------------
 // column-0 spectral bounds (filtered_tdma_kernels.cuh:46-67)
 // ---------------------------------------------------------------------------
-__global__ void k_set_rho(const double* __restrict__ A, const double* __restrict__ B,
-                          const double* __restrict__ C, int n_sys, int n_row,
-                          double* __restrict__ A_rho, double* __restrict__ C_rho) {
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k > n_row) return;
-    if (k < n_row) {
-        double bk = B[(size_t)k * n_sys];
-        A_rho[k] = (bk != 0.0) ? fabs(A[(size_t)k * n_sys] / bk) : 0.0;
-        C_rho[k] = (bk != 0.0) ? fabs(C[(size_t)k * n_sys] / bk) : 0.0;
-    } else {
-        A_rho[k] = 0.0;
-        C_rho[k] = 0.0;
+// one block per partition; a partition's J takes rows 1..m-1, so A_rho of its
+// row 0 holds its full_J_scale instead
+__global__ __launch_bounds__(256) void k_set_rho(const double* __restrict__ A,
+                                                 const double* __restrict__ B,
+                                                 const double* __restrict__ C, int n_sys,
+                                                 int n_row, double* __restrict__ A_rho,
+                                                 double* __restrict__ C_rho) {
+    __shared__ double red[4];
+    const int P = gridDim.x;
+    int s, m;
+    part_of(n_row, P, blockIdx.x, s, m);
+    double r = 0.0;
+    for (int k = threadIdx.x; k < m; k += 256) {
+        const size_t o = (size_t)(s + k) * n_sys;
+        const double bk = B[o];
+        const double a = (bk != 0.0) ? fabs(A[o] / bk) : 0.0;
+        const double c = (bk != 0.0) ? fabs(C[o] / bk) : 0.0;
+        if (k > 0) {
+            A_rho[s + k] = a;
+            r = fmax(r, fmax(a, c));
+        }
+        C_rho[s + k] = c;
+    }
+    r = group_max(r, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = r;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        r = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+        if (m > 0) A_rho[s] = full_J_scale(r, m);
+        if (blockIdx.x == 0) A_rho[n_row] = C_rho[n_row] = 0.0;
     }
 }
 
@@ -145,7 +191,7 @@ __global__ __launch_bounds__(256) void k_compute_J(const double* __restrict__ pa
     int s, m;
     part_of(n_row, P, p, s, m);
     double vb = 0.0, vr = 0.0;
-    for (int t = threadIdx.x; t < n_tiles; t += 256) vb = fmax(vb, part[(size_t)t * P + p]);
+    for (int t = threadIdx.x; t < n_tiles; t += 256) vb = fmax(vb, fabs(part[(size_t)t * P + p]));  // (sign: tile stored)
     for (int k = 1 + threadIdx.x; k < m; k += 256)
         vr = fmax(vr, fmax(fabs(A_rho[s + k]), fabs(C_rho[s + k])));
     vb = group_max(vb, 64);
@@ -1101,6 +1147,10 @@ __global__ __launch_bounds__(Q * 32) __attribute__((amdgpu_waves_per_eu(WPE))) v
 //   PASS 0: v2 (J_p known) -> x stored.
 //   PASS 1: v1 first pass  -> x0, xN of every (partition, system) to xbuf,
 //           per-tile max of |x0|,|xN| to partial (J needs all systems).
+//              With rho (no guard), a tile whose own maxima already give
+//              J = m - 1 in every partition has nothing to wait for: J grows
+//              with the maximum over all tiles. It stores x here and leaves
+//              its maxima negative; the second pass passes it by.
 //   PASS 2: v1 second pass -> recompute the sweeps, take x0, xN from xbuf and
 //           J_p, store x.
 // ---------------------------------------------------------------------------
@@ -1308,13 +1358,19 @@ __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE))) voi
                                                          double* __restrict__ xbuf,
                                                          double* __restrict__ partial,
                                                          double eps_value, int eps_direct,
-                                                         int* __restrict__ Jsys) {
+                                                         int* __restrict__ Jsys,
+                                                         const double* __restrict__ rho) {
+    // adjacent tiles on one XCD, for the 128-byte lines that they share (v2,
+    // 65537 x 512, P = 8: 433 to 408 us; 30001 x 200, P = 4, v1: 115 to 104)
+    const int blk = xcd_tile(blockIdx.x, gridDim.x);
+    // PASS 2: nothing left where the first pass stored x
+    if (PASS == 2 && !GRD && __builtin_signbit(partial[(size_t)blk * P])) return;
     extern __shared__ double lds[];
     const int S = 1 << lgS;
     const int t = threadIdx.x;
     const int sl = t & (S - 1);
     const int p = t >> lgS;
-    const int i_raw = blockIdx.x * S + sl;
+    const int i_raw = blk * S + sl;
     const bool live = i_raw < n_sys;
     // dead lanes shadow the last system (of their parity when CSH = 1)
     const int i = live ? i_raw : n_sys - (1 << CSH) + (i_raw & ((1 << CSH) - 1));
@@ -1457,22 +1513,31 @@ __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE))) voi
         detR = has_right ? dr : 1.0;
     }
 
+    int Jf = J;
     if (PASS == 1) {
-        if (live) {
-            xbuf[(size_t)(2 * p) * ld + i] = x0;
-            xbuf[(size_t)(2 * p + 1) * ld + i] = xN;
-        }
         // dead lanes shadow a live system, so they do not change the max;
         // with CSH = 1 the two parities reduce separately (xor offsets >= 2)
         double v = fmax(fabs(x0), fabs(xN));
         const int width = S < 64 ? S : 64;
         for (int off = width >> 1; off >= (1 << CSH); off >>= 1)
             v = fmax(v, __shfl_xor(v, off, 64));
-        if (sl < (1 << CSH)) partial[((size_t)sl * gridDim.x + blockIdx.x) * P + p] = v;
-        return;
+        // rho given: a tile whose own maxima already ask for the full
+        // correction in every partition takes it here, and says so by the sign
+        const double from =
+            rho ? full_J_from(rho[r0], m, P, eps_value, eps_direct) : __builtin_nan("");
+        const bool now = __syncthreads_and(full_J(from, v)) != 0;
+        if (sl < (1 << CSH))
+            partial[((size_t)sl * gridDim.x + blk) * P + p] = now ? -fabs(v) : fabs(v);
+        if (!now) {
+            if (live) {
+                xbuf[(size_t)(2 * p) * ld + i] = x0;
+                xbuf[(size_t)(2 * p + 1) * ld + i] = xN;
+            }
+            return;
+        }
+        Jf = m - 1;
     }
 
-    int Jf = J;
     if (PASS == 3) {
         // learned J of this (system, partition), then the first dropped
         // term of each side against eps_; a larger one falls back to the
@@ -1550,7 +1615,12 @@ __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE))) voi
 // k_filtered_fused over the StreamRing of k_pascal_stream. Same shape
 // requirements (S = 32, two partitions per wave, n_sys % 32 == 0).
 //   PASS 0: v2 -> x stored (M stores per tile).
-//   PASS 1: v1 first pass -> x0, xN to xbuf, per-tile max to partial
+//   PASS 1: v1 first pass -> x0, xN to xbuf, per-tile max to partial, or x at
+//           once where the wave's two maxima already give J = m - 1 (as
+//           k_filtered_fused): 65536 x 512, P = 8, J = 63: 506 to 324 us, one
+//           read of the rows (1.34 GB with the stores) instead of two. With J
+//           = 29 nothing is stored early: 502 to 497, from the second pass's
+//           order
 //           (3 stores per tile).
 //   PASS 2: v1 second pass -> x0, xN from xbuf (one more DMA per tile into
 //           an LDS block, issued ahead of the sweep), x stored (M stores per
@@ -1561,7 +1631,7 @@ __global__ __launch_bounds__(Q * 32) __attribute__((amdgpu_waves_per_eu(WPE))) v
     const double* __restrict__ A, const double* __restrict__ B, const double* __restrict__ C,
     double* D, int n_sys, int n_row, int n_tiles, int cyclic, const int* __restrict__ Jp,
     double* __restrict__ xbuf, double* __restrict__ partial, double eps_value, int eps_direct,
-    int* __restrict__ Jsys) {
+    int* __restrict__ Jsys, const double* __restrict__ rho) {
     constexpr int S = 32, NW = Q / 2;
     static_assert(Q % 2 == 0 && M % R == 0 && R >= 2, "stream shape");
     static_assert(!GRD || VERSION == 1, "the guard runs the v1 sweeps");
@@ -1585,7 +1655,23 @@ __global__ __launch_bounds__(Q * 32) __attribute__((amdgpu_waves_per_eu(WPE))) v
     int r0, m0;
     part_of(n_row, Q, p, r0, m0);
     int J0 = (VERSION == 2 || PASS == 2 || (GRD && PASS == 0)) ? Jp[p] : m0;
-    asm volatile("" : "+v"(J0));  // J is loaded before the ring starts
+    constexpr bool LEFT = PASS == 2 && !GRD;
+    const int stride = (int)gridDim.x;
+    // PASS 2 takes the tiles from the last one down: those rows are the ones
+    // that the first pass has left in the 256 MB last-level cache
+    auto tile_at = [&](int T) { return PASS == 2 ? n_tiles - 1 - T : T; };
+    // PASS 2: a turn's tile was stored by the first pass if the maximum that it
+    // left in partial is negative; the turns b, b + stride, ... of one lane each
+    auto max_of = [&](int b) {
+        const int T = b + l * stride;
+        return partial[(size_t)tile_at(T < n_tiles ? T : 0) * Q + 2 * w];
+    };
+    double max0 = LEFT ? max_of(blockIdx.x) : 0.0;
+    // PASS 1 with rho: from which tile maximum on this lane's partition takes
+    // the full correction at once
+    double from = PASS == 1 && rho ? rho[r0] : __builtin_nan("");
+    // loaded before the ring starts
+    asm volatile("" : "+v"(J0), "+v"(max0), "+v"(from));
     // PASS 2: rows 4w..4w+3 of xbuf (x0, xN of partitions 2w, 2w+1), two
     // systems per lane, as the ring's sub-blocks
     const double* xsrc = xbuf + (size_t)(4 * w + (l >> 4)) * ld + 2 * (l & 15);
@@ -1593,14 +1679,37 @@ __global__ __launch_bounds__(Q * 32) __attribute__((amdgpu_waves_per_eu(WPE))) v
     int dcnt0;
     rg.init(ring[w], A, B, C, D, n_sys, n_row, w, l, dcnt0);
 
-    int tile = blockIdx.x;
-    rg.prologue(tile, dcnt0);
+    int tbase = blockIdx.x;
+    auto left_of = [&](int b, double v) {
+        return __ballot(b + l * stride < n_tiles && !__builtin_signbit(v));
+    };
+    unsigned long long left = 0;
+    auto after = [&](int T) {  // the turn that follows T here, n_tiles or more if none
+        if (!LEFT) return T + stride;
+        while (!left) {
+            tbase += 64 * stride;
+            if (tbase >= n_tiles) return n_tiles;
+            left = left_of(tbase, max_of(tbase));
+        }
+        const int b = __builtin_ctzll(left);
+        left &= left - 1;
+        return tbase + b * stride;
+    };
+    int turn = blockIdx.x;
+    if (LEFT) {
+        left = left_of(tbase, max0);
+        turn = after(turn);
+        if (turn >= n_tiles) return;
+    }
+    rg.prologue(tile_at(turn), dcnt0);
+    if (PASS == 1) from = full_J_from(from, m0, Q, eps_value, eps_direct);
     bool first = true;
-    for (; tile < n_tiles; tile += gridDim.x) {
+    for (int next; turn < n_tiles; turn = next) {
+        const int tile = tile_at(turn);
         int m = m0, dcnt = dcnt0, J = J0;
         asm volatile("" : "+v"(m), "+v"(dcnt), "+v"(J));
-        const int next = tile + (int)gridDim.x;
-        const int ntile = next < n_tiles ? next : tile;
+        next = after(turn);
+        const int ntile = next < n_tiles ? tile_at(next) : tile;
         const int i = tile * S + sl;
         const size_t base = (size_t)r0 * ld + (size_t)i;
         double x0 = 0.0, xN = 0.0;
@@ -1719,13 +1828,21 @@ __global__ __launch_bounds__(Q * 32) __attribute__((amdgpu_waves_per_eu(WPE))) v
         }
         // the next tile's first R rows have landed before this tile's stores
         wait_vmcnt<0>();
+        int Jf = J;
+        bool store = PASS != 1;
         if (PASS == 1) {
-            xbuf[(size_t)(2 * p) * ld + i] = x0;
-            xbuf[(size_t)(2 * p + 1) * ld + i] = xN;
             const double v = group_max(fmax(fabs(x0), fabs(xN)), S);
-            if (sl == 0) partial[(size_t)tile * Q + p] = v;
-        } else {
-            int Jf = J;
+            // both partitions of the wave in full already: x now, and the sign
+            // of the maxima says so
+            store = __ballot(!full_J(from, v)) == 0;
+            if (sl == 0) partial[(size_t)tile * Q + p] = store ? -fabs(v) : fabs(v);
+            Jf = m - 1;
+            if (!store) {
+                xbuf[(size_t)(2 * p) * ld + i] = x0;
+                xbuf[(size_t)(2 * p + 1) * ld + i] = xN;
+            }
+        }
+        if (store) {
             if (PASS == 3) {
                 // learned J of this (system, partition), checked against eps_
                 // by the first dropped term of each side (as k_filtered_fused)
@@ -2467,10 +2584,9 @@ static inline int log2i(int v) {
 }
 
 hipError_t launch_set_rho(const double* A, const double* B, const double* C, int n_sys, int n_row,
-                          double* rho, hipStream_t st) {
-    const int n = n_row + 1;
-    hipLaunchKernelGGL(k_set_rho, dim3((n + 255) / 256), dim3(256), 0, st, A, B, C, n_sys, n_row,
-                       rho, rho + n);
+                          int P, double* rho, hipStream_t st) {
+    hipLaunchKernelGGL(k_set_rho, dim3(P), dim3(256), 0, st, A, B, C, n_sys, n_row, rho,
+                       rho + n_row + 1);
     return hipGetLastError();
 }
 
@@ -2660,7 +2776,8 @@ hipError_t launch_filtered_fused(int M, int maxt, int version, int pass, const d
                                  const double* B, const double* C, double* D, int n_sys, int n_row,
                                  int P, int S, int cyclic, int csh, const int* Jp, double* xbuf,
                                  double* partial, double eps_value, int eps_direct, int* Jsys,
-                                 int guard, hipStream_t st) {
+                                 int guard, const double* rho, hipStream_t st) {
+    if (pass == 2 && !guard && !partial) return hipErrorInvalidValue;
     const int lgS = log2i(S);
     const dim3 grid((n_sys + S - 1) / S), block(S * P);
     // the guard runs after the first pass of v1 only
@@ -2672,11 +2789,11 @@ hipError_t launch_filtered_fused(int M, int maxt, int version, int pass, const d
         if (csh)                                                                             \
             hipLaunchKernelGGL((k_filtered_fused<m_, t_, v_, p_, pf_, w_, 1, g_>), grid, block, \
                                lds, st, A, B, C, D, n_sys, n_row, P, lgS, cyclic, Jp, xbuf,   \
-                               partial, eps_value, eps_direct, Jsys);                        \
+                               partial, eps_value, eps_direct, Jsys, rho);                   \
         else                                                                                 \
             hipLaunchKernelGGL((k_filtered_fused<m_, t_, v_, p_, pf_, w_, 0, g_>), grid, block, \
                                lds, st, A, B, C, D, n_sys, n_row, P, lgS, cyclic, Jp, xbuf,   \
-                               partial, eps_value, eps_direct, Jsys);                        \
+                               partial, eps_value, eps_direct, Jsys, rho);                   \
     } while (0)
 #define X(m_, t_, pf_, w_)                                \
     if (M == m_ && maxt == t_) {                          \
@@ -2839,7 +2956,8 @@ hipError_t launch_filtered_stream(int M, int Q, int version, int pass, const dou
                                   const double* B, const double* C, double* D, int n_sys,
                                   int n_row, int cyclic, const int* Jp, double* xbuf,
                                   double* partial, double eps_value, int eps_direct, int* Jsys,
-                                  int guard, hipStream_t st) {
+                                  int guard, const double* rho, hipStream_t st) {
+    if (pass == 2 && !guard && !partial) return hipErrorInvalidValue;
     if (!stream_eligible(n_sys, A, B, C, D)) return hipErrorInvalidValue;
     if ((pass == 3 || guard) && !Jsys) return hipErrorInvalidValue;
     if (guard && pass == 1) return hipErrorInvalidValue;
@@ -2850,7 +2968,7 @@ hipError_t launch_filtered_stream(int M, int Q, int version, int pass, const dou
         const dim3 grid(resident_grid(k, q_ * 32, n_tiles)), block(q_ * 32);                 \
         hipLaunchKernelGGL((k_filtered_stream<m_, q_, r_, v_, p_, w_, g_>), grid, block, 0, st, \
                            A, B, C, D, n_sys, n_row, n_tiles, cyclic, Jp, xbuf, partial,     \
-                           eps_value, eps_direct, Jsys);                                     \
+                           eps_value, eps_direct, Jsys, rho);                                \
     } while (0)
     // the guard's variants: one wave per SIMD (its LDS flags and exact reduced
     // solve make them larger), none for 16 partitions (their ring fills the
