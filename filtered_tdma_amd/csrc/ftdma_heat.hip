@@ -26,6 +26,8 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "../../include/ftdma.h"
@@ -1037,6 +1039,8 @@ struct ftd_heat {
     } filt[3];
     int use_fused = 1;
     int fuse_rhs = 0;  // the fused z sweep forms the rhs (no k_rhs_z pass) this step
+    char* pinned = nullptr;  // ftd_heat_field's staging (kCopyThreads x 2 slots), on first use
+    hipEvent_t slot[16] = {};  // and its slots' events
     char plan[256] = "";  // how the last enqueued step ran each sweep (ftd_heat_last_plan)
 };
 
@@ -1457,6 +1461,95 @@ ftd_status enqueue_step(ftd_heat* h) {
     return FTD_OK;
 }
 
+// Large fields go to pageable host memory through a pinned ring that the handle
+// keeps (12 MiB): each of a few threads has two slots, asks for the next of its
+// pieces while it copies the last one out. One thread's copy, and the page
+// faults of a new destination most of all, took longer than the link: 100
+// steps and the field of 256^3 cells (137 MB) 36.0 -> 27.1 ms. From 16 MiB on; a
+// smaller field is a few pieces, less than the threads cost.
+constexpr int kCopyThreads = 6;
+constexpr size_t kCopyPiece = (size_t)1 << 20;
+constexpr size_t kCopyFrom = (size_t)16 << 20;
+static_assert(2 * kCopyThreads <= 16, "ftd_heat::slot");
+
+// the ring and its events; false: not to be had, the plain copy does
+bool copy_ring(ftd_heat* h) {
+    if (h->pinned) return true;
+    for (int k = 0; k < 2 * kCopyThreads; ++k)
+        if (!h->slot[k] &&
+            hipEventCreateWithFlags(&h->slot[k], hipEventDisableTiming) != hipSuccess) {
+            h->slot[k] = nullptr;
+            (void)hipGetLastError();
+            return false;
+        }
+    if (hipHostMalloc((void**)&h->pinned, 2 * kCopyThreads * kCopyPiece, hipHostMallocDefault) !=
+        hipSuccess) {
+        h->pinned = nullptr;
+        (void)hipGetLastError();
+        return false;
+    }
+    return true;
+}
+
+// pieces t, t + kCopyThreads, ... of src to dst; 0: all copied
+hipError_t copy_pieces(ftd_heat* h, int dev, int t, const char* src, char* dst, size_t bytes) {
+    hipError_t e = hipSetDevice(dev);
+    const size_t n = (bytes + kCopyPiece - 1) / kCopyPiece;
+    char* const ring = h->pinned + (size_t)2 * t * kCopyPiece;
+    auto len = [&](size_t k) { return std::min(kCopyPiece, bytes - k * kCopyPiece); };
+    auto ask = [&](size_t k, int u) {
+        if (e != hipSuccess || k >= n) return;
+        e = hipMemcpyAsync(ring + u * kCopyPiece, src + k * kCopyPiece, len(k),
+                           hipMemcpyDeviceToHost, h->stream);
+        if (e == hipSuccess) e = hipEventRecord(h->slot[2 * t + u], h->stream);
+    };
+    ask(t, 0);
+    int u = 0;
+    for (size_t k = t; k < n && e == hipSuccess; k += kCopyThreads, u ^= 1) {
+        ask(k + kCopyThreads, u ^ 1);
+        if (e != hipSuccess) break;
+        if ((e = hipEventSynchronize(h->slot[2 * t + u])) != hipSuccess) break;
+        std::memcpy(dst + k * kCopyPiece, ring + u * kCopyPiece, len(k));
+    }
+    return e;
+}
+
+// src (device) to dst (host), after the work queued on the handle's stream;
+// waits for it
+hipError_t copy_to_host(ftd_heat* h, const double* src, double* dst, size_t bytes) {
+    hipError_t e;
+    hipPointerAttribute_t at{};
+    // (memory that the runtime knows, pinned or managed, it copies to itself)
+    const bool known = hipPointerGetAttributes(&at, dst) == hipSuccess &&
+                       at.type != hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+    int dev = 0;
+    if (bytes >= kCopyFrom && !known && hipGetDevice(&dev) == hipSuccess && copy_ring(h)) {
+        hipError_t got[kCopyThreads];
+        std::thread th[kCopyThreads];
+        for (int t = 1; t < kCopyThreads; ++t) {
+            auto part = [=, &got] {
+                got[t] = copy_pieces(h, dev, t, (const char*)src, (char*)dst, bytes);
+            };
+            try {
+                th[t] = std::thread(part);
+            } catch (const std::system_error&) {
+                part();  // no thread to be had: here
+            }
+        }
+        got[0] = copy_pieces(h, dev, 0, (const char*)src, (char*)dst, bytes);
+        for (int t = 1; t < kCopyThreads; ++t)
+            if (th[t].joinable()) th[t].join();
+        e = hipStreamSynchronize(h->stream);
+        for (int t = 0; t < kCopyThreads; ++t)
+            if (got[t] != hipSuccess) e = got[t];
+        return e;
+    }
+    if ((e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, h->stream)) != hipSuccess)
+        return e;
+    return hipStreamSynchronize(h->stream);
+}
+
 // the materialized sweep of direction d runs the fused plan's partitioning
 // (with one caller partition the plan picks it), so both give the same bits
 ftd_status sync_solver_plan(ftd_heat* h, int d) {
@@ -1588,6 +1681,9 @@ ftd_status ftd_heat_destroy(ftd_heat* h) {
         if (p) hipFree(p);
     for (AdiRow* p : h->coef)
         if (p) hipFree(p);
+    if (h->pinned) hipHostFree(h->pinned);
+    for (hipEvent_t e : h->slot)
+        if (e) hipEventDestroy(e);
     if (h->e0) hipEventDestroy(h->e0);
     if (h->e1) hipEventDestroy(h->e1);
     if (h->own_stream && h->stream) hipStreamDestroy(h->stream);
@@ -1709,14 +1805,12 @@ ftd_status ftd_heat_set_fused(ftd_heat* h, int enable) {
 ftd_status ftd_heat_field(ftd_heat* h, double* host_out) {
     if (!h || !host_out) return herr(FTD_ERR_INVALID, "null argument");
     const Dims& g = h->g;
-    // packed into rhs (free between steps), then one linear copy
+    // packed into rhs (free between steps), then copied linearly
     const size_t lines = (size_t)g.ny1 * (h->nz + 2);
     hipLaunchKernelGGL((k_lines<true>), dim3((unsigned)lines), dim3(128), 0, h->stream, h->th,
                        h->rhs, g);
     HH(hipGetLastError());
-    HH(hipMemcpyAsync(host_out, h->rhs, sizeof(double) * lines * g.nx1, hipMemcpyDeviceToHost,
-                      h->stream));
-    HH(hipStreamSynchronize(h->stream));
+    HH(copy_to_host(h, h->rhs, host_out, sizeof(double) * lines * g.nx1));
     return FTD_OK;
 }
 
