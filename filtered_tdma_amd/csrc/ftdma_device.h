@@ -14,6 +14,33 @@ __host__ __device__ inline void part_of(int n, int P, int p, int& s, int& m) {
     m = base + (p < rem ? 1 : 0);
 }
 
+// float -> int truncation that saturates instead of being undefined, NaN -> 0
+__device__ inline long long trunc_sat(double x) {
+    if (x != x) return 0;
+    if (x >= 2147483647.0) return 2147483647LL;
+    if (x <= -2147483648.0) return -2147483648LL;
+    return (long long)(int)x;
+}
+
+// k_cal_J_rhs_bound's formula (filtered_tdma_kernels.cuh:245-259) with the
+// clamp to [0, n_row-1]
+__device__ inline int cal_J_gpu(double rho, double max_b, double eps, int n_row) {
+    if (rho == 0.0 || rho >= 0.5) return n_row - 1;
+    double lambda_p = (1.0 + sqrt(1.0 - 4.0 * rho * rho)) * 0.5;
+    double q = rho / lambda_p;
+    double Bv = q * (2.0 + q) / ((1.0 - q) * (1.0 - 2.0 * rho)) * max_b;
+    long long J = trunc_sat(log(eps / Bv) / log(q)) + 1;
+    if (J > n_row - 1) J = n_row - 1;
+    if (J < 0) J = 0;
+    return (int)J;
+}
+
+// max over aligned groups of `width` lanes (width a power of two <= 64)
+__device__ inline double group_max(double v, int width) {
+    for (int off = width >> 1; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
+    return v;
+}
+
 // Reduced system of NR rows (B == 1) in LDS, row k of this lane's system at
 // index k * S, solved by Thomas in place (x to Dr). 4 rows at a time: their
 // values are read into registers first and c', d' are carried in registers,

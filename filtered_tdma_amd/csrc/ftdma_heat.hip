@@ -28,9 +28,11 @@
 #include <string>
 #include <system_error>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/ftdma.h"
+#include "ftdma_device.h"
 #include "ftdma_kernels.h"
 #include "ftdma_xcd.h"
 
@@ -619,29 +621,228 @@ __global__ __launch_bounds__(adi_threads(M, RHSZ)) void k_adi_yz(const double* _
 }
 
 // ---------------------------------------------------------------------------
-// Fused y or z sweep of the filtered kinds over the caller's partitions in
+// Fused y or z sweeps of the filtered kinds over the caller's partitions in
 // that direction (Dirichlet walls). The rows are generated as k_build forms
 // them (a = -s.a, b = 1 - s.b, c = -s.c of the direction; d = for z the
 // explicit rhs of th as k_rhs_z forms it, for y the rhs array; the wall
 // fold-in on the system's first and last rows), and the solve is
 // k_filtered_fused's (ftdma_kernels.hip), statement for statement: the bits
-// of the materialized build + solve + scatter, x written into rhs.
-//   VERSION 2, PASS 0: one pass with J[q] (k_bound_maxabs + k_compute_J).
-//   VERSION 1, PASS 1: x0, xN of every (partition, system) to xbuf, the
-//     tile's largest |x0|, |xN| per partition to partial[tile * Q + q];
-//   VERSION 1, PASS 2: the same sweeps, x0, xN from xbuf, J[q] applied.
-// One lane per (system, partition q); S systems per workgroup.
+// of the materialized build + solve + scatter, x written into rhs. One lane
+// per (system, partition q); S systems per workgroup.
+//
+//   filtered_v2 (k_adi_filt2): J first (k_bound_maxabs + k_compute_J), since
+//     its sweeps depend on J; one pass.
+//   filtered (k_adi_filt1, k_filt_correct): the sweeps do not depend on J, so
+//     the first pass stores them (x0 and xN in the partition's end rows) with
+//     the tile's largest |x0|, |xN| per partition, and the second corrects the rows
+//     that J reaches.
 // ---------------------------------------------------------------------------
+
+// the tile's place of a lane of k_adi_filt1 / 2
+template <int DIR>
+struct FiltLane {
+    int q, sl, n_sys, N, blk, s, ii, oo, r0, m;
+    bool live;
+    size_t rs, here0;
+    __device__ __forceinline__ FiltLane(const Dims& g, int nz, int Q, int lgS, bool whole) {
+        const int S = 1 << lgS;
+        const int t = threadIdx.x;
+        sl = t & (S - 1);
+        // whole: every wave holds one partition, so its rows' bounds are scalar
+        q = whole ? __builtin_amdgcn_readfirstlane(t >> lgS) : t >> lgS;
+        n_sys = g.nx * (DIR == 2 ? g.ny : nz);
+        N = DIR == 2 ? nz : g.ny;
+        // z: each XCD takes a contiguous run of system blocks, so the halo lines
+        // of th its workgroups read are the ones their neighbours read
+        blk = DIR == 2 ? ftd::xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
+        const int s_raw = blk * S + sl;
+        live = s_raw < n_sys;
+        s = live ? s_raw : n_sys - 1;  // dead lanes shadow the last system
+        ii = s % g.nx + 1;
+        oo = s / g.nx + 1;
+        rs = DIR == 2 ? (size_t)g.px * g.ny1 : (size_t)g.px;
+        here0 = DIR == 2 ? cell(g, ii, oo, 1) : cell(g, ii, 1, oo);
+        ftd::part_of(N, Q, q, r0, m);
+    }
+};
+
+// filtered: the sweeps of every partition, their elimination factors from a
+// table (filt_table) as in the exact sweeps: a lane carries only d. One pass
+// over th or rhs instead of two that each formed every row's a', c' again. At
+// 64^3, z in 4 partitions of 16 rows: 5.6 us, J 3.8 with its launch 3.8 more, 7.6
+// for the second pass, now 7.7 and 6.2; at 256^3 the whole step, z in 4, 0.358 -> 0.256 ms.
+template <int M, int DIR, int SPAN>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_adi_filt1(
+    const double* __restrict__ th, double* rhs, Dims g, int nz, double sa, double sc, int Q,
+    int lgS, Stencil st, const AdiRow* __restrict__ tab, const double* __restrict__ cx,
+    const double* __restrict__ cy, const double* __restrict__ cz, double* __restrict__ partial) {
+    extern __shared__ double lds[];
+    const int S = 1 << lgS;
+    const FiltLane<DIR> L(g, nz, Q, lgS, SPAN == 1);
+    const int q = L.q, m = L.m, sl = L.sl;
+    double* const sDl = lds;         // d0 of every partition
+    double* const sDr = lds + Q * S; // dN
+    // SPAN 0: the table in LDS, read by each lane at its own partition
+    AdiRow* const ltab = (AdiRow*)(lds + 2 * Q * S);
+    if (SPAN == 0)
+        for (int k = threadIdx.x; k < 4 * Q * M; k += S * Q)
+            ((double*)ltab)[k] = ((const double*)tab)[k];
+    // the couplings to the neighbours: a0 and cN of this partition, cN of
+    // the one before and a0 of the one after
+    const int ql = q > 0 ? q - 1 : 0, qr = q < Q - 1 ? q + 1 : Q - 1;
+    int unused, ml;
+    ftd::part_of(L.N, Q, ql, unused, ml);
+    const double a0 = tab[q * M].c, cN = tab[q * M + m - 1].cf;
+    const double cNl = tab[ql * M + ml - 1].cf, a0r = tab[qr * M].c;
+    const size_t lo = L.here0, hi = L.here0 + (size_t)(L.N - 1) * L.rs;
+    const double wl = q == 0 ? sa * (th[lo - L.rs] + th[lo]) : 0.0;
+    const double wh = q == Q - 1 ? sc * (th[hi + L.rs] + th[hi]) : 0.0;
+    LaneCell<double> out(rhs, L.here0);
+    out += (ptrdiff_t)((size_t)L.r0 * L.rs);
+
+    auto solve = [&](auto rows, auto pf) {
+        constexpr int PF = decltype(pf)::value;
+        const double aj = -sa;
+        double d[M];
+#pragma unroll
+        for (int j = 0; j < PF && j < M; ++j) d[j] = rows(j);
+        if (SPAN == 0) __syncthreads();
+        const AdiTable<M, SPAN> T(SPAN == 0 ? ltab : tab, q, Q);
+        double dN = 0.0;
+#pragma unroll
+        for (int j = 0; j < M; ++j) {
+            if (j + PF < M) d[j + PF] = rows(j + PF);
+            const double k = T.inv(j);
+            if (j < m) {
+                FTD_ADI_BRANCH;
+                double dj = d[j];
+                if (j == 0) dj = q == 0 ? dj + wl : dj;
+                if (j >= 2) dj = (j == m - 1 && q == Q - 1) ? dj + wh : dj;
+                if (j < 2)
+                    d[j] = dj * k;
+                else
+                    d[j] = k * (dj - aj * d[j >= 1 ? j - 1 : 0]);
+                if (j == m - 1) dN = d[j];
+            }
+        }
+#pragma unroll
+        for (int j = M - 3; j >= 1; --j) {
+            const double k = T.cf(j);
+            if (j <= m - 3) {
+                FTD_ADI_BRANCH;
+                d[j] = d[j] - k * d[j + 1];
+            }
+        }
+        const double d0 = T.a(0) * (d[0] - T.cf(0) * d[1]);
+        // neighbour exchange and the interface 2x2 solves, both formed on
+        // every lane and selected
+        sDl[q * S + sl] = d0;
+        sDr[q * S + sl] = dN;
+        __syncthreads();
+        const double xl = (d0 - a0 * sDr[ql * S + sl]) / (1.0 - cNl * a0);
+        const double xr = (dN - cN * sDl[qr * S + sl]) / (1.0 - a0r * cN);
+        const double x0 = q > 0 ? xl : d0;
+        const double xN = q < Q - 1 ? xr : dN;
+        // dead lanes shadow a live system of this workgroup: the max holds
+        const double v = ftd::group_max(fmax(fabs(x0), fabs(xN)), S);
+        if (sl == 0) partial[(size_t)L.blk * Q + q] = v;
+        if (L.live) {
+#pragma unroll
+            for (int j = 0; j < M; ++j) {
+                if (j < m) {
+                    out[0] = j == 0 ? x0 : j == m - 1 ? xN : d[j];
+                    out += (ptrdiff_t)L.rs;
+                }
+            }
+        }
+    };
+    if constexpr (DIR == 2) {
+        LaneCell<const double> c0(th, L.here0);
+        c0 += (ptrdiff_t)((size_t)L.r0 * L.rs);
+        RowRhsZ<LaneCell<const double>> rows{c0, cz + L.r0 + 1, (ptrdiff_t)g.px, (ptrdiff_t)L.rs, m,
+                     st.xa, st.xc, st.ya, st.yc, st.za, st.zc, 1.0 + st.xb + st.yb + st.zb,
+                     st.c0 * cx[L.ii] * cy[L.oo]};
+        solve(rows, std::integral_constant<int, M <= 16 ? 8 : 4>{});
+    } else {
+        RowAt<LaneCell<double>> rows{out, (ptrdiff_t)L.rs, m};
+        solve(rows, std::integral_constant<int, M>{});
+    }
+}
+
+// The truncated correction (k_final_pass) of k_adi_filt1's rows: x_j -= a'_j x0
+// up to row J, c'_j xN from row m - 1 - J on; 8 rows of a partition per
+// thread, each thread by itself, the rows that J does not reach untouched.
+// OWN_J: a workgroup finds its partition's J itself from the tile maxima (as
+// k_compute_J does, whose launch that saves) with its rows' loads in flight.
+constexpr int kCorrRows = 8;
+template <int DIR, bool OWN_J>
+__global__ __launch_bounds__(64) void k_filt_correct(
+    double* rhs, Dims g, int nz, int Q, int M, int nb, const AdiRow* __restrict__ tab,
+    int* __restrict__ J_all, const double* __restrict__ partial, int n_tiles,
+    const double* __restrict__ rho, double eps_value, int eps_direct) {
+    const int n_sys = g.nx * (DIR == 2 ? g.ny : nz);
+    const int N = DIR == 2 ? nz : g.ny;
+    const int q = blockIdx.y / nb, j0 = (blockIdx.y - q * nb) * kCorrRows;
+    int r0, m;
+    ftd::part_of(N, Q, q, r0, m);
+    if (j0 >= m) return;
+    const int s_raw = blockIdx.x * 64 + threadIdx.x;
+    const int s = s_raw < n_sys ? s_raw : n_sys - 1;
+    const int ii = s % g.nx + 1, oo = s / g.nx + 1;
+    const size_t rs = DIR == 2 ? (size_t)g.px * g.ny1 : (size_t)g.px;
+    double* const p = rhs + (DIR == 2 ? cell(g, ii, oo, 1) : cell(g, ii, 1, oo)) + (size_t)r0 * rs;
+    double d[kCorrRows];
+    int J;
+    if (OWN_J) {
+#pragma unroll
+        for (int u = 0; u < kCorrRows; ++u) d[u] = p[(size_t)(j0 + u < m ? j0 + u : m - 1) * rs];
+    }
+    if (OWN_J) {
+        const double* const c_rho = rho + (N + 1);
+        double vb = 0.0, vr = 0.0;
+        for (int t = threadIdx.x; t < n_tiles; t += 64) vb = fmax(vb, partial[(size_t)t * Q + q]);
+        for (int k = 1 + threadIdx.x; k < m; k += 64)
+            vr = fmax(vr, fmax(fabs(rho[r0 + k]), fabs(c_rho[r0 + k])));
+        vb = ftd::group_max(vb, 64);
+        vr = ftd::group_max(vr, 64);
+        const double Nl = (double)(m * Q);
+        J = ftd::cal_J_gpu(vr, vb, eps_direct ? eps_value : eps_value / (Nl * Nl), m);
+        if (blockIdx.x == 0 && j0 == 0 && threadIdx.x == 0) J_all[q] = J;
+    } else {
+        J = J_all[q];
+    }
+    const int jL = J < m - 2 ? J : m - 2;
+    const int jR = (m - 1) - J > 1 ? (m - 1) - J : 1;
+    if (s_raw >= n_sys || (j0 > jL && j0 + kCorrRows <= jR)) return;
+    const double x0 = p[0], xN = p[(size_t)(m - 1) * rs];
+    const AdiRow* const T = tab + (size_t)q * M + j0;
+    if (!OWN_J) {
+#pragma unroll
+        for (int u = 0; u < kCorrRows; ++u) {
+            const int j = j0 + u;
+            if (j >= 1 && j <= m - 2 && (j <= jL || j >= jR)) d[u] = p[(size_t)j * rs];
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < kCorrRows; ++u) {
+        const int j = j0 + u;
+        if (j >= 1 && j <= m - 2 && (j <= jL || j >= jR)) {
+            double x = d[u];
+            if (j <= jL) x = x - T[u].a * x0;
+            if (j >= jR) x = x - T[u].c * xN;
+            p[(size_t)j * rs] = x;
+        }
+    }
+}
+
 // rows is taken by value: a reference kept the row source's rolling state
 // in scratch memory (1.5 KB per lane in the 64-row filtered_v2 z variant)
-template <int M, int VERSION, int PASS, typename Rows>
-__device__ __forceinline__ void filt_lane(Rows rows, const double* __restrict__ th, int Q, int q,
-                                          int S, int sl, int m, int n_sys, int s, bool live,
-                                          double sa, double sb, double sc, size_t lo, size_t hi,
-                                          size_t rs, double* pbase, const int* __restrict__ Jp,
-                                          double* __restrict__ xbuf, double* __restrict__ partial,
-                                          int tile, double* lds) {
-    const int J = (VERSION == 2 || PASS == 2) ? Jp[q] : m;
+template <int M, typename Rows>
+__device__ __forceinline__ void filt2_lane(Rows rows, const double* __restrict__ th, int Q, int q,
+                                          int S, int sl, int m, bool live, double sa, double sb,
+                                          double sc, size_t lo, size_t hi, size_t rs,
+                                          double* pbase, const int* __restrict__ Jp, double* lds) {
+    const int J = Jp[q];
     constexpr int PF = M >= 32 ? 2 : 4;
     double rd[M];
 #pragma unroll
@@ -650,7 +851,7 @@ __device__ __forceinline__ void filt_lane(Rows rows, const double* __restrict__ 
     double a[M], c[M], d[M];
     double aN = 0.0, cN = 0.0, dN = 0.0;
     double b1 = 1.0;
-    // forward sweep (k_fwd_pass_v1 / k_fwd_pass_v2)
+    // forward sweep (k_fwd_pass_v2)
 #pragma unroll
     for (int j = 0; j < M; ++j) {
         if (j + PF < M) rd[j + PF] = rows(j + PF);
@@ -664,7 +865,7 @@ __device__ __forceinline__ void filt_lane(Rows rows, const double* __restrict__ 
                 c[j] = cj * r;
                 d[j] = dj * r;
                 if (j == 1) b1 = bj;
-            } else if (VERSION == 1 || j <= J) {
+            } else if (j <= J) {
                 const double inv = 1.0 / (bj - aj * c[j - 1]);
                 d[j] = inv * (dj - aj * d[j - 1]);
                 c[j] = inv * cj;
@@ -675,7 +876,7 @@ __device__ __forceinline__ void filt_lane(Rows rows, const double* __restrict__ 
                 c[j] = inv * cj;
                 a[j] = aj;  // left raw, as the skip-A loop leaves A[j]
             }
-            if (VERSION == 2 && j == 1 && J == 0) {
+            if (j == 1 && J == 0) {
                 // k_fwd_pass_v2 with J == 0 eliminates the normalised row 1
                 // against itself
                 const double inv = 1.0 / (b1 - a[1] * c[1]);
@@ -689,23 +890,18 @@ __device__ __forceinline__ void filt_lane(Rows rows, const double* __restrict__ 
             }
         }
     }
-    // backward sweep (k_bwd_pass_v1 / k_bwd_pass_v2)
+    // backward sweep (k_bwd_pass_v2)
     const int lo_c = (m - 2) - J;
 #pragma unroll
     for (int j = M - 3; j >= 1; --j) {
         if (j <= m - 3) {
             const double cj = c[j];
             d[j] = d[j] - cj * d[j + 1];
-            if (VERSION == 1) {
-                a[j] = a[j] - cj * a[j + 1];
-                c[j] = -cj * c[j + 1];
-            } else {
-                if (J >= 2 && j < J) {
-                    const double an = (J == m - 1 && j == m - 3) ? aN : a[j + 1];
-                    a[j] = a[j] - cj * an;
-                }
-                if (j > lo_c) c[j] = -cj * c[j + 1];
+            if (J >= 2 && j < J) {
+                const double an = (J == m - 1 && j == m - 3) ? aN : a[j + 1];
+                a[j] = a[j] - cj * an;
             }
+            if (j > lo_c) c[j] = -cj * c[j + 1];
         }
     }
     // pack_reduced: row 0 keeps d0, a0 (its c0 coupling dropped)
@@ -713,40 +909,23 @@ __device__ __forceinline__ void filt_lane(Rows rows, const double* __restrict__ 
     const double d0p = rr * (d[0] - c[0] * d[1]);
     const double a0p = rr * a[0];
 
-    double x0, xN;
-    if (PASS == 2) {
-        x0 = xbuf[(size_t)(2 * q) * n_sys + s];
-        xN = xbuf[(size_t)(2 * q + 1) * n_sys + s];
-    } else {
-        // neighbour exchange through LDS and the interface 2x2 solves, both
-        // formed on every lane and selected (no lane-divergent branch while
-        // the rows are held in registers)
-        double* sC = lds;
-        double* sDr = sC + Q * S;
-        double* sA = sDr + Q * S;
-        double* sDl = sA + Q * S;
-        sC[q * S + sl] = cN;
-        sDr[q * S + sl] = dN;
-        sA[q * S + sl] = a0p;
-        sDl[q * S + sl] = d0p;
-        __syncthreads();
-        const int ql = q > 0 ? q - 1 : 0, qr = q < Q - 1 ? q + 1 : Q - 1;
-        const double xl = (d0p - a0p * sDr[ql * S + sl]) / (1.0 - sC[ql * S + sl] * a0p);
-        const double xr = (dN - cN * sDl[qr * S + sl]) / (1.0 - sA[qr * S + sl] * cN);
-        x0 = q > 0 ? xl : d0p;
-        xN = q < Q - 1 ? xr : dN;
-    }
-    if (PASS == 1) {
-        if (live) {
-            xbuf[(size_t)(2 * q) * n_sys + s] = x0;
-            xbuf[(size_t)(2 * q + 1) * n_sys + s] = xN;
-        }
-        // dead lanes shadow a live system of this workgroup: the max holds
-        double v = fmax(fabs(x0), fabs(xN));
-        for (int off = S >> 1; off >= 1; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
-        if (sl == 0) partial[(size_t)tile * Q + q] = v;
-        return;
-    }
+    // neighbour exchange through LDS and the interface 2x2 solves, both
+    // formed on every lane and selected (no lane-divergent branch while
+    // the rows are held in registers)
+    double* sC = lds;
+    double* sDr = sC + Q * S;
+    double* sA = sDr + Q * S;
+    double* sDl = sA + Q * S;
+    sC[q * S + sl] = cN;
+    sDr[q * S + sl] = dN;
+    sA[q * S + sl] = a0p;
+    sDl[q * S + sl] = d0p;
+    __syncthreads();
+    const int ql = q > 0 ? q - 1 : 0, qr = q < Q - 1 ? q + 1 : Q - 1;
+    const double xl = (d0p - a0p * sDr[ql * S + sl]) / (1.0 - sC[ql * S + sl] * a0p);
+    const double xr = (dN - cN * sDl[qr * S + sl]) / (1.0 - sA[qr * S + sl] * cN);
+    const double x0 = q > 0 ? xl : d0p;
+    const double xN = q < Q - 1 ? xr : dN;
     // k_final_pass: truncated correction
     const int jL = J < m - 2 ? J : m - 2;
     const int jR = (m - 1) - J > 1 ? (m - 1) - J : 1;
@@ -772,47 +951,26 @@ __device__ __forceinline__ void filt_lane(Rows rows, const double* __restrict__ 
 
 // DIR 2 (z: systems (x, y), rows strided by a plane, d formed from th) or
 // 1 (y: systems (x, z), rows strided by a line, d read from rhs)
-template <int M, int VERSION, int PASS, int DIR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(M >= 64 ? 1 : 2))) void k_adi_filt(
+template <int M, int DIR>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(M >= 64 ? 1 : 2))) void k_adi_filt2(
     const double* __restrict__ th, double* rhs, Dims g, int nz, double sa, double sb, double sc,
     int Q, int lgS, Stencil st, const double* __restrict__ cx, const double* __restrict__ cy,
-    const double* __restrict__ cz, const int* __restrict__ Jp, double* __restrict__ xbuf,
-    double* __restrict__ partial) {
+    const double* __restrict__ cz, const int* __restrict__ Jp) {
     extern __shared__ double lds[];
-    const int S = 1 << lgS;
-    const int t = threadIdx.x;
-    const int sl = t & (S - 1);
-    const int q = t >> lgS;
-    const int n_sys = g.nx * (DIR == 2 ? g.ny : nz);
-    const int N = DIR == 2 ? nz : g.ny;
-    // z: each XCD takes a contiguous run of system blocks, so the halo lines
-    // of th its workgroups read are the ones their neighbours read
-    const int blk = DIR == 2 ? ftd::xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
-    const int s_raw = blk * S + sl;
-    const bool live = s_raw < n_sys;
-    const int s = live ? s_raw : n_sys - 1;  // dead lanes shadow the last system
-    const int ii = s % g.nx + 1, oo = s / g.nx + 1;
-    const size_t rs = DIR == 2 ? (size_t)g.px * g.ny1 : (size_t)g.px;
-    const size_t here0 = DIR == 2 ? cell(g, ii, oo, 1) : cell(g, ii, 1, oo);
-    int r0, m;
-    {
-        const int base = N / Q, rem = N % Q;
-        r0 = q * base + (q < rem ? q : rem);
-        m = base + (q < rem ? 1 : 0);
-    }
-    const size_t lo = here0, hi = here0 + (size_t)(N - 1) * rs;
-    double* const pbase = rhs + here0 + (size_t)r0 * rs;
+    const FiltLane<DIR> L(g, nz, Q, lgS, false);
+    const size_t lo = L.here0, hi = L.here0 + (size_t)(L.N - 1) * L.rs;
+    double* const pbase = rhs + L.here0 + (size_t)L.r0 * L.rs;
     if constexpr (DIR == 2) {
-        RowRhsZ<const double*> rows{th + here0 + (size_t)r0 * rs, cz + r0 + 1, (ptrdiff_t)g.px,
-                                    (ptrdiff_t)rs, m,
+        RowRhsZ<const double*> rows{th + L.here0 + (size_t)L.r0 * L.rs, cz + L.r0 + 1,
+                     (ptrdiff_t)g.px, (ptrdiff_t)L.rs, L.m,
                      st.xa, st.xc, st.ya, st.yc, st.za, st.zc, 1.0 + st.xb + st.yb + st.zb,
-                     st.c0 * cx[ii] * cy[oo]};
-        filt_lane<M, VERSION, PASS>(rows, th, Q, q, S, sl, m, n_sys, s, live, sa, sb, sc, lo, hi,
-                                    rs, pbase, Jp, xbuf, partial, blk, lds);
+                     st.c0 * cx[L.ii] * cy[L.oo]};
+        filt2_lane<M>(rows, th, Q, L.q, 1 << lgS, L.sl, L.m, L.live, sa, sb, sc, lo, hi, L.rs,
+                      pbase, Jp, lds);
     } else {
-        RowAt<const double*> rows{pbase, (ptrdiff_t)rs, m};
-        filt_lane<M, VERSION, PASS>(rows, th, Q, q, S, sl, m, n_sys, s, live, sa, sb, sc, lo, hi,
-                                    rs, pbase, Jp, xbuf, partial, blk, lds);
+        RowAt<const double*> rows{pbase, (ptrdiff_t)L.rs, L.m};
+        filt2_lane<M>(rows, th, Q, L.q, 1 << lgS, L.sl, L.m, L.live, sa, sb, sc, lo, hi, L.rs,
+                      pbase, Jp, lds);
     }
 }
 
@@ -1031,7 +1189,7 @@ struct ftd_heat {
     } fused[3];
     AdiRow* coef[3] = {nullptr, nullptr, nullptr};  // elimination factors of the fused sweeps
     // fused y, z sweeps of the filtered kinds over the caller's partitions
-    // (k_adi_filt): enabled, rows per lane, partitions, log2 systems per
+    // (k_adi_filt1, k_adi_filt2): enabled, rows per lane, partitions, log2 systems per
     // workgroup, dynamic LDS bytes of the exchange (x stays materialized)
     struct Filt {
         int on = 0, M = 0, Q = 0, lgS = 0;
@@ -1106,16 +1264,63 @@ void adi_table(int N, int Q, int M, bool thomas, double sa, double sb, double sc
     }
 }
 
+// The same for the filtered kind's sweep over Q partitions (k_adi_filt1), by
+// k_filtered_fused's statements: rows 0 and 1 multiplied by inv = 1 / b; row 0:
+// a = 1 / (1 - a'_1 c'_0), c = a'_0 of the reduced row.
+void filt_table(int N, int Q, int M, double sa, double sb, double sc, std::vector<AdiRow>& tab) {
+    tab.assign((size_t)Q * M + 2 * Q, AdiRow{1.0, 0.0, 0.0, 0.0});
+    std::vector<double> a(M), c(M);
+    for (int q = 0; q < Q; ++q) {
+        const int base = N / Q, rem = N % Q, m = base + (q < rem ? 1 : 0);
+        AdiRow* const t = &tab[(size_t)q * M];
+        for (int j = 0; j < m; ++j) {
+            const double aj = -sa, cj = -sc;
+            double bj = 1.0 - sb;
+            if (j == 0 && q == 0) bj += sa;
+            if (j == m - 1 && q == Q - 1) bj += sc;
+            if (j < 2) {
+                const double r = 1.0 / bj;
+                t[j].inv = r;
+                a[j] = aj * r;
+                c[j] = cj * r;
+            } else {
+                const double inv = 1.0 / (bj - aj * c[j - 1]);
+                t[j].inv = inv;
+                c[j] = inv * cj;
+                a[j] = -inv * aj * a[j - 1];
+            }
+            t[j].cf = c[j];
+        }
+        for (int j = m - 3; j >= 1; --j) {
+            const double cj = c[j];
+            a[j] = a[j] - cj * a[j + 1];
+            c[j] = -cj * c[j + 1];
+        }
+        for (int j = 1; j < m; ++j) {
+            t[j].a = a[j];
+            t[j].c = c[j];
+        }
+        const double rr = 1.0 / (1.0 - a[1] * c[0]);
+        t[0].a = rr;
+        t[0].c = rr * a[0];
+    }
+}
+
 // forms and uploads the factors of direction d's fused sweep (no step is in
 // flight: steps are waited for)
 hipError_t upload_table(ftd_heat* h, int d) {
     const ftd_heat::Fused& f = h->fused[d];
-    if (!f.on) return hipSuccess;
+    const ftd_heat::Filt& ft = h->filt[d];
+    const bool filt = ft.on && h->kind == FTD_KIND_FILTERED;
+    if (!f.on && !filt) return hipSuccess;
     const int N[3] = {h->g.nx, h->g.ny, h->nz};
     const double sa[3] = {h->s.xa, h->s.ya, h->s.za}, sb[3] = {h->s.xb, h->s.yb, h->s.zb},
                  sc[3] = {h->s.xc, h->s.yc, h->s.zc};
     std::vector<AdiRow> tab;
-    adi_table(N[d], f.Q, f.M, f.thomas != 0, sa[d], sb[d], sc[d], tab);
+    if (f.on)
+        adi_table(N[d], f.Q, f.M, f.thomas != 0, sa[d], sb[d], sc[d], tab);
+    else
+        filt_table(N[d], ft.Q, ft.M, sa[d], sb[d], sc[d], tab);
     return hipMemcpy(h->coef[d], tab.data(), sizeof(AdiRow) * tab.size(), hipMemcpyHostToDevice);
 }
 
@@ -1242,6 +1447,40 @@ bool filt_ready(ftd_heat* h, int d) {
     return ftd::handle_filtered_state(h->solver[d], &J, &rho, &ev, &ed) == FTD_OK;
 }
 
+// k_filt_correct finds J itself up to this many tiles (each of its workgroups
+// reads all of their maxima), beyond it k_compute_J does once
+constexpr int kOwnJTiles = 512;
+
+template <int M, int DIR, int SPAN>
+hipError_t launch_filt1_t(ftd_heat* h, hipStream_t st, int* J, const double* rho, double ev,
+                          int ed) {
+    const ftd_heat::Filt& f = h->filt[DIR];
+    const Dims g = h->g;
+    const Stencil& s = h->s;
+    const int S = 1 << f.lgS, n_sys = g.nx * (DIR == 2 ? g.ny : h->nz);
+    const int N = DIR == 2 ? h->nz : g.ny;
+    const int tiles = (n_sys + S - 1) / S;
+    double* const partial = h->B;  // (the materialized sweeps' B: tile maxima)
+    const size_t lds = sizeof(double) * 2 * S * f.Q + (SPAN == 0 ? sizeof(AdiRow) * f.Q * M : 0);
+    hipLaunchKernelGGL((k_adi_filt1<M, DIR, SPAN>), dim3(tiles), dim3(S * f.Q), lds, st, h->th,
+                       h->rhs, g, h->nz, DIR == 2 ? s.za : s.ya, DIR == 2 ? s.zc : s.yc, f.Q,
+                       f.lgS, s, h->coef[DIR], h->cx, h->cy, h->cz, partial);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const int nb = ((N + f.Q - 1) / f.Q + kCorrRows - 1) / kCorrRows;
+    const dim3 grid((n_sys + 63) / 64, f.Q * nb);
+    if (tiles <= kOwnJTiles) {
+        hipLaunchKernelGGL((k_filt_correct<DIR, true>), grid, dim3(64), 0, st, h->rhs, g, h->nz,
+                           f.Q, M, nb, h->coef[DIR], J, partial, tiles, rho, ev, ed);
+        return hipGetLastError();
+    }
+    if ((e = ftd::launch_compute_J(partial, tiles, f.Q, N, rho, ev, ed, 0, J, st)) != hipSuccess)
+        return e;
+    hipLaunchKernelGGL((k_filt_correct<DIR, false>), grid, dim3(64), 0, st, h->rhs, g, h->nz, f.Q,
+                       M, nb, h->coef[DIR], J, partial, tiles, rho, ev, ed);
+    return hipGetLastError();
+}
+
 template <int M, int DIR>
 hipError_t launch_filt_t(ftd_heat* h, hipStream_t st) {
     const ftd_heat::Filt& f = h->filt[DIR];
@@ -1251,39 +1490,31 @@ hipError_t launch_filt_t(ftd_heat* h, hipStream_t st) {
     int ed;
     if (ftd::handle_filtered_state(h->solver[DIR], &J, &rho, &ev, &ed) != FTD_OK)
         return hipErrorInvalidValue;
+    if (h->kind == FTD_KIND_FILTERED) {
+        // (how a wave holds the factor table: AdiTable)
+        if (f.lgS >= 6) return launch_filt1_t<M, DIR, 1>(h, st, J, rho, ev, ed);
+        if constexpr (M <= 32)
+            if (f.lgS == 5) return launch_filt1_t<M, DIR, 2>(h, st, J, rho, ev, ed);
+        return launch_filt1_t<M, DIR, 0>(h, st, J, rho, ev, ed);
+    }
     const Dims g = h->g;
     const int S = 1 << f.lgS, n_sys = g.nx * (DIR == 2 ? g.ny : h->nz);
     const int N = DIR == 2 ? h->nz : g.ny;
     const dim3 grid((n_sys + S - 1) / S), block(S * f.Q);
-    // scratch: the materialized sweeps' A (x0, xN: 2Q x n_sys) and B (tile
-    // maxima); sweeps run one after the other on the stream
-    double* const xbuf = h->A;
-    double* const partial = h->B;
+    double* const partial = h->B;  // (the materialized sweeps' B: tile maxima)
     const Stencil& s = h->s;
     const double sa = DIR == 2 ? s.za : s.ya, sb = DIR == 2 ? s.zb : s.yb,
                  sc = DIR == 2 ? s.zc : s.yc;
     hipError_t e;
-    if (h->kind == FTD_KIND_FILTERED_V2) {
-        const dim3 gb((n_sys + 255) / 256, f.Q);
-        hipLaunchKernelGGL((k_bound_maxabs<DIR>), gb, dim3(256), 0, st, h->th, h->rhs, g, h->nz,
-                           f.Q, sa, sc, s, h->cx, h->cy, h->cz, partial);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-        if ((e = ftd::launch_compute_J(partial, (int)gb.x, f.Q, N, rho, ev, ed, 0, J, st)) !=
-            hipSuccess)
-            return e;
-        hipLaunchKernelGGL((k_adi_filt<M, 2, 0, DIR>), grid, block, f.lds, st, h->th, h->rhs, g,
-                           h->nz, sa, sb, sc, f.Q, f.lgS, s, h->cx, h->cy, h->cz, J, xbuf,
-                           partial);
-        return hipGetLastError();
-    }
-    hipLaunchKernelGGL((k_adi_filt<M, 1, 1, DIR>), grid, block, f.lds, st, h->th, h->rhs, g, h->nz,
-                       sa, sb, sc, f.Q, f.lgS, s, h->cx, h->cy, h->cz, J, xbuf, partial);
+    const dim3 gb((n_sys + 255) / 256, f.Q);
+    hipLaunchKernelGGL((k_bound_maxabs<DIR>), gb, dim3(256), 0, st, h->th, h->rhs, g, h->nz, f.Q,
+                       sa, sc, s, h->cx, h->cy, h->cz, partial);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    if ((e = ftd::launch_compute_J(partial, (int)grid.x, f.Q, N, rho, ev, ed, 0, J, st)) !=
+    if ((e = ftd::launch_compute_J(partial, (int)gb.x, f.Q, N, rho, ev, ed, 0, J, st)) !=
         hipSuccess)
         return e;
-    hipLaunchKernelGGL((k_adi_filt<M, 1, 2, DIR>), grid, block, 0, st, h->th, h->rhs, g, h->nz,
-                       sa, sb, sc, f.Q, f.lgS, s, h->cx, h->cy, h->cz, J, xbuf, partial);
+    hipLaunchKernelGGL((k_adi_filt2<M, DIR>), grid, block, f.lds, st, h->th, h->rhs, g, h->nz, sa,
+                       sb, sc, f.Q, f.lgS, s, h->cx, h->cy, h->cz, J);
     return hipGetLastError();
 }
 

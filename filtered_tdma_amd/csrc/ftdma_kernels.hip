@@ -47,33 +47,6 @@
 
 namespace ftd {
 
-// float -> int truncation that saturates instead of being undefined, NaN -> 0
-__device__ inline long long trunc_sat(double x) {
-    if (x != x) return 0;
-    if (x >= 2147483647.0) return 2147483647LL;
-    if (x <= -2147483648.0) return -2147483648LL;
-    return (long long)(int)x;
-}
-
-// k_cal_J_rhs_bound's formula (filtered_tdma_kernels.cuh:245-259) with the
-// clamp to [0, n_row-1]
-__device__ inline int cal_J_gpu(double rho, double max_b, double eps, int n_row) {
-    if (rho == 0.0 || rho >= 0.5) return n_row - 1;
-    double lambda_p = (1.0 + sqrt(1.0 - 4.0 * rho * rho)) * 0.5;
-    double q = rho / lambda_p;
-    double Bv = q * (2.0 + q) / ((1.0 - q) * (1.0 - 2.0 * rho)) * max_b;
-    long long J = trunc_sat(log(eps / Bv) / log(q)) + 1;
-    if (J > n_row - 1) J = n_row - 1;
-    if (J < 0) J = 0;
-    return (int)J;
-}
-
-// max over aligned groups of `width` lanes (width a power of two <= 64)
-__device__ inline double group_max(double v, int width) {
-    for (int off = width >> 1; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
-    return v;
-}
-
 // From which boundary maximum v of any one tile on cal_J_gpu gives m - 1, the
 // full correction, for v and every larger one: eps / (B1 v) <= q^(m-2).
 // full_J_scale is B1 q^(m-2), which the column-0 bound alone settles (0: full
