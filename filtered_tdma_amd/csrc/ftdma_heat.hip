@@ -669,8 +669,8 @@ struct FiltLane {
 // filtered: the sweeps of every partition, their elimination factors from a
 // table (filt_table) as in the exact sweeps: a lane carries only d. One pass
 // over th or rhs instead of two that each formed every row's a', c' again. At
-// 64^3, z in 4 partitions of 16 rows: 5.6 us, J 3.8 with its launch 3.8 more, 7.6
-// for the second pass, now 7.7 and 6.2; at 256^3 the whole step, z in 4, 0.358 -> 0.256 ms.
+// 64^3, z in 4 partitions of 16 rows: 5.6 us + J 3.8 + 7.6 for the second
+// pass, FILT1 now.
 template <int M, int DIR, int SPAN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_adi_filt1(
     const double* __restrict__ th, double* rhs, Dims g, int nz, double sa, double sc, int Q,
@@ -1035,10 +1035,18 @@ __host__ __device__ inline int x_tile_stride(int N) { return N + 2 - (N & 1); }
 // workgroup first copies its S lines of rhs into an LDS tile (coalesced,
 // line stride x_tile_stride(N)), solves from the tile, writes x back into the tile and copies the tile to
 // theta (coalesced).
-template <int M, bool THOMAS, int SPAN>
+//
+// GHOSTS: another step follows, whose Dirichlet ghosts this one leaves beside
+// the cells that they mirror (k_dirichlet's values): the sweep is the last of
+// the step, only a line's own wall rows read th's ghosts in it, and they are
+// read before. Saves that launch, 4.3 us at 64^3.
+template <int M, bool THOMAS, int SPAN, bool GHOSTS>
 __global__ __launch_bounds__(256) void k_adi_x(double* th, const double* __restrict__ rhs, Dims g,
                                                int nz, double sa, double sc, int Q, int lgS,
-                                               const AdiRow* __restrict__ tab) {
+                                               const AdiRow* __restrict__ tab,
+                                               const double* __restrict__ cx,
+                                               const double* __restrict__ cy,
+                                               const double* __restrict__ cz) {
     extern __shared__ double lds[];
     const int S = 1 << lgS;
     const int t = threadIdx.x;
@@ -1104,10 +1112,32 @@ __global__ __launch_bounds__(256) void k_adi_x(double* th, const double* __restr
     __syncthreads();
     for (int l = w < nw ? w : nl; l < nl; l += nw) {
         const int s2 = first + l;
-        double* dst = th + cell(g, 1, s2 % g.ny + 1, s2 / g.ny + 1);
+        const int j = s2 % g.ny + 1, k = s2 / g.ny + 1;
+        double* dst = th + cell(g, 1, j, k);
         const double* src = tile + l * LS;
 #pragma unroll 4
         for (int i = lane; i < N; i += step) dst[i] = src[i];
+        if constexpr (GHOSTS) {
+            if (lane == 0) {
+                const double ubc = -cy[j] * cz[k];
+                dst[-1] = 2.0 * ubc - src[0];
+                dst[N] = 2.0 * ubc - src[N - 1];
+            }
+            if (j == 1 || j == g.ny) {
+                double* const gy = th + cell(g, 1, j == 1 ? 0 : g.ny + 1, k);
+                for (int i = lane; i < N; i += step) {
+                    const double ubc = -cx[i + 1] * cz[k];
+                    gy[i] = 2.0 * ubc - src[i];
+                }
+            }
+            if (k == 1 || k == nz) {
+                double* const gz = th + cell(g, 1, j, k == 1 ? 0 : nz + 1);
+                for (int i = lane; i < N; i += step) {
+                    const double ubc = -cx[i + 1] * cy[j];
+                    gz[i] = 2.0 * ubc - src[i];
+                }
+            }
+        }
     }
 }
 
@@ -1177,8 +1207,10 @@ struct ftd_heat {
     ftd_handle* solver[3] = {nullptr, nullptr, nullptr};  // x, y, z sweeps
     int rho_set[3] = {0, 0, 0};  // the solver's column-0 bounds are set (materialized sweeps)
     long steps_done = 0;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
+    // captured: one step, kGraphSteps steps
+    hipGraph_t graph[2] = {nullptr, nullptr};
+    hipGraphExec_t exec[2] = {nullptr, nullptr};
+    int ghosts = 0;  // the step being enqueued leaves the next one's Dirichlet ghosts
     hipEvent_t e0 = nullptr, e1 = nullptr;
     double last_ms = 0.0;
     // fused sweep per direction (x, y, z): enabled, rows per lane, Thomas,
@@ -1540,8 +1572,12 @@ hipError_t launch_adi_t(ftd_heat* h, int d, hipStream_t st) {
     const dim3 grid((n_sys + S - 1) / S), block(T);
     const double sa[3] = {h->s.xa, h->s.ya, h->s.za}, sc[3] = {h->s.xc, h->s.yc, h->s.zc};
     if (d == 0) {
-        hipLaunchKernelGGL((k_adi_x<M, TH, SPAN>), grid, block, f.lds, st, h->th, h->rhs, g, h->nz,
-                           sa[0], sc[0], f.Q, f.lgS, h->coef[0]);
+        if (h->ghosts)
+            hipLaunchKernelGGL((k_adi_x<M, TH, SPAN, true>), grid, block, f.lds, st, h->th, h->rhs,
+                               g, h->nz, sa[0], sc[0], f.Q, f.lgS, h->coef[0], h->cx, h->cy, h->cz);
+        else
+            hipLaunchKernelGGL((k_adi_x<M, TH, SPAN, false>), grid, block, f.lds, st, h->th, h->rhs,
+                               g, h->nz, sa[0], sc[0], f.Q, f.lgS, h->coef[0], h->cx, h->cy, h->cz);
     } else if (d == 2 && h->fuse_rhs) {
         hipLaunchKernelGGL((k_adi_yz<M, TH, true, SPAN>), grid, block, f.lds, st, h->th, h->rhs, g,
                            h->nz, d, sa[d], sc[d], f.Q, f.lgS, h->s, h->coef[d], h->cx, h->cy,
@@ -1577,9 +1613,14 @@ hipError_t launch_adi(ftd_heat* h, int d, hipStream_t st) {
 // dynamic LDS above the default limit must be declared for the kernel
 template <int M, bool TH, int SPAN>
 hipError_t allow_lds_t(int d, size_t bytes) {
-    if (d == 0)
-        return hipFuncSetAttribute((const void*)k_adi_x<M, TH, SPAN>,
+    if (d == 0) {
+        const hipError_t ex = hipFuncSetAttribute((const void*)k_adi_x<M, TH, SPAN, true>,
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                  (int)bytes);
+        if (ex != hipSuccess) return ex;
+        return hipFuncSetAttribute((const void*)k_adi_x<M, TH, SPAN, false>,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    }
     const hipError_t e = hipFuncSetAttribute((const void*)k_adi_yz<M, TH, false, SPAN>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     if (e != hipSuccess || d != 2) return e;
@@ -1606,11 +1647,22 @@ void launch_dirichlet(ftd_heat* h, hipStream_t st) {
                            h->th, g, faces, h->cx, h->cy, h->cz);
 }
 
-ftd_status enqueue_step(ftd_heat* h) {
+// Up to 2^15 lines: the two ghosts of a line are parts of cache lines of their
+// own, which in a sweep bound by memory cost more than the launch (128^3
+// filtered 66.3 -> 64.8 us a step with it, 256^3 218 -> 227).
+bool ghosts_by_x(const ftd_heat* h) {
+    return h->use_fused && h->fused[0].on && !h->periodic[0] && !h->periodic[1] &&
+           !h->periodic[2] && (long)h->g.ny * h->nz <= 32768;
+}
+
+// one step; have: its Dirichlet ghosts are in place; leave: it leaves the next
+// one's (the x sweep of the step has to run fused, ghosts_by_x)
+ftd_status enqueue_step(ftd_heat* h, bool have = false, bool leave = false) {
     const Dims g = h->g;
     hipStream_t st = h->stream;
     const dim3 b2(16, 16);
-    launch_dirichlet(h, st);
+    if (!have) launch_dirichlet(h, st);
+    h->ghosts = leave;
     // the fused z sweep forms the rhs itself (k_adi_yz<..., RHSZ>), except a
     // one-partition (Thomas) sweep with fewer workgroups than CUs: that one
     // is a serial chain per lane on part of the chip, and the separate rhs
@@ -1797,6 +1849,49 @@ ftd_status sync_solver_plan(ftd_heat* h, int d) {
     return FTD_OK;
 }
 
+// Steps of the longer graph. Between two graphs the device waits about 5 us for
+// the next one's first kernel, inside one 1 us or none; and the steps of one
+// leave each other's ghosts. 64^3 filtered: 48.6 -> 44.3 us a step with both. Captured once a call has
+// kGraphFrom times as many steps left, which pay for the capture.
+constexpr int kGraphSteps = 8;
+constexpr int kGraphFrom = 4;
+
+// graph k (0: one step, 1: kGraphSteps) of the present plan
+ftd_status capture(ftd_heat* h, int k) {
+    if (h->exec[k]) return FTD_OK;
+    const int n = k ? kGraphSteps : 1;
+    const bool fold = ghosts_by_x(h);
+    HH(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
+    ftd_status s = FTD_OK;
+    for (int i = 0; i < n && s == FTD_OK; ++i)
+        s = enqueue_step(h, fold && i > 0, fold && i < n - 1);
+    hipGraph_t graph = nullptr;
+    const hipError_t e = hipStreamEndCapture(h->stream, &graph);
+    if (s != FTD_OK) {
+        if (graph) hipGraphDestroy(graph);
+        return s;
+    }
+    HH(e);
+    h->graph[k] = graph;
+    const hipError_t ei = hipGraphInstantiate(&h->exec[k], graph, nullptr, nullptr, 0);
+    if (ei != hipSuccess) {
+        h->exec[k] = nullptr;
+        h->graph[k] = nullptr;
+        hipGraphDestroy(graph);
+    }
+    HH(ei);
+    return FTD_OK;
+}
+
+void drop_graphs(ftd_heat* h) {
+    for (int k = 0; k < 2; ++k) {
+        if (h->exec[k]) hipGraphExecDestroy(h->exec[k]);
+        if (h->graph[k]) hipGraphDestroy(h->graph[k]);
+        h->exec[k] = nullptr;
+        h->graph[k] = nullptr;
+    }
+}
+
 void centres(std::vector<double>& c, int n) {
     c.resize(n + 2);
     const double dd = 2.0 / (double)n;
@@ -1905,8 +2000,7 @@ ftd_status ftd_heat_create(ftd_heat** out, int nx, int ny, int nz, const int* pa
 
 ftd_status ftd_heat_destroy(ftd_heat* h) {
     if (!h) return FTD_OK;
-    if (h->exec) hipGraphExecDestroy(h->exec);
-    if (h->graph) hipGraphDestroy(h->graph);
+    drop_graphs(h);
     for (ftd_handle* s : h->solver) ftd_destroy(s);
     for (double* p : {h->th, h->rhs, h->A, h->B, h->C, h->D, h->cx, h->cy, h->cz})
         if (p) hipFree(p);
@@ -1955,34 +2049,29 @@ ftd_status ftd_heat_init(ftd_heat* h) {
 
 // nsteps ADI steps; use_graph != 0 captures one step into a hipGraph on first
 // use and replays it (the first step always runs eagerly so that every
-// solver scratch buffer exists before capture). Waits for the last step and
-// records its device time.
+// solver scratch buffer exists before capture), and kGraphSteps steps into
+// another in a call of several times as many. Waits for the last step and records its device
+// time.
 ftd_status ftd_heat_step(ftd_heat* h, int nsteps, int use_graph) {
     if (!h) return herr(FTD_ERR_INVALID, "null handle");
-    for (int t = 0; t < nsteps; ++t) {
+    for (int t = 0; t < nsteps;) {
         const bool last = t == nsteps - 1;
+        int done = 1;
         if (last) HH(hipEventRecord(h->e0, h->stream));
         if (use_graph && h->steps_done > 0) {
-            if (!h->exec) {
-                HH(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-                ftd_status s = enqueue_step(h);
-                hipGraph_t graph = nullptr;
-                hipError_t e = hipStreamEndCapture(h->stream, &graph);
-                if (s != FTD_OK) {
-                    if (graph) hipGraphDestroy(graph);
-                    return s;
-                }
-                HH(e);
-                h->graph = graph;
-                HH(hipGraphInstantiate(&h->exec, h->graph, nullptr, nullptr, 0));
-            }
-            HH(hipGraphLaunch(h->exec, h->stream));
+            const int left = nsteps - t;
+            const int k = left > (h->exec[1] ? 1 : kGraphFrom) * kGraphSteps;
+            ftd_status s = capture(h, k);
+            if (s != FTD_OK) return s;
+            HH(hipGraphLaunch(h->exec[k], h->stream));
+            done = k ? kGraphSteps : 1;
         } else {
             ftd_status s = enqueue_step(h);
             if (s != FTD_OK) return s;
         }
         if (last) HH(hipEventRecord(h->e1, h->stream));
-        ++h->steps_done;
+        t += done;
+        h->steps_done += done;
     }
     if (nsteps > 0) {
         HH(hipEventSynchronize(h->e1));
@@ -2020,15 +2109,8 @@ ftd_status ftd_heat_set_plan(ftd_heat* h, int dir, int rows_per_lane, int system
 ftd_status ftd_heat_set_fused(ftd_heat* h, int enable) {
     if (!h) return herr(FTD_ERR_INVALID, "null handle");
     h->use_fused = enable != 0;
-    if (h->exec) {
-        HH(hipStreamSynchronize(h->stream));
-        hipGraphExecDestroy(h->exec);
-        h->exec = nullptr;
-    }
-    if (h->graph) {
-        hipGraphDestroy(h->graph);
-        h->graph = nullptr;
-    }
+    if (h->exec[0] || h->exec[1]) HH(hipStreamSynchronize(h->stream));
+    drop_graphs(h);
     return FTD_OK;
 }
 
