@@ -430,6 +430,7 @@ struct AdiTable {
 // registers. rows(j) returns d of local row j (clamped to the partition),
 // store(j, x) writes x of local row j. The d loads run PF rows ahead of their
 // use (by value: a reference kept a row source's rolling state in scratch).
+// wl, wh: the wall fold-in of the system's first and last rows.
 // Restates k_thomas_fused (Q == 1) and k_pascal_fused (Q >= 2, non-cyclic):
 // rows 0, 1 of a partition divided by b, modified elimination,
 // 2Q-row reduced system in LDS, interior update.
@@ -439,15 +440,11 @@ struct AdiTable {
     if (SPAN == 1) asm volatile("")
 template <int M, int PF, bool THOMAS, int SPAN, typename Rows, typename Store>
 __device__ __forceinline__ void adi_solve_lane(int Q, int q, int cnt, int S, int sl, double sa,
-                                               double sc, const double* __restrict__ th, size_t lo,
-                                               size_t hi, size_t rs, bool live, double* lds,
+                                               double wl, double wh, bool live, double* lds,
                                                const AdiTable<M, SPAN>& T, Rows rows,
                                                Store store) {
     const double aj = -sa;
     double d[M];
-    // the wall fold-in of the system's first and last rows
-    const double wl = (THOMAS || q == 0) ? sa * (th[lo - rs] + th[lo]) : 0.0;
-    const double wh = (THOMAS || q == Q - 1) ? sc * (th[hi + rs] + th[hi]) : 0.0;
 #pragma unroll
     for (int j = 0; j < PF && j < M; ++j) d[j] = rows(j);
     double dN = 0.0;
@@ -603,20 +600,19 @@ __global__ __launch_bounds__(adi_threads(M, RHSZ)) void k_adi_yz(const double* _
         out += (ptrdiff_t)rs;
     };
     const AdiTable<M, SPAN> T(tab, q, Q);
+    const size_t hi0 = here0 + (size_t)(N - 1) * rs;
+    const double wl = (THOMAS || q == 0) ? sa * (th[here0 - rs] + th[here0]) : 0.0;
+    const double wh = (THOMAS || q == Q - 1) ? sc * (th[hi0 + rs] + th[hi0]) : 0.0;
     if (RHSZ) {
         LaneCell<const double> c0(th, here0);
         c0 += (ptrdiff_t)((size_t)r0 * rs);
         RowRhsZ<LaneCell<const double>> rows{c0, cz + r0 + 1, (ptrdiff_t)g.px, (ptrdiff_t)rs, cnt,
                      st.xa, st.xc, st.ya, st.yc, st.za, st.zc, 1.0 + st.xb + st.yb + st.zb,
                      st.c0 * cx[ii] * cy[oo]};
-        adi_solve_lane<M, 4, THOMAS, SPAN>(Q, q, cnt, S, sl, sa, sc, th, here0,
-                                           here0 + (size_t)(N - 1) * rs, rs, live, lds, T, rows,
-                                           store);
+        adi_solve_lane<M, 4, THOMAS, SPAN>(Q, q, cnt, S, sl, sa, wl, wh, live, lds, T, rows, store);
     } else {
         RowAt<LaneCell<double>> rows{first, (ptrdiff_t)rs, cnt};
-        adi_solve_lane<M, M, THOMAS, SPAN>(
-            Q, q, cnt, S, sl, sa, sc, th, here0, here0 + (size_t)(N - 1) * rs, rs, live, lds, T,
-            rows, store);
+        adi_solve_lane<M, M, THOMAS, SPAN>(Q, q, cnt, S, sl, sa, wl, wh, live, lds, T, rows, store);
     }
 }
 
@@ -1067,11 +1063,24 @@ __global__ __launch_bounds__(256) void k_adi_x(double* th, const double* __restr
     // cells start on 128-byte boundaries, tile lines on 16-byte ones), so
     // every line of the tile is in flight at once with no register staging
     // and a wave's DMAs stay under the count of operations it can track.
-    const int step = nt < 64 ? nt : 64, nw = nt / step, w = t / step, lane = t - w * step;
+    // The wave's number is scalar and the lines are counted along, so that a
+    // line's address costs no division; the walls' cells and the factor table
+    // are asked for with the lines: at 64^3, one wave of 16 lines on every CU,
+    // 14.5 -> 13.4 us; 256^3 77 -> 73.
+    const int step = nt < 64 ? nt : 64, nw = nt / step;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
+    const int j0 = (first + w) % g.ny + 1, k0 = (first + w) / g.ny + 1;  // the wave's first line
+    auto next_line = [&](int& j, int& k) {
+        j += nw;
+        while (j > g.ny) {
+            j -= g.ny;
+            ++k;
+        }
+    };
     const int nu = N >> 1;  // 16-byte units per line; an odd N leaves 8 bytes
-    for (int l = w < nw ? w : nl; l < nl; l += nw) {
-        const int s = first + l;
-        const char* src = (const char*)(rhs + cell(g, 1, s % g.ny + 1, s / g.ny + 1));
+    int j = j0, k = k0;
+    for (int l = w < nw ? w : nl; l < nl; l += nw, next_line(j, k)) {
+        const char* src = (const char*)(rhs + cell(g, 1, j, k));
         char* dst = (char*)(tile + (size_t)l * LS);
         for (int e = 0; e < nu; e += step) {
             if (e + lane < nu)
@@ -1084,18 +1093,20 @@ __global__ __launch_bounds__(256) void k_adi_x(double* th, const double* __restr
                                              (__attribute__((address_space(3))) void*)(dst + 16 * nu),
                                              4, 0, 0);
     }
+    // threads past S * Q (a Thomas tile of fewer than 64 lines is launched
+    // as one full wave, so that its copies use 64 lanes and hold the
+    // factor table) solve a line along, as dead lanes do
+    const int s_raw = first + sl;
+    const bool live = s_raw < n_sys && q < Q;
+    const int s = live ? s_raw : n_sys - 1;
+    const int qq = THOMAS ? 0 : SPAN == 1 ? __builtin_amdgcn_readfirstlane(q) : q;
+    const size_t here0 = cell(g, 1, s % g.ny + 1, s / g.ny + 1);
+    const double wl = (THOMAS || qq == 0) ? sa * (th[here0 - 1] + th[here0]) : 0.0;
+    const double wh = (THOMAS || qq == Q - 1) ? sc * (th[here0 + N] + th[here0 + N - 1]) : 0.0;
+    const AdiTable<M, SPAN> T(tab, THOMAS ? 0 : q, Q);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    const AdiTable<M, SPAN> T(tab, THOMAS ? 0 : q, Q);
     {
-        // threads past S * Q (a Thomas tile of fewer than 64 lines is launched
-        // as one full wave, so that its copies use 64 lanes and hold the
-        // factor table) solve a line along, as dead lanes do
-        const int s_raw = first + sl;
-        const bool live = s_raw < n_sys && q < Q;
-        const int s = live ? s_raw : n_sys - 1;
-        const int qq = THOMAS ? 0 : SPAN == 1 ? __builtin_amdgcn_readfirstlane(q) : q;
-        const size_t here0 = cell(g, 1, s % g.ny + 1, s / g.ny + 1);
         int r0, cnt;
         {
             const int base = N / Q, rem = N % Q;
@@ -1106,13 +1117,14 @@ __global__ __launch_bounds__(256) void k_adi_x(double* th, const double* __restr
         double* myline = tile + (size_t)lt * LS + r0;
         RowAt<const double*> rows{myline, 1, cnt};
         adi_solve_lane<M, (M < 32 ? M : 32), THOMAS, SPAN>(
-            Q, qq, cnt, S, sl, sa, sc, th, here0, here0 + (size_t)(N - 1), 1, live, red, T, rows,
-            [&](int j, double x) { myline[j] = x; });
+            Q, qq, cnt, S, sl, sa, wl, wh, live, red, T, rows,
+            [&](int jj, double x) { myline[jj] = x; });
     }
     __syncthreads();
-    for (int l = w < nw ? w : nl; l < nl; l += nw) {
-        const int s2 = first + l;
-        const int j = s2 % g.ny + 1, k = s2 / g.ny + 1;
+    j = j0;
+    k = k0;
+#pragma unroll 4
+    for (int l = w < nw ? w : nl; l < nl; l += nw, next_line(j, k)) {
         double* dst = th + cell(g, 1, j, k);
         const double* src = tile + l * LS;
 #pragma unroll 4
