@@ -336,8 +336,8 @@ ftd_status ftd_heat_destroy(ftd_heat* h);
 /* re-initialise the field to t = 0 (mpi_subdomain.cpp:164-173) */
 ftd_status ftd_heat_init(ftd_heat* h);
 
-/* nsteps time steps (solve_theta.cpp:92-334); use_graph != 0 replays one
- * step captured into a hipGraph. Waits for the last step. */
+/* nsteps time steps (solve_theta.cpp:92-334); use_graph != 0 replays hipGraphs
+ * of one step, and in calls of 32 more steps of 8. Waits for the last step. */
 ftd_status ftd_heat_step(ftd_heat* h, int nsteps, int use_graph);
 
 /* Extension: fused sweeps on (default) or off. Where a sweep's coefficients
