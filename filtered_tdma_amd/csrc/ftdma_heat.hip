@@ -374,17 +374,38 @@ __device__ __forceinline__ double lane_value(double v, int lane) {
                             __builtin_amdgcn_readlane(__double2loint(v), lane));
 }
 
+// value v of lane `lane` (a constant) of each 16 lanes (DPP row_newbcast), for all
+// of the 16: they are active together
+__device__ __forceinline__ double row16_value(double v, int lane) {
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+#define FTD_ROW16(n)                                                          \
+    case n:                                                                   \
+        return __hiloint2double(                                              \
+            __builtin_amdgcn_update_dpp(0, hi, 0x150 + n, 0xf, 0xf, true),    \
+            __builtin_amdgcn_update_dpp(0, lo, 0x150 + n, 0xf, 0xf, true));
+    switch (lane) {
+        FTD_ROW16(0) FTD_ROW16(1) FTD_ROW16(2) FTD_ROW16(3) FTD_ROW16(4) FTD_ROW16(5)
+        FTD_ROW16(6) FTD_ROW16(7) FTD_ROW16(8) FTD_ROW16(9) FTD_ROW16(10) FTD_ROW16(11)
+        FTD_ROW16(12) FTD_ROW16(13) FTD_ROW16(14) FTD_ROW16(15)
+    }
+    return v;
+#undef FTD_ROW16
+}
+
 // A wave's part of the table. With S >= 64 systems per workgroup a wave holds
 // one partition (SPAN 1): lane l keeps row l and the rows reach the others by
 // v_readlane, with no load in the chain of rows (scalar loads there cost a
 // round trip per few rows). At S = 32 and up to 32 rows it holds two (SPAN 2):
 // rows of the lower in lanes 0..31, of the upper in 32..63, each lane takes its
-// own. Else (SPAN 0) each lane loads its own rows. Made with every lane of the
+// own. At S = 16 and up to 32 rows (SPAN 4) every 16 lanes hold a partition:
+// each its rows l and l + 16, which reach the others of the 16 by a DPP row
+// broadcast. Else (SPAN 0) each lane loads its own rows. Made with every lane of the
 // wave active, in workgroups of whole waves for SPAN 1.
 template <int M, int SPAN>
 struct AdiTable {
-    AdiRow own;        // SPAN 1, 2: this lane's row
-    AdiRow red;        // SPAN 1, 2: row l of the reduced system
+    AdiRow own;        // SPAN 1, 2, 4: this lane's row
+    AdiRow own2;       // SPAN 4: and its second one
+    AdiRow red;        // SPAN 1, 2, 4: row l of the reduced system
     const AdiRow* p;   // SPAN 0: the partition's rows
     const AdiRow* rp;  // SPAN 0: the reduced rows
     bool upper;
@@ -396,19 +417,25 @@ struct AdiTable {
             upper = false;
         } else {
             const int q0 = __builtin_amdgcn_readfirstlane(q);
-            const int part = SPAN == 2 && l >= 32 && q0 + 1 < Q ? q0 + 1 : q0;
-            const int row = SPAN == 2 ? l & 31 : l;
+            const int part = SPAN == 4                             ? q
+                             : SPAN == 2 && l >= 32 && q0 + 1 < Q ? q0 + 1
+                                                                  : q0;
+            const int row = SPAN == 4 ? l & 15 : SPAN == 2 ? l & 31 : l;
             own = tab[part * M + (row < M ? row : M - 1)];
+            if (SPAN == 4 && M > 16) own2 = tab[part * M + 16 + row];
             red = tab[Q * M + (l < 2 * Q ? l : 0)];
             upper = SPAN == 2 && l >= 32;
             // every lane's rows are here now: the loads must not sink into a
             // branch that some lanes skip
             asm volatile("" : "+v"(own.inv), "+v"(own.cf), "+v"(own.a), "+v"(own.c));
+            if (SPAN == 4 && M > 16)
+                asm volatile("" : "+v"(own2.inv), "+v"(own2.cf), "+v"(own2.a), "+v"(own2.c));
             asm volatile("" : "+v"(red.inv), "+v"(red.cf), "+v"(red.a));
         }
     }
     __device__ __forceinline__ double get(double AdiRow::* f, int j) const {
         if (SPAN == 0) return p[j].*f;
+        if (SPAN == 4) return row16_value(j < 16 ? own.*f : own2.*f, j & 15);
         const double lo = lane_value(own.*f, j);
         if (SPAN == 1) return lo;
         const double hi = lane_value(own.*f, 32 + (j & 31));
@@ -1431,9 +1458,13 @@ void plan_fused(ftd_heat* h, int d, int N, int n_sys, int rows_per_lane = 0,
     // the tile down to 16 lines until the grid covers the CUs (64^3: 256
     // tiles of 16 lines, 0.073 ms per step against 0.087 with 64 tiles of 64;
     // 8-line tiles were slower again). The bits do not depend on the tile.
+    // Partitions of up to 32 rows take 16 lines always: four workgroups to a CU
+    // where 32 lines leave room for two, so that more of them are in their copies
+    // while one solves (256^3: 212 -> 208 us a step, 200^3 129 -> 124, 128^3
+    // 50.4 -> 49.2, 100^3 52.4 -> 48.8; 8 lines 231 at 256^3).
     if (d == 0 && !systems_per_tile) {
         const int cus = device_cus();
-        while (S > 16 && (n_sys + S - 1) / S < cus) S >>= 1;
+        while (S > 16 && ((!f.thomas && f.M <= 32) || (n_sys + S - 1) / S < cus)) S >>= 1;
     }
     auto lds_of = [&](int S_) {
         const size_t red = f.thomas ? 0 : (size_t)2 * Q * S_;
@@ -1617,6 +1648,7 @@ hipError_t launch_adi_t(ftd_heat* h, int d, hipStream_t st) {
            : (f).thomas                            ? F<m_, true, 0>(__VA_ARGS__) \
            : (f).lgS >= 6                          ? F<m_, false, 1>(__VA_ARGS__) \
            : (f).lgS == 5 && m_ <= 32 ? F<m_, false, m_ <= 32 ? 2 : 0>(__VA_ARGS__) \
+           : (f).lgS == 4 && m_ <= 32 ? F<m_, false, m_ <= 32 ? 4 : 0>(__VA_ARGS__) \
                                       : F<m_, false, 0>(__VA_ARGS__);
 
 hipError_t launch_adi(ftd_heat* h, int d, hipStream_t st) {
