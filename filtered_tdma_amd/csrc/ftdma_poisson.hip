@@ -357,13 +357,17 @@ __global__ __launch_bounds__(kModeThreads, 3) void k_mode_solve(double* __restri
     }
 }
 
-// the FFT plans of layout k: lines of nxh modes (0) or of p->pitch (1)
+// the FFT plans of layout k: lines of nxh modes (0) or of p->pitch (1). A pair
+// takes about 13 ms to make: create makes the one that the step uses,
+// ftd_poisson_solver the other, since a solver has to be asked for to be tuned
 ftd_status fft_plans(ftd_poisson* p, int k) {
+    if (p->have_fwd[k] && p->have_bwd[k]) return FTD_OK;
     const int w = k ? p->pitch : p->nxh;
     int n2[2] = {p->ny, p->nx}, real[2] = {p->ny, p->nx}, modes[2] = {p->ny, w};
     const int dr = p->nx * p->ny, dm = w * p->ny;
-    if (hipfftPlanMany(&p->fwd[k], 2, n2, real, 1, dr, modes, 1, dm, HIPFFT_D2Z, p->nz) !=
-        HIPFFT_SUCCESS)
+    if (!p->have_fwd[k] &&
+        hipfftPlanMany(&p->fwd[k], 2, n2, real, 1, dr, modes, 1, dm, HIPFFT_D2Z, p->nz) !=
+            HIPFFT_SUCCESS)
         return perr(FTD_ERR_HIP, "hipfftPlanMany (D2Z) failed");
     p->have_fwd[k] = 1;
     if (hipfftPlanMany(&p->bwd[k], 2, n2, modes, 1, dm, real, 1, dr, HIPFFT_Z2D, p->nz) !=
@@ -397,10 +401,12 @@ ftd_status poisson_spectral(ftd_poisson* p) {
         PF(hipfftExecZ2D(p->bwd[k], reinterpret_cast<hipfftDoubleComplex*>(p->hat), p->rhs));
         return FTD_OK;
     }
+    ftd_status s = fft_plans(p, 0);
+    if (s != FTD_OK) return s;
     PF(hipfftExecD2Z(p->fwd[0], p->rhs, reinterpret_cast<hipfftDoubleComplex*>(p->hat)));
     hipLaunchKernelGGL(k_pin_zero_mode, dim3(1), dim3(64), 0, p->stream, p->hat);
     PH(hipGetLastError());
-    const ftd_status s = ftd_solve_complex(p->solver, p->A, p->B, p->C, p->hat);
+    s = ftd_solve_complex(p->solver, p->A, p->B, p->C, p->hat);
     if (s != FTD_OK) return perr(s, std::string("z solve: ") + ftd_last_error_string());
     PF(hipfftExecZ2D(p->bwd[0], reinterpret_cast<hipfftDoubleComplex*>(p->hat), p->rhs));
     return FTD_OK;
@@ -509,8 +515,7 @@ ftd_status ftd_poisson_create(ftd_poisson** out, int nx, int ny, int nz, double 
     if (e == hipSuccess) e = hipEventCreate(&p->e1);
     if (e != hipSuccess)
         return bail(perr(FTD_ERR_HIP, std::string("ftd_poisson_create: ") + hipGetErrorString(e)));
-    ftd_status s = fft_plans(p, 0);
-    if (s == FTD_OK && p->pitch > nxh) s = fft_plans(p, 1);
+    ftd_status s = fft_plans(p, p->pitch > nxh);
     if (s != FTD_OK) return bail(s);
     s = ftd_create(&p->solver, kind, nm, nz, partitions, eps_constant, p->stream);
     if (s != FTD_OK) return bail(perr(s, std::string("z solver: ") + ftd_last_error_string()));
@@ -533,7 +538,11 @@ ftd_status ftd_poisson_destroy(ftd_poisson* p) {
     return FTD_OK;
 }
 
-ftd_handle* ftd_poisson_solver(ftd_poisson* p) { return p ? p->solver : nullptr; }
+ftd_handle* ftd_poisson_solver(ftd_poisson* p) {
+    if (!p) return nullptr;
+    (void)fft_plans(p, 0);  // (if they cannot be made, the step that needs them says so)
+    return p->solver;
+}
 
 ftd_status ftd_poisson_solve(ftd_poisson* p, double* U, double* V, double* W, double* P, double dt) {
     if (!p) return perr(FTD_ERR_INVALID, "null handle");
