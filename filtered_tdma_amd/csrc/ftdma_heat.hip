@@ -1571,6 +1571,8 @@ hipError_t launch_filt_t(ftd_heat* h, hipStream_t st) {
         if (f.lgS >= 6) return launch_filt1_t<M, DIR, 1>(h, st, J, rho, ev, ed);
         if constexpr (M <= 32)
             if (f.lgS == 5) return launch_filt1_t<M, DIR, 2>(h, st, J, rho, ev, ed);
+        if constexpr (M <= 32)
+            if (f.lgS == 4) return launch_filt1_t<M, DIR, 4>(h, st, J, rho, ev, ed);
         return launch_filt1_t<M, DIR, 0>(h, st, J, rho, ev, ed);
     }
     const Dims g = h->g;
