@@ -51,14 +51,15 @@ namespace ftd {
 // full correction, for v and every larger one: eps / (B1 v) <= q^(m-2).
 // full_J_scale is B1 q^(m-2), which the column-0 bound alone settles (0: full
 // for every v, NaN: no v that can be told), full_J compares v with eps over
-// it, with 1e-9 to spare for the rounding of the logarithms.
+// it, with 1e-9 to spare for the rounding of the logarithms. A subnormal
+// scale has too few bits for that: no v can be told.
 __device__ inline double full_J_scale(double rho, int m) {
     if (rho == 0.0 || rho >= 0.5) return 0.0;
     const double lambda_p = (1.0 + sqrt(1.0 - 4.0 * rho * rho)) * 0.5;
     const double q = rho / lambda_p;
     const double B1 = q * (2.0 + q) / ((1.0 - q) * (1.0 - 2.0 * rho));
     const double T = B1 * exp((double)(m - 2) * log(q));
-    return T > 0.0 && T < __builtin_inf() ? T : __builtin_nan("");
+    return T >= __DBL_MIN__ && T < __builtin_inf() ? T : __builtin_nan("");
 }
 
 // the v itself: -1 for every v, NaN for none
