@@ -165,7 +165,13 @@ __global__ __launch_bounds__(256) void k_compute_J(const double* __restrict__ pa
     int s, m;
     part_of(n_row, P, p, s, m);
     double vb = 0.0, vr = 0.0;
-    for (int t = threadIdx.x; t < n_tiles; t += 256) vb = fmax(vb, fabs(part[(size_t)t * P + p]));  // (sign: tile stored)
+    // (a negative maximum: the first pass stored that tile with J = m - 1)
+    bool stored = false;
+    for (int t = threadIdx.x; t < n_tiles; t += 256) {
+        const double v = part[(size_t)t * P + p];
+        stored |= __builtin_signbit(v);
+        vb = fmax(vb, fabs(v));
+    }
     for (int k = 1 + threadIdx.x; k < m; k += 256)
         vr = fmax(vr, fmax(fabs(A_rho[s + k]), fabs(C_rho[s + k])));
     vb = group_max(vb, 64);
@@ -174,13 +180,13 @@ __global__ __launch_bounds__(256) void k_compute_J(const double* __restrict__ pa
         red_b[threadIdx.x >> 6] = vb;
         red_r[threadIdx.x >> 6] = vr;
     }
-    __syncthreads();
+    stored = __syncthreads_or(stored) != 0;
     if (threadIdx.x == 0) {
         double mb = fmax(fmax(red_b[0], red_b[1]), fmax(red_b[2], red_b[3]));
         double rho = fmax(fmax(red_r[0], red_r[1]), fmax(red_r[2], red_r[3]));
         double Nl = (double)(m * P);
         double eps = eps_direct ? eps_value : eps_value / (Nl * Nl);
-        J_out[blockIdx.x] = cal_J_gpu(rho, mb, eps, m);
+        J_out[blockIdx.x] = stored ? m - 1 : cal_J_gpu(rho, mb, eps, m);
     }
 }
 
@@ -1592,9 +1598,7 @@ __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE))) voi
 //   PASS 1: v1 first pass -> x0, xN to xbuf, per-tile max to partial, or x at
 //           once where the wave's two maxima already give J = m - 1 (as
 //           k_filtered_fused): 65536 x 512, P = 8, J = 63: 506 to 324 us, one
-//           read of the rows (1.34 GB with the stores) instead of two. With J
-//           = 29 nothing is stored early: 502 to 497, from the second pass's
-//           order
+//           read of the rows (1.34 GB with the stores) instead of two
 //           (3 stores per tile).
 //   PASS 2: v1 second pass -> x0, xN from xbuf (one more DMA per tile into
 //           an LDS block, issued ahead of the sweep), x stored (M stores per
@@ -1631,21 +1635,39 @@ __global__ __launch_bounds__(Q * 32) __attribute__((amdgpu_waves_per_eu(WPE))) v
     int J0 = (VERSION == 2 || PASS == 2 || (GRD && PASS == 0)) ? Jp[p] : m0;
     constexpr bool LEFT = PASS == 2 && !GRD;
     const int stride = (int)gridDim.x;
-    // PASS 2 takes the tiles from the last one down: those rows are the ones
-    // that the first pass has left in the 256 MB last-level cache
-    auto tile_at = [&](int T) { return PASS == 2 ? n_tiles - 1 - T : T; };
+    // PASS 2 starts with the tiles of the last turn, each with its workgroup: the
+    // 256 MB last-level cache has their rows, and the L2 of this XCD the end of
+    // them (8192 x 400, P = 8, one turn, in reverse order: 66 against 64 us). Then
+    // the others from the last one down, as far as that cache helps (32768 x
+    // 400, 4 turns: 212 in their own order, 208; 65536 x 512, 8: 520, 508), in
+    // their own order above 12 turns (262144 x 128, 16: 654 against 662).
+    const int before = (n_tiles - 1) / stride * stride, ends = n_tiles - before;
+    const bool down = before < 12 * stride;
+    auto tile_at = [&](int T) {
+        return PASS != 2 ? T : T < ends ? before + T : down ? n_tiles - 1 - T : T - ends;
+    };
     // PASS 2: a turn's tile was stored by the first pass if the maximum that it
-    // left in partial is negative; the turns b, b + stride, ... of one lane each
+    // left in partial is negative; the turns b, b + stride, ... of one lane each.
+    // Where J of either partition is below m - 1 nothing was (k_compute_J): the
+    // ring then starts without waiting for the maxima (8192 x 400: 0.4 us).
     auto max_of = [&](int b) {
         const int T = b + l * stride;
         return partial[(size_t)tile_at(T < n_tiles ? T : 0) * Q + 2 * w];
     };
-    double max0 = LEFT ? max_of(blockIdx.x) : 0.0;
-    // PASS 1 with rho: from which tile maximum on this lane's partition takes
-    // the full correction at once
-    double from = PASS == 1 && rho ? rho[r0] : __builtin_nan("");
+    // PASS 1 with rho: the full_J_scale of the wave's two partitions, by scalar
+    // loads, which the ring's start does not wait for (8192 x 256, P = 8, one
+    // tile per CU: the solve 37.9 against 37.3 us)
+    double from[2] = {};
+    if (PASS == 1) {
+        const double* const r = rho ? rho : A;  // (without it unused, and any address does)
+        for (int k = 0; k < 2; ++k) {
+            int row, rows;
+            part_of(n_row, Q, 2 * w + k, row, rows);
+            from[k] = r[row];
+        }
+    }
     // loaded before the ring starts
-    asm volatile("" : "+v"(J0), "+v"(max0), "+v"(from));
+    asm volatile("" : "+v"(J0));
     // PASS 2: rows 4w..4w+3 of xbuf (x0, xN of partitions 2w, 2w+1), two
     // systems per lane, as the ring's sub-blocks
     const double* xsrc = xbuf + (size_t)(4 * w + (l >> 4)) * ld + 2 * (l & 15);
@@ -1657,9 +1679,10 @@ __global__ __launch_bounds__(Q * 32) __attribute__((amdgpu_waves_per_eu(WPE))) v
     auto left_of = [&](int b, double v) {
         return __ballot(b + l * stride < n_tiles && !__builtin_signbit(v));
     };
+    const bool some = LEFT && __ballot(J0 < m0 - 1) == 0;
     unsigned long long left = 0;
     auto after = [&](int T) {  // the turn that follows T here, n_tiles or more if none
-        if (!LEFT) return T + stride;
+        if (!some) return T + stride;
         while (!left) {
             tbase += 64 * stride;
             if (tbase >= n_tiles) return n_tiles;
@@ -1670,13 +1693,16 @@ __global__ __launch_bounds__(Q * 32) __attribute__((amdgpu_waves_per_eu(WPE))) v
         return tbase + b * stride;
     };
     int turn = blockIdx.x;
-    if (LEFT) {
-        left = left_of(tbase, max0);
+    if (some) {
+        left = left_of(tbase, max_of(tbase));
         turn = after(turn);
         if (turn >= n_tiles) return;
     }
     rg.prologue(tile_at(turn), dcnt0);
-    if (PASS == 1) from = full_J_from(from, m0, Q, eps_value, eps_direct);
+    // from which tile maximum on this lane's partition takes the full correction
+    const double v_full = PASS == 1 && rho ? full_J_from(l < 32 ? from[0] : from[1], m0, Q,
+                                                         eps_value, eps_direct)
+                                           : __builtin_nan("");
     bool first = true;
     for (int next; turn < n_tiles; turn = next) {
         const int tile = tile_at(turn);
@@ -1808,7 +1834,7 @@ __global__ __launch_bounds__(Q * 32) __attribute__((amdgpu_waves_per_eu(WPE))) v
             const double v = group_max(fmax(fabs(x0), fabs(xN)), S);
             // both partitions of the wave in full already: x now, and the sign
             // of the maxima says so
-            store = __ballot(!full_J(from, v)) == 0;
+            store = __ballot(!full_J(v_full, v)) == 0;
             if (sl == 0) partial[(size_t)tile * Q + p] = store ? -fabs(v) : fabs(v);
             Jf = m - 1;
             if (!store) {
