@@ -25,6 +25,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <system_error>
 #include <thread>
@@ -1269,6 +1270,9 @@ struct ftd_heat {
     } filt[3];
     int use_fused = 1;
     int fuse_rhs = 0;  // the fused z sweep forms the rhs (no k_rhs_z pass) this step
+    // one call at a time packs or overwrites rhs: a field may be read by several
+    // threads at once, and while another one steps
+    std::mutex calls;
     char* pinned = nullptr;  // ftd_heat_field's staging (kCopyThreads x 2 slots), on first use
     hipEvent_t slot[16] = {};  // and its slots' events
     char plan[256] = "";  // how the last enqueued step ran each sweep (ftd_heat_last_plan)
@@ -2067,6 +2071,7 @@ ftd_status ftd_heat_destroy(ftd_heat* h) {
 // periodic wrap, Dirichlet ghosts (main.cpp:45-49)
 ftd_status ftd_heat_init(ftd_heat* h) {
     if (!h) return herr(FTD_ERR_INVALID, "null handle");
+    const std::lock_guard<std::mutex> one(h->calls);
     const int nx1 = h->g.nx1, ny1 = h->g.ny1, nz1 = h->nz + 2;
     std::vector<double> f((size_t)nx1 * ny1 * nz1);
     for (int k = 0; k < nz1; ++k)
@@ -2101,6 +2106,7 @@ ftd_status ftd_heat_init(ftd_heat* h) {
 // time.
 ftd_status ftd_heat_step(ftd_heat* h, int nsteps, int use_graph) {
     if (!h) return herr(FTD_ERR_INVALID, "null handle");
+    const std::lock_guard<std::mutex> one(h->calls);
     for (int t = 0; t < nsteps;) {
         const bool last = t == nsteps - 1;
         int done = 1;
@@ -2164,6 +2170,7 @@ ftd_status ftd_heat_set_fused(ftd_heat* h, int enable) {
 // copies the field with ghosts ((nz+2)(ny+2)(nx+2), x fastest) to host memory
 ftd_status ftd_heat_field(ftd_heat* h, double* host_out) {
     if (!h || !host_out) return herr(FTD_ERR_INVALID, "null argument");
+    const std::lock_guard<std::mutex> one(h->calls);
     const Dims& g = h->g;
     // packed into rhs (free between steps), then copied linearly
     const size_t lines = (size_t)g.ny1 * (h->nz + 2);

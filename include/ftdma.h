@@ -337,7 +337,7 @@ ftd_status ftd_heat_destroy(ftd_heat* h);
 ftd_status ftd_heat_init(ftd_heat* h);
 
 /* nsteps time steps (solve_theta.cpp:92-334); use_graph != 0 replays hipGraphs
- * of one step, and in calls of 32 more steps of 8. Waits for the last step. */
+ * of one step and, from a call of more than 32 on, of 8. Waits for the last step. */
 ftd_status ftd_heat_step(ftd_heat* h, int nsteps, int use_graph);
 
 /* Extension: fused sweeps on (default) or off. Where a sweep's coefficients
@@ -359,7 +359,10 @@ ftd_status ftd_heat_set_fused(ftd_heat* h, int enable);
  * field. A captured step is dropped. */
 ftd_status ftd_heat_set_plan(ftd_heat* h, int dir, int rows_per_lane, int systems_per_tile);
 
-/* the field with ghosts, (nz+2)(ny+2)(nx+2) doubles, x fastest, to host memory */
+/* the field with ghosts, (nz+2)(ny+2)(nx+2) doubles, x fastest, to host memory.
+ * Safe beside another thread's ftd_heat_field, ftd_heat_l2, ftd_heat_step or
+ * ftd_heat_init on the same handle: these run one at a time, so the field is
+ * that before or after such a call. */
 ftd_status ftd_heat_field(ftd_heat* h, double* host_out);
 
 /* L2 error at t = steps * dt, as main.cpp:59-81 prints it */
