@@ -117,18 +117,31 @@ __global__ void k_periodic(double* __restrict__ th, Dims g, int face) {
 // 2-D copy to pageable memory goes line by line (100 steps and the field:
 // 35.3 against 6.0 ms at 64^3, 485 against 37.6 at 256^3). One workgroup per
 // line; the pack itself is a copy of the field on the device.
+// (A grid holds fewer than 2^32 threads: above kLinesGrid lines it comes round again.)
+constexpr size_t kLinesGrid = (size_t)1 << 24;
+
 template <bool PACK>
 __global__ __launch_bounds__(128) void k_lines(double* __restrict__ field,
-                                               double* __restrict__ packed, Dims g) {
-    const size_t line = blockIdx.x;
-    double* const f = field + kOrigin + line * g.px;
-    double* const p = packed + line * g.nx1;
-    for (int i = threadIdx.x; i < g.nx1; i += 128) {
-        if (PACK)
-            p[i] = f[i];
-        else
-            f[i] = p[i];
+                                               double* __restrict__ packed, Dims g,
+                                               size_t lines) {
+    for (size_t line = blockIdx.x; line < lines; line += gridDim.x) {
+        double* const f = field + kOrigin + line * g.px;
+        double* const p = packed + line * g.nx1;
+        for (int i = threadIdx.x; i < g.nx1; i += 128) {
+            if (PACK)
+                p[i] = f[i];
+            else
+                f[i] = p[i];
+        }
     }
+}
+
+template <bool PACK>
+hipError_t launch_lines(double* field, double* packed, const Dims& g, hipStream_t st) {
+    const size_t lines = (size_t)g.ny1 * (g.nz + 2);
+    hipLaunchKernelGGL((k_lines<PACK>), dim3((unsigned)std::min(lines, kLinesGrid)), dim3(128), 0,
+                       st, field, packed, g, lines);
+    return hipGetLastError();
 }
 
 struct Stencil {
@@ -2083,9 +2096,7 @@ ftd_status ftd_heat_init(ftd_heat* h) {
     // rhs is free between steps: every step writes its cells before reading them
     HH(hipMemcpyAsync(h->rhs, f.data(), sizeof(double) * f.size(), hipMemcpyHostToDevice,
                       h->stream));
-    hipLaunchKernelGGL((k_lines<false>), dim3((unsigned)(ny1 * nz1)), dim3(128), 0, h->stream,
-                       h->th, h->rhs, g);
-    HH(hipGetLastError());
+    HH(launch_lines<false>(h->th, h->rhs, g, h->stream));
     const dim3 b2(16, 16);
     for (int d = 0; d < 3; ++d) {
         if (!h->periodic[d]) continue;
@@ -2174,9 +2185,7 @@ ftd_status ftd_heat_field(ftd_heat* h, double* host_out) {
     const Dims& g = h->g;
     // packed into rhs (free between steps), then copied linearly
     const size_t lines = (size_t)g.ny1 * (h->nz + 2);
-    hipLaunchKernelGGL((k_lines<true>), dim3((unsigned)lines), dim3(128), 0, h->stream, h->th,
-                       h->rhs, g);
-    HH(hipGetLastError());
+    HH(launch_lines<true>(h->th, h->rhs, g, h->stream));
     HH(copy_to_host(h, h->rhs, host_out, sizeof(double) * lines * g.nx1));
     return FTD_OK;
 }
