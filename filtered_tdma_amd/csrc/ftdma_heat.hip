@@ -27,14 +27,13 @@
 #include <cstring>
 #include <mutex>
 #include <string>
-#include <system_error>
-#include <thread>
 #include <type_traits>
 #include <vector>
 
 #include "../../include/ftdma.h"
 #include "ftdma_device.h"
 #include "ftdma_kernels.h"
+#include "ftdma_threads.h"
 #include "ftdma_xcd.h"
 
 namespace {
@@ -1873,20 +1872,9 @@ hipError_t copy_to_host(ftd_heat* h, const double* src, double* dst, size_t byte
     int dev = 0;
     if (bytes >= kCopyFrom && !known && hipGetDevice(&dev) == hipSuccess && copy_ring(h)) {
         hipError_t got[kCopyThreads];
-        std::thread th[kCopyThreads];
-        for (int t = 1; t < kCopyThreads; ++t) {
-            auto part = [=, &got] {
-                got[t] = copy_pieces(h, dev, t, (const char*)src, (char*)dst, bytes);
-            };
-            try {
-                th[t] = std::thread(part);
-            } catch (const std::system_error&) {
-                part();  // no thread to be had: here
-            }
-        }
-        got[0] = copy_pieces(h, dev, 0, (const char*)src, (char*)dst, bytes);
-        for (int t = 1; t < kCopyThreads; ++t)
-            if (th[t].joinable()) th[t].join();
+        ftd::run_parts<kCopyThreads>([&](int t) {
+            got[t] = copy_pieces(h, dev, t, (const char*)src, (char*)dst, bytes);
+        });
         e = hipStreamSynchronize(h->stream);
         for (int t = 0; t < kCopyThreads; ++t)
             if (got[t] != hipSuccess) e = got[t];
