@@ -1244,6 +1244,7 @@ ftd_status herr(ftd_status s, const std::string& m) {
 }  // namespace
 
 struct ftd_heat {
+    int device = 0;  // current when the handle was made
     Dims g{};
     int nz = 0;
     int rhs_kb = kRhsKB;  // planes per z run of k_rhs_z
@@ -1838,8 +1839,8 @@ bool copy_ring(ftd_heat* h) {
 }
 
 // pieces t, t + kCopyThreads, ... of src to dst; 0: all copied
-hipError_t copy_pieces(ftd_heat* h, int dev, int t, const char* src, char* dst, size_t bytes) {
-    hipError_t e = hipSetDevice(dev);
+hipError_t copy_pieces(ftd_heat* h, int t, const char* src, char* dst, size_t bytes) {
+    hipError_t e = hipSetDevice(h->device);
     const size_t n = (bytes + kCopyPiece - 1) / kCopyPiece;
     char* const ring = h->pinned + (size_t)2 * t * kCopyPiece;
     auto len = [&](size_t k) { return std::min(kCopyPiece, bytes - k * kCopyPiece); };
@@ -1860,6 +1861,21 @@ hipError_t copy_pieces(ftd_heat* h, int dev, int t, const char* src, char* dst, 
     return e;
 }
 
+// The handle's device is the calling thread's current one meanwhile: a thread
+// that reads a field may have another (a new thread has device 0), and the pack
+// and the ring's events belong to the handle's.
+struct OnDevice {
+    int back = -1;
+    explicit OnDevice(int dev) {
+        int cur = dev;
+        if (hipGetDevice(&cur) == hipSuccess && cur != dev && hipSetDevice(dev) == hipSuccess)
+            back = cur;
+    }
+    ~OnDevice() {
+        if (back >= 0) (void)hipSetDevice(back);
+    }
+};
+
 // src (device) to dst (host), after the work queued on the handle's stream;
 // waits for it
 hipError_t copy_to_host(ftd_heat* h, const double* src, double* dst, size_t bytes) {
@@ -1869,11 +1885,10 @@ hipError_t copy_to_host(ftd_heat* h, const double* src, double* dst, size_t byte
     const bool known = hipPointerGetAttributes(&at, dst) == hipSuccess &&
                        at.type != hipMemoryTypeUnregistered;
     (void)hipGetLastError();
-    int dev = 0;
-    if (bytes >= kCopyFrom && !known && hipGetDevice(&dev) == hipSuccess && copy_ring(h)) {
+    if (bytes >= kCopyFrom && !known && copy_ring(h)) {
         hipError_t got[kCopyThreads];
         ftd::run_parts<kCopyThreads>([&](int t) {
-            got[t] = copy_pieces(h, dev, t, (const char*)src, (char*)dst, bytes);
+            got[t] = copy_pieces(h, t, (const char*)src, (char*)dst, bytes);
         });
         e = hipStreamSynchronize(h->stream);
         for (int t = 0; t < kCopyThreads; ++t)
@@ -1970,6 +1985,7 @@ ftd_status ftd_heat_create(ftd_heat** out, int nx, int ny, int nz, const int* pa
     }
     h->kind = kind;
     h->dt = dt;
+    (void)hipGetDevice(&h->device);
     const double ddx = 2.0 / nx, ddy = 2.0 / ny, ddz = 2.0 / nz;
     const double bx = dt / (2.0 * ddx * ddx), by = dt / (2.0 * ddy * ddy), bz = dt / (2.0 * ddz * ddz);
     h->s = Stencil{bx, -2.0 * bx, bx, by, -2.0 * by, by, bz, -2.0 * bz, bz, dt * 3.0 * kPi * kPi};
@@ -2170,6 +2186,7 @@ ftd_status ftd_heat_set_fused(ftd_heat* h, int enable) {
 ftd_status ftd_heat_field(ftd_heat* h, double* host_out) {
     if (!h || !host_out) return herr(FTD_ERR_INVALID, "null argument");
     const std::lock_guard<std::mutex> one(h->calls);
+    const OnDevice on(h->device);
     const Dims& g = h->g;
     // packed into rhs (free between steps), then copied linearly
     const size_t lines = (size_t)g.ny1 * (h->nz + 2);
