@@ -33,6 +33,7 @@
 #include "../../include/ftdma.h"
 #include "ftdma_device.h"
 #include "ftdma_kernels.h"
+#include "ftdma_lanes.h"
 #include "ftdma_threads.h"
 #include "ftdma_xcd.h"
 
@@ -286,8 +287,9 @@ __device__ __forceinline__ void adi_row(bool first, bool last, double sa, double
 // A cell of a lane as a base that is the same for the whole wave (the first
 // lane's cell) and the lane's byte offset from it: with a uniform row index the
 // row's address is then scalar arithmetic, and the load takes the offset from
-// one register (the lanes of a wave hold consecutive systems, a few lines or
-// planes at most, so 32 bits hold it).
+// one register. The lanes of a wave hold consecutive systems, on one line or
+// plane or a few: where 32 bits do not hold that (planes of 4 GiB), the sweep is
+// not planned (lanes_fit).
 template <typename T>
 struct LaneCell {
     T* base;
@@ -1441,13 +1443,20 @@ int rhs_planes(int nx, int ny, int nz) {
     return kb;
 }
 
+// LaneCell's offsets in the sweep along d = 1 (y) or 2 (z)
+bool lanes_fit(const ftd_heat* h, int d) {
+    const size_t line = sizeof(double) * (size_t)h->g.px;
+    return ftd::lane_offsets_fit(h->g.nx, d == 2 ? line : line * h->g.ny1);
+}
+
 void plan_fused(ftd_heat* h, int d, int N, int n_sys, int rows_per_lane = 0,
                 int systems_per_tile = 0) {
     ftd_heat::Fused f;
     const int P = h->parts[d];
     // with one caller partition every kind solves alike (the filtered kinds'
     // single-partition solve is the exact one), so their sweeps fuse too
-    if ((h->kind != FTD_KIND_PASCAL && P != 1) || h->periodic[d] || N < 3 || n_sys < 1) {
+    if ((h->kind != FTD_KIND_PASCAL && P != 1) || h->periodic[d] || N < 3 || n_sys < 1 ||
+        (d > 0 && !lanes_fit(h, d))) {
         h->fused[d] = f;
         return;
     }
@@ -1510,7 +1519,8 @@ void plan_filt(ftd_heat* h, int d) {
     const int Q = h->parts[d], N = d == 2 ? h->nz : h->g.ny;
     const int n_sys = h->g.nx * (d == 2 ? h->g.ny : h->nz);
     h->filt[d] = f;
-    if (d == 0 || h->kind == FTD_KIND_PASCAL || Q < 2 || Q > 16 || h->periodic[d] || n_sys < 1)
+    if (d == 0 || h->kind == FTD_KIND_PASCAL || Q < 2 || Q > 16 || h->periodic[d] || n_sys < 1 ||
+        !lanes_fit(h, d))
         return;
     const int m_max = (N + Q - 1) / Q, m_min = N / Q;
     if (m_max > 64 || m_min < 3) return;
