@@ -11,7 +11,7 @@ namespace ftd {
 // `pitch` bytes on: a line in the z sweep, a plane in the y sweep.
 inline bool lane_offsets_fit(int nx, size_t pitch) {
     const size_t runs = (63 + (size_t)nx - 1) / nx;  // crossed by 64 systems at most
-    return runs * pitch + sizeof(double) * ((size_t)nx - 1) <= UINT32_MAX;
+    return runs * pitch + sizeof(double) * (size_t)(nx < 64 ? nx : 64) <= UINT32_MAX;
 }
 
 }  // namespace ftd
