@@ -535,7 +535,10 @@ __device__ __forceinline__ void adi_solve_lane(int Q, int q, int cnt, int S, int
     lds[(2 * q) * S + sl] = d0;
     lds[(2 * q + 1) * S + sl] = dN;
     __syncthreads();
-    if (q == 0) {
+    // partition 0's wave, and of the table held by lanes (SPAN 2, 4) all of it:
+    // a reduced row may be in a lane of another partition, whose register may be
+    // moved while it is off. The lanes of one system read and write the same.
+    if ((SPAN == 0 ? q : __builtin_amdgcn_readfirstlane(q)) == 0) {
         // the reduced rows 4 at a time: their values are read into registers
         // first, so the serial chain is the arithmetic, not a round trip
         // through LDS per row
