@@ -29,6 +29,7 @@
 
 #include "../../include/ftdma.h"
 #include "ftdma_device.h"
+#include "ftdma_fft.h"
 #include "ftdma_kernels.h"
 #include "ftdma_xcd.h"
 
@@ -38,8 +39,7 @@ struct ftd_poisson {
     hipStream_t stream = nullptr;  // the caller's
     // plans of lines of nxh modes back to back (ftd_solve_complex's layout) and
     // of lines of `pitch` modes where that is another layout
-    hipfftHandle fwd[2] = {0, 0}, bwd[2] = {0, 0};
-    int have_fwd[2] = {0, 0}, have_bwd[2] = {0, 0};
+    ftd::FftPair fft[2];
     double* A = nullptr;    // [nz][nm] coefficients, built once
     double* B = nullptr;
     double* C = nullptr;
@@ -361,23 +361,9 @@ __global__ __launch_bounds__(kModeThreads, 3) void k_mode_solve(double* __restri
 // takes about 13 ms to make: create makes the one that the step uses,
 // ftd_poisson_solver the other, since a solver has to be asked for to be tuned
 ftd_status fft_plans(ftd_poisson* p, int k) {
-    if (p->have_fwd[k] && p->have_bwd[k]) return FTD_OK;
-    const int w = k ? p->pitch : p->nxh;
-    int n2[2] = {p->ny, p->nx}, real[2] = {p->ny, p->nx}, modes[2] = {p->ny, w};
-    const int dr = p->nx * p->ny, dm = w * p->ny;
-    if (!p->have_fwd[k] &&
-        hipfftPlanMany(&p->fwd[k], 2, n2, real, 1, dr, modes, 1, dm, HIPFFT_D2Z, p->nz) !=
-            HIPFFT_SUCCESS)
-        return perr(FTD_ERR_HIP, "hipfftPlanMany (D2Z) failed");
-    p->have_fwd[k] = 1;
-    if (hipfftPlanMany(&p->bwd[k], 2, n2, modes, 1, dm, real, 1, dr, HIPFFT_Z2D, p->nz) !=
-        HIPFFT_SUCCESS)
-        return perr(FTD_ERR_HIP, "hipfftPlanMany (Z2D) failed");
-    p->have_bwd[k] = 1;
-    if (hipfftSetStream(p->fwd[k], p->stream) != HIPFFT_SUCCESS ||
-        hipfftSetStream(p->bwd[k], p->stream) != HIPFFT_SUCCESS)
-        return perr(FTD_ERR_HIP, "hipfftSetStream failed");
-    return FTD_OK;
+    const char* failed =
+        ftd::fft_make(p->fft[k], p->nx, p->ny, p->nz, k ? p->pitch : p->nxh, p->stream);
+    return failed ? perr(FTD_ERR_HIP, failed) : FTD_OK;
 }
 
 ftd_status poisson_spectral(ftd_poisson* p) {
@@ -387,7 +373,7 @@ ftd_status poisson_spectral(ftd_poisson* p) {
         int Q, S;
         mode_shape(p->nz, Q, S);
         const int k = p->pitch != p->nxh;
-        PF(hipfftExecD2Z(p->fwd[k], p->rhs, reinterpret_cast<hipfftDoubleComplex*>(p->hat)));
+        PF(hipfftExecD2Z(p->fft[k].fwd, p->rhs, reinterpret_cast<hipfftDoubleComplex*>(p->hat)));
         int lgS = 0;
         while ((1 << lgS) < S) ++lgS;
         const int n = p->ny * p->pitch;
@@ -398,17 +384,17 @@ ftd_status poisson_spectral(ftd_poisson* p) {
         hipLaunchKernelGGL(k_mode_solve, dim3((n + S - 1) / S), dim3(S * Q), mode_lds(p->nz, Q, S),
                            p->stream, p->hat, p->nxh, p->pitch, p->ny, p->nz, Q, lgS, p->coef);
         PH(hipGetLastError());
-        PF(hipfftExecZ2D(p->bwd[k], reinterpret_cast<hipfftDoubleComplex*>(p->hat), p->rhs));
+        PF(hipfftExecZ2D(p->fft[k].bwd, reinterpret_cast<hipfftDoubleComplex*>(p->hat), p->rhs));
         return FTD_OK;
     }
     ftd_status s = fft_plans(p, 0);
     if (s != FTD_OK) return s;
-    PF(hipfftExecD2Z(p->fwd[0], p->rhs, reinterpret_cast<hipfftDoubleComplex*>(p->hat)));
+    PF(hipfftExecD2Z(p->fft[0].fwd, p->rhs, reinterpret_cast<hipfftDoubleComplex*>(p->hat)));
     hipLaunchKernelGGL(k_pin_zero_mode, dim3(1), dim3(64), 0, p->stream, p->hat);
     PH(hipGetLastError());
     s = ftd_solve_complex(p->solver, p->A, p->B, p->C, p->hat);
     if (s != FTD_OK) return perr(s, std::string("z solve: ") + ftd_last_error_string());
-    PF(hipfftExecZ2D(p->bwd[0], reinterpret_cast<hipfftDoubleComplex*>(p->hat), p->rhs));
+    PF(hipfftExecZ2D(p->fft[0].bwd, reinterpret_cast<hipfftDoubleComplex*>(p->hat), p->rhs));
     return FTD_OK;
 }
 
@@ -525,10 +511,7 @@ ftd_status ftd_poisson_create(ftd_poisson** out, int nx, int ny, int nz, double 
 
 ftd_status ftd_poisson_destroy(ftd_poisson* p) {
     if (!p) return FTD_OK;
-    for (int k = 0; k < 2; ++k) {
-        if (p->have_fwd[k]) hipfftDestroy(p->fwd[k]);
-        if (p->have_bwd[k]) hipfftDestroy(p->bwd[k]);
-    }
+    for (ftd::FftPair& f : p->fft) ftd::fft_free(f);
     if (p->solver) ftd_destroy(p->solver);
     for (double* b : {p->A, p->B, p->C, p->rhs, p->hat, p->met, p->coef})
         if (b) hipFree(b);

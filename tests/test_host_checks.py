@@ -10,7 +10,7 @@ CPP = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="g++ is not installed")
-@pytest.mark.parametrize("name", ["parts_check", "lanes_check"])
+@pytest.mark.parametrize("name", ["parts_check", "lanes_check", "fft_check"])
 def test_host_check(name, tmp_path):
     exe = str(tmp_path / name)
     cmd = ["g++", "-std=c++17", "-O1", "-Wall", "-pthread", "-D__HIP_PLATFORM_AMD__",
