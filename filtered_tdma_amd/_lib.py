@@ -25,7 +25,7 @@ EXPORTS = (
     "ftd_heat_l2", "ftd_heat_last_step_ms", "ftd_heat_last_error_string", "ftd_heat_set_fused",
     "ftd_heat_set_plan", "ftd_heat_last_plan",
     "ftd_poisson_create", "ftd_poisson_destroy", "ftd_poisson_solver", "ftd_poisson_solve",
-    "ftd_poisson_solve_rhs", "ftd_poisson_last_ms", "ftd_poisson_last_error_string",
+    "ftd_poisson_last_path", "ftd_poisson_solve_rhs", "ftd_poisson_last_ms", "ftd_poisson_last_error_string",
     "ftd_poisson_set_profiling",
 )
 
@@ -107,6 +107,8 @@ def load() -> ctypes.CDLL:
     L.ftd_poisson_destroy.argtypes = [vp]
     L.ftd_poisson_solver.argtypes = [vp]
     L.ftd_poisson_solver.restype = vp
+    L.ftd_poisson_last_path.argtypes = [vp]
+    L.ftd_poisson_last_path.restype = ctypes.c_char_p
     L.ftd_poisson_solve.argtypes = [vp, dp, dp, dp, dp, c_double]
     L.ftd_poisson_solve_rhs.argtypes = [vp, dp, dp]
     L.ftd_poisson_set_profiling.argtypes = [vp, c_int]

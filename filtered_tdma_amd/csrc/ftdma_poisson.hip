@@ -527,6 +527,10 @@ ftd_handle* ftd_poisson_solver(ftd_poisson* p) {
     return p->solver;
 }
 
+const char* ftd_poisson_last_path(const ftd_poisson* p) {
+    return p ? ftd_last_path(p->solver) : "none";
+}
+
 ftd_status ftd_poisson_solve(ftd_poisson* p, double* U, double* V, double* W, double* P, double dt) {
     if (!p) return perr(FTD_ERR_INVALID, "null handle");
     if (!U || !V || !W || !P) return perr(FTD_ERR_INVALID, "null field pointer");

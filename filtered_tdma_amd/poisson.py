@@ -62,7 +62,7 @@ class ChannelPoisson:
         _lib.check(_lib.load().ftd_set_j_mode(_lib.load().ftd_poisson_solver(self._h), int(mode)))
 
     def solver_path(self) -> str:
-        return _lib.load().ftd_last_path(_lib.load().ftd_poisson_solver(self._h)).decode()
+        return _lib.load().ftd_poisson_last_path(self._h).decode()
 
     def last_ms(self) -> float:
         return _lib.load().ftd_poisson_last_ms(self._h)

@@ -407,6 +407,11 @@ ftd_status ftd_poisson_destroy(ftd_poisson* p);
  * was made. */
 ftd_handle* ftd_poisson_solver(ftd_poisson* p);
 
+/* Extension (diagnostics): the kernel path of the last step's wall-normal solve
+ * (as ftd_last_path), without what a caller that means to change the solver
+ * needs: ftd_poisson_solver makes the FFT plans of the solve on arrays. */
+const char* ftd_poisson_last_path(const ftd_poisson* p);
+
 /* One pressure step (solve, :493-533): rhs = div(u*)/dt, FFT, wall-normal
  * solves with the (0,0) mode pinned, inverse FFT scaled by 1/(nx ny), then
  * P += dp and u -= dt grad dp (project_, :470-490). U, V, W, P are device
