@@ -1355,8 +1355,21 @@ namespace ftd {
 void handle_keep_thomas(ftd_handle* h) { h->keep_thomas = 1; }
 
 bool handle_is_plain(const ftd_handle* h, hipStream_t st) {
-    return h->P == 1 && h->stream == st && !h->t_M && !h->force_general && !h->no_stream &&
-           !h->profiling;
+    return h->P == 1 && h->stream == st && !h->t_M && !h->force_general && !h->no_stream;
+}
+
+hipError_t handle_time_begin(ftd_handle* h) {
+    return h->profiling ? hipEventRecord(h->ev0, h->stream) : hipSuccess;
+}
+
+hipError_t handle_time_end(ftd_handle* h) {
+    if (!h->profiling) return hipSuccess;
+    float ms = 0.0f;
+    hipError_t e = hipEventRecord(h->ev1, h->stream);
+    if (e == hipSuccess) e = hipEventSynchronize(h->ev1);
+    if (e == hipSuccess) e = hipEventElapsedTime(&ms, h->ev0, h->ev1);
+    if (e == hipSuccess) h->last_ms = ms;
+    return e;
 }
 
 void handle_note_path(ftd_handle* h, const char* path) {

@@ -176,11 +176,14 @@ namespace ftd {
 // one partition of up to 64 rows solved by plain Thomas at every batch size
 // (the heat step, whose fused sweeps are the same Thomas)
 void handle_keep_thomas(ftd_handle* h);
-// a handle of one caller partition whose tuning, stream and profiling are as
-// they were made (the pressure step then solves its modes itself), and the path
-// that such a caller's solve took (ftd_last_path)
+// a handle of one caller partition whose tuning and stream are as they were made
+// (the pressure step then solves its modes itself), the path that such a
+// caller's solve took (ftd_last_path), and its device time where the handle is
+// profiled (ftd_last_gpu_ms), around the launch
 bool handle_is_plain(const ftd_handle* h, hipStream_t st);
 void handle_note_path(ftd_handle* h, const char* path);
+hipError_t handle_time_begin(ftd_handle* h);
+hipError_t handle_time_end(ftd_handle* h);
 int handle_filtered_state(ftd_handle* h, int** J, const double** rho, double* eps_value,
                           int* eps_direct);
 }  // namespace ftd

@@ -368,7 +368,7 @@ ftd_status fft_plans(ftd_poisson* p, int k) {
 
 ftd_status poisson_spectral(ftd_poisson* p) {
     // the solver as it was made solves in k_mode_solve; one that the caller
-    // tuned, moved to another stream or times solves by itself
+    // tuned or moved to another stream solves by itself
     if (p->pitch && ftd::handle_is_plain(p->solver, p->stream)) {
         int Q, S;
         mode_shape(p->nz, Q, S);
@@ -381,9 +381,11 @@ ftd_status poisson_spectral(ftd_poisson* p) {
         std::snprintf(path, sizeof path, "pascal_modes M=%d T=%d S=%d Q=%d", kModeRows,
                       kModeThreads, S, Q);
         ftd::handle_note_path(p->solver, path);
+        PH(ftd::handle_time_begin(p->solver));
         hipLaunchKernelGGL(k_mode_solve, dim3((n + S - 1) / S), dim3(S * Q), mode_lds(p->nz, Q, S),
                            p->stream, p->hat, p->nxh, p->pitch, p->ny, p->nz, Q, lgS, p->coef);
         PH(hipGetLastError());
+        PH(ftd::handle_time_end(p->solver));
         PF(hipfftExecZ2D(p->fft[k].bwd, reinterpret_cast<hipfftDoubleComplex*>(p->hat), p->rhs));
         return FTD_OK;
     }

@@ -403,8 +403,9 @@ ftd_status ftd_poisson_destroy(ftd_poisson* p);
 /* The solver of the wall-normal systems (n_sys = (nx/2+1) ny complex, n_row
  * = nz), e.g. for ftd_set_j_mode or ftd_set_tuning. Owned by p. With one
  * partition and 17 to 512 rows the step solves the modes itself (ftd_last_path:
- * "pascal_modes") as long as this handle is tuned, profiled and streamed as it
- * was made. */
+ * "pascal_modes") as long as this handle is tuned and streamed as it was made;
+ * a tuned one (ftd_set_tuning, or ftd_autotune, which times real solves on
+ * arrays) solves on arrays, which is slower here. */
 ftd_handle* ftd_poisson_solver(ftd_poisson* p);
 
 /* Extension (diagnostics): the kernel path of the last step's wall-normal solve
