@@ -212,6 +212,12 @@ __global__ __launch_bounds__(256) void k_compute_J(const double* __restrict__ pa
 #define FTD_ST(v, p) (*(p) = (v))
 #endif
 
+// whether n values of T are whole 128-byte lines
+template <typename T>
+__device__ __forceinline__ bool whole_lines(int n) {
+    return n % (int)(128 / sizeof(T)) == 0;
+}
+
 template <bool NT, typename T>
 __device__ __forceinline__ double load_row(const T* p) {
     return (double)(NT ? FTD_LD(p) : *p);
@@ -352,10 +358,15 @@ __global__ __launch_bounds__(256) void k_thomas_cyclic_fused(const double* __res
 // ---------------------------------------------------------------------------
 // TC: storage type of A, B, C; TD: of the right-hand side Din. The solution
 // goes to X (float64), which may be Din itself when TD is double.
-// NT: row loads and stores marked nontemporal. Adjacent tiles run on one XCD
-// (xcd_tile), so a 128-byte line that two tiles share (rows that do not
-// start on lines, tiles under 16 systems) is fetched once, into that XCD's
-// L2, if both leave it there (NT = false). Measured at the launcher.
+// NT: row loads and stores marked nontemporal. Where tiles share 128-byte lines
+// (rows that do not start on lines, tiles under a line), adjacent ones run on
+// one XCD (xcd_tile), so that a shared line is fetched once, into that XCD's
+// L2, if both leave it there (NT = false). Measured at the launcher. Tiles of
+// whole lines run round the XCDs as they come: with a run of tiles each, the
+// XCDs would ask for columns the same power of two apart at one time (complex
+// 16384 x 256: 54 against 47.5 us; 131072 x 250: 249, 236; the other way only
+// complex 33024 x 256: 128, 132). Lanes of 16 rows keep the runs (65536 x 48:
+// 25.5 against 26.4).
 template <int M, int MAXT, bool CYCLIC, int PF, int WPE, typename TC, typename TD, int CSH = 0,
           bool NT = true>
 __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE))) void k_pascal_fused(
@@ -366,7 +377,8 @@ __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE))) voi
     const int t = threadIdx.x;
     const int sl = t & (S - 1);
     const int q = t >> lgS;
-    const int i_raw = xcd_tile(blockIdx.x, gridDim.x) * S + sl;
+    const bool apart = NT && M >= 32 && whole_lines<TC>(n_sys >> CSH) && whole_lines<TC>(S >> CSH);
+    const int i_raw = (apart ? (int)blockIdx.x : xcd_tile(blockIdx.x, gridDim.x)) * S + sl;
     const bool live = i_raw < n_sys;
     // dead lanes shadow the last system (of their parity when CSH = 1)
     const int i = live ? i_raw : n_sys - (1 << CSH) + (i_raw & ((1 << CSH) - 1));
@@ -1340,9 +1352,12 @@ __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE))) voi
                                                          double eps_value, int eps_direct,
                                                          int* __restrict__ Jsys,
                                                          const double* __restrict__ rho) {
-    // adjacent tiles on one XCD, for the 128-byte lines that they share (v2,
-    // 65537 x 512, P = 8: 433 to 408 us; 30001 x 200, P = 4, v1: 115 to 104)
-    const int blk = xcd_tile(blockIdx.x, gridDim.x);
+    // tiles that share 128-byte lines: adjacent ones on one XCD (v2, 65537 x 512,
+    // P = 8: 433 to 408 us; 30001 x 200, P = 4, v1: 115 to 104); others as they come
+    // (k_pascal_fused; v2, 65536 x 100, P = 5: 71.4 to 69.5)
+    const bool apart =
+        M >= 32 && whole_lines<double>(n_sys >> CSH) && whole_lines<double>((1 << lgS) >> CSH);
+    const int blk = apart ? (int)blockIdx.x : xcd_tile(blockIdx.x, gridDim.x);
     // PASS 2: nothing left where the first pass stored x
     if (PASS == 2 && !GRD && __builtin_signbit(partial[(size_t)blk * P])) return;
     extern __shared__ double lds[];
