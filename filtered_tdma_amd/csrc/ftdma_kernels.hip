@@ -1340,8 +1340,10 @@ __device__ __forceinline__ int learned_J_checked(const double (&a)[M], const dou
     return dropped_exceeds<M>(a, c, m, Jl, x0, xN, eps) ? (m - 1) | (1 << 16) : Jl;
 }
 
+// (16-row lanes, first pass: held to the registers of three waves per SIMD, 172
+// to 160; complex 40000 x 60, P = 4: 60.7 to 58.1 us, 56.7 before the early store)
 template <int M, int MAXT, int VERSION, int PASS, int PF, int WPE, int CSH, int GRD>
-__global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE))) void k_filtered_fused(const double* __restrict__ A,
+__global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(M == 16 && PASS == 1 ? 3 : WPE))) void k_filtered_fused(const double* __restrict__ A,
                                                          const double* __restrict__ B,
                                                          const double* __restrict__ C,
                                                          double* __restrict__ D, int n_sys,
@@ -1390,6 +1392,9 @@ __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE))) voi
     // PASS 3 features: max |a/b|, |c/b| over rows 1..m-1, raw d of rows 0
     // and m-1, max |d|
     double f_rho = 0.0, f_d0 = 0.0, f_dN = 0.0, f_dmax = 0.0;
+
+    // PASS 1 with rho: the partition's full_J_scale, asked for with the first rows
+    double scale = PASS == 1 && rho ? rho[r0] : __builtin_nan("");
 
 #pragma unroll
     for (int j = 0; j < PF && j < M; ++j) FTD_LOAD_ROW(j);
@@ -1448,7 +1453,7 @@ __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE))) voi
             d[j] = d[j] - cj * d[j + 1];
             if (VERSION == 1) {
                 a[j] = a[j] - cj * a[j + 1];
-                c[j] = -cj * c[j + 1];
+                if (PASS != 1) c[j] = -cj * c[j + 1];
             } else {
                 if (J >= 2 && j < J) {
                     // seed A[J]; with J == m-1 the first update (j = m-3)
@@ -1460,6 +1465,7 @@ __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE))) voi
             }
         }
     }
+    if (PASS == 1) asm volatile("" : "+v"(scale));  // (here by now: not asked for at its use)
     // pack_reduced: row 0 keeps d0, a0 (c0 coupling dropped)
     const double rr = 1.0 / (1.0 - a[1] * c[0]);
     const double d0p = rr * (d[0] - c[0] * d[1]);
@@ -1518,8 +1524,7 @@ __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE))) voi
             v = fmax(v, __shfl_xor(v, off, 64));
         // rho given: a tile whose own maxima already ask for the full
         // correction in every partition takes it here, and says so by the sign
-        const double from =
-            rho ? full_J_from(rho[r0], m, P, eps_value, eps_direct) : __builtin_nan("");
+        const double from = rho ? full_J_from(scale, m, P, eps_value, eps_direct) : scale;
         const bool now = __syncthreads_and(full_J(from, v)) != 0;
         if (sl < (1 << CSH))
             partial[((size_t)sl * gridDim.x + blk) * P + p] = now ? -fabs(v) : fabs(v);
@@ -1530,7 +1535,22 @@ __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE))) voi
             }
             return;
         }
-        Jf = m - 1;
+        // every row corrected from both sides (J = m - 1), from the last one up:
+        // the backward chain of c', which no other tile needs, goes along
+        // (8192 x 400, P = 8, complex, J < m - 1: this pass 36.4 against 35.1 us)
+        if (live) {
+            double cj = 0.0;
+#pragma unroll
+            for (int j = M - 1; j >= 0; --j) {
+                cj = j <= m - 3 ? -c[j] * cj : c[j];
+                if (j < m)
+                    FTD_ST(j == 0       ? x0
+                           : j == m - 1 ? xN
+                                        : (d[j] - a[j] * x0) - cj * xN,
+                           D + base + (size_t)j * ld);
+            }
+        }
+        return;
     }
 
     if (PASS == 3) {
