@@ -197,6 +197,25 @@ bool fused_of(int Q, int n_row, FusedShape& out) {
     return false;
 }
 
+// Whether plain Thomas takes a real, not periodic batch of one partition of up
+// to 64 rows. Above 32 rows a small batch waits for the chain of a lane's rows,
+// which 16-row partitions shorten (4096 x 64: 15.0 to 8.1 us, 66049 x 48: 38.5
+// to 25.1, 1024 x 48: 10.6 to 6.8); one that fills the chip many times over does
+// not (262144 x 64: 115 against 123). Between, where rows are whole lines, it is
+// how far the last round of one Thomas wave per SIMD (65536 systems) is filled;
+// us, Thomas against partitions, operands out of the caches:
+//   64 rows: 40960: 23.3, 21.6; 49152: 24.8, 26.0; 65536: 29.4, 36.3; 90112:
+//     46.2, 45.6; 98304: 48.0, 49.4; 114688: 51.0, 58.0
+//   48 rows: 49152: 21.4, 19.7; 57344: 22.7, 22.7; 65536: 24.1, 25.7; 98304:
+//     41.3, 38.6; 114688: 42.0, 44.8
+bool thomas_pays(int n_sys, int n_row) {
+    if (n_row <= 32 || n_sys >= 131072) return true;
+    if (n_sys % 16) return false;
+    const int last = (n_sys - 1) % 65536 + 1;
+    const bool second = n_sys > 65536;
+    return last >= (n_row > 48 ? (second ? 32768 : 49152) : (second ? 49152 : 57344));
+}
+
 // Partitions and tile of a real exact solve whose partitions the engine
 // chooses; out.M == 0: the long-system streamed kernel (Q and S set). Lines
 // drawn from a sweep over 512..131104 systems of 65..1024 rows; both sides of
@@ -285,13 +304,9 @@ ftd_status solve_exact(ftd_handle* h, double* A, double* B, double* C, double* D
     if (cyclic && n_row < 3) return fail(FTD_ERR_UNSUPPORTED, "periodic solve needs n_row >= 3");
     FusedShape fs;
     if (!h->force_general && !h->t_M && h->P == 1 && n_row >= 3 && ftd::thomas_fused_rows(n_row) &&
-        (csh || cyclic || h->keep_thomas || n_row <= 32 || n_sys >= 131072)) {
+        (csh || cyclic || h->keep_thomas || thomas_pays(n_sys, n_row))) {
         // one partition that fits a lane: plain (or Sherman-Morrison periodic)
-        // Thomas in registers, the reference's single-rank path. Above 32 rows
-        // (not periodic) only where the batch fills the chip many times over (262144 x 64: 115
-        // against 123 us); a smaller one waits for the chain of its rows, and
-        // 16-row partitions shorten it (4096 x 64: 15.0 to 8.1 us, 66049 x 48:
-        // 38.5 to 25.1, 1024 x 48: 11.1 to 8.0)
+        // Thomas in registers, the reference's single-rank path
         if (cyclic) {
             std::snprintf(h->path, sizeof h->path, "thomas_cyclic_fused M=%d",
                           ftd::thomas_fused_rows(n_row));
