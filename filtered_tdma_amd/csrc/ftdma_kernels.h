@@ -167,8 +167,8 @@ hipError_t launch_gen_filtered_final(const double* A, const double* C, double* D
 // For a caller inside the library that runs a filtered kind's sweeps itself
 // (the heat step's fused filtered z sweep): the handle's J per partition
 // (device), its column-0 bounds as set by ftd_set_rho (device, A_rho then
-// C_rho, n_row + 1 each; A_rho of a partition's first row holds the partition's
-// full_J_scale) and its eps_ setting. An error for a handle that is
+// C_rho, n_row + 1 each; A_rho of the first row of a partition of up to 64 rows
+// holds the partition's full_J_scale) and its eps_ setting. An error for a handle that is
 // not a filtered kind over more than one partition, or that has learned J or
 // the guard switched on (those run on the handle's own solve).
 struct ftd_handle;
