@@ -236,13 +236,15 @@ bool thomas_pays(int n_sys, int n_row) {
 //  * above, 32-system tiles where rows are whole lines and the tiles fill the
 //    CUs (32768 x 512: 146 against 163), else 16 (66049 x 257: 170 against
 //    193; 2048 x 300: 12.7 against 15.8).
+//    Periodic ones of whole lines keep 64-row lanes, half the periodic reduced
+//    rows (100000 x 300: 296 against 304; 16384 x 448: 65.4, 67.2).
 //  * 449..512 rows of whole 32-system tiles keep 8 partitions, which the
 //    streamed kernel runs (262144 x 512: 980 against 1018).
 //  * above 512 rows the streamed long-system kernel (66049 x 768: 562 against
 //    609; 131104 x 1024: 1081 against 1125); with fewer than two 16-system
 //    tiles per CU and up to 1024 rows, 32-row lanes (2048 x 768: 23.3 against
 //    26.7).
-bool own_shape(int n_sys, int n_row, FusedShape& out) {
+bool own_shape(int n_sys, int n_row, int cyclic, FusedShape& out) {
     if (n_row < 33) return false;  // caller: Thomas, or the general choice
     if (n_row <= 64)
         return shape_for(16, 512, (n_row + 15) / 16, n_row, n_sys <= 16384 ? 32 : 64, out);
@@ -257,6 +259,8 @@ bool own_shape(int n_sys, int n_row, FusedShape& out) {
     if (n_row > 448 && n_sys % 32 == 0) return shape_for(64, 256, 8, n_row, 32, out);
     if (n_row <= 256 && n_sys <= 8192)
         return shape_for(16, 512, (n_row + 15) / 16, n_row, n_sys <= 4096 ? 16 : 32, out);
+    if (cyclic && n_row > 256 && lines && n_sys >= 8192)
+        return shape_for(64, 256, (n_row + 63) / 64, n_row, 32, out);
     const int Q = (n_row + 31) / 32;
     const int S = n_row > 256         ? (lines && n_sys >= 8192 ? 32 : 16)
                   : n_sys <= 16384    ? 64
@@ -321,7 +325,7 @@ ftd_status solve_exact(ftd_handle* h, double* A, double* B, double* C, double* D
     // or more rows in one than a lane holds). Without the streamed kernels
     // (set_tuning -2) the fused kernel runs the same partitions.
     const bool own = !h->force_general && !h->t_M && !csh && n_row >= 3 &&
-                     !caller_shape(h, n_row, fs) && own_shape(n_sys, n_row, fs);
+                     !caller_shape(h, n_row, fs) && own_shape(n_sys, n_row, cyclic, fs);
     const int Sl = own && !fs.M ? fs.S : 0;
     if (Sl && !h->no_stream) {
         std::snprintf(h->path, sizeof h->path, "pascal_stream M=64 Q=%d R=4 S=%d", fs.Q, Sl);
@@ -950,7 +954,7 @@ static ftd_status solve_f32_common(ftd_handle* h, const float* A, const float* B
     // the shapes of own_shape hold for FP32 storage as well (131072 x 256: 174
     // against 193 us with 64-row lanes, 131104 x 80: 58 against 78)
     const bool own = !h->t_M && h->n_row >= 6 && !caller_shape(h, h->n_row, fs) &&
-                     own_shape(h->n_sys, h->n_row, fs) && fs.M;
+                     own_shape(h->n_sys, h->n_row, 0, fs) && fs.M;
     if (h->n_row < 6 || !(own || pick_pascal(h, h->n_row, fs)))
         return fail(FTD_ERR_UNSUPPORTED, "no fused kernel holds this system for FP32 storage");
     if (h->profiling) FTD_HIP(hipEventRecord(h->ev0, h->stream));
