@@ -370,8 +370,8 @@ struct RowRhsZ {
 // registers out of the sweeps: a whole partition's loads fit in flight, four
 // waves per SIMD. At 256^3 the y sweep went from 58.7 to 50.9 us (5.3 TB/s), the
 // z sweep from 92.6 to 88 (its five stencil loads a row), at 64^3 y from 12.0 to
-// 9.2 and x from 17.6 to 14.5 (one wave's instructions on a part of the CUs); the
-// 256^3 x sweep stays at 77 (its LDS tile's copy-in, solve and copy-out).
+// 9.2 and x from 17.6 to 14.5 (one wave's instructions on a part of the CUs). The
+// 256^3 x sweep stayed at 77 by this; its tiles took it to 69 (plan_fused).
 //
 // Row j of partition q at tab[q * M + j]:
 //   inv   1 / (b - a c'_{j-1}); the rows that are divided by b (0 and 1 of a
@@ -1418,13 +1418,6 @@ hipError_t upload_table(ftd_heat* h, int d) {
     return hipMemcpy(h->coef[d], tab.data(), sizeof(AdiRow) * tab.size(), hipMemcpyHostToDevice);
 }
 
-// The partition count the sweep's solver picks for (N rows, P partitions):
-// P == 1 -> plain Thomas when N <= 64, else ceil(N / 64) internal
-// partitions (up to 16); P > 1 -> P. Then the fused sweep's shape, or off.
-// rows_per_lane (16, 32, 64; 0 = automatic) sets how many rows one lane
-// holds, and with one caller partition (P == 1) thereby the number of
-// internal partitions Q; systems_per_tile (power of two; 0 = automatic)
-// the systems of one workgroup (S * Q <= 256)
 // compute units of the current device (1 if it cannot be read)
 int device_cus() {
     int dev = 0, cus = 0;
@@ -1452,6 +1445,13 @@ bool lanes_fit(const ftd_heat* h, int d) {
     return ftd::lane_offsets_fit(h->g.nx, d == 2 ? line : line * h->g.ny1);
 }
 
+// The partition count the sweep's solver picks for (N rows, P partitions):
+// P == 1 -> plain Thomas when N <= 64, else ceil(N / 64) internal
+// partitions (up to 16); P > 1 -> P. Then the fused sweep's shape, or off.
+// rows_per_lane (16, 32, 64; 0 = automatic) sets how many rows one lane
+// holds, and with one caller partition (P == 1) thereby the number of
+// internal partitions Q; systems_per_tile (power of two; 0 = automatic)
+// the systems of one workgroup (S * Q <= 256 in x, adi_threads in y and z)
 void plan_fused(ftd_heat* h, int d, int N, int n_sys, int rows_per_lane = 0,
                 int systems_per_tile = 0) {
     ftd_heat::Fused f;
@@ -2130,8 +2130,8 @@ ftd_status ftd_heat_init(ftd_heat* h) {
 // nsteps ADI steps; use_graph != 0 captures one step into a hipGraph on first
 // use and replays it (the first step always runs eagerly so that every
 // solver scratch buffer exists before capture), and kGraphSteps steps into
-// another in a call of several times as many. Waits for the last step and records its device
-// time.
+// another in a call of several times as many. Waits for the last step and
+// records its device time.
 ftd_status ftd_heat_step(ftd_heat* h, int nsteps, int use_graph) {
     if (!h) return herr(FTD_ERR_INVALID, "null handle");
     const std::lock_guard<std::mutex> one(h->calls);

@@ -14,17 +14,18 @@
 //
 // The whole state of a system stays on the chip between its sweeps: 40 B/row,
 // where the lane-per-system Thomas that took such systems moves 72 and runs
-// all rows in one chain (4096 x 2048: 1160 us; here 75). Tiles share cache
+// all rows in one chain (4096 x 2048: 1160 us with the operands in the caches,
+// 1630 out of them; here 75 and 109). Tiles share cache
 // lines below 16 systems, and wherever n_sys is not a multiple of 16, so the
 // tiles that run at one time on one XCD are adjacent (xcd_tile), and their
 // loads and stores stay in its L2 until the neighbours have used the rest
 // of the line; whole-line tiles keep the nontemporal hint (NT). A ring of 4
 // row-steps is the fastest for that reason: what is in flight for 32
-// neighbouring tiles has to stay in one 4 MB L2 (4096 x 2048: 4 / 8 / 16
-// row-steps 108 / 120 / 124 us with both operands' sets out of the caches;
-// 131072 x 1024: 1115 / 1133 / 1208 us). What bounds it: lines fetched by
-// two tiles at S < 16 (2.5-3.3 TB/s), and at few tiles a lane's chain of
-// divisions, one wave per SIMD (1024 x 2048: 33 us).
+// neighbouring tiles has to stay in one 4 MB L2 (operands out of the caches,
+// 4096 x 2048: 4 / 8 / 16 row-steps 108 / 120 / 124 us; 131072 x 1024: 1115 /
+// 1133 / 1208 us). What bounds it: out of the caches, lines fetched by two
+// tiles at S < 16 (2.5-3.3 TB/s); at few tiles a lane's chain of divisions, one
+// wave per SIMD (1024 x 2048: 35 us in the caches, 47 out of them).
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
@@ -173,8 +174,10 @@ struct Forward<M> {
                                                double&) {}
 };
 
-// ns: row-steps per tile, the longest partition's rows rounded up to kStep, at
-// least R (a tile refills the ring for the next one) and at most M.
+// ns: row-steps per tile, the longest partition's rows, odd numbers too, and at
+// least R (a tile refills the ring for the next one); at most M. With an odd
+// ns the last pair's second read takes the slot that already holds, or will
+// hold, the next tile's first row, and drops it; only the first is refilled.
 template <int S, bool CYCLIC, bool NT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1))) void k_pascal_lines(
     const double* __restrict__ A, const double* __restrict__ B, const double* __restrict__ C,

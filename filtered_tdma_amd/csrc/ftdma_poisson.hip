@@ -466,7 +466,7 @@ ftd_status ftd_poisson_create(ftd_poisson** out, int nx, int ny, int nz, double 
     hC[0] = 0.0;
     // one caller partition: every kind solves exactly, over partitions of the
     // engine's choice. Lines of the spectra padded to whole 128-byte lines (the
-    // FFTs of 256^3 in 90 + 86 us where lines of 129 modes took 125 + 127),
+    // FFTs of 256^3 in 96 + 94 us where lines of 129 modes took 134 + 137),
     // unless the padding would be more than a fifth of them
     int mq, ms;
     mode_shape(nz, mq, ms);

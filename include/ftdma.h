@@ -75,8 +75,26 @@ ftd_status ftd_destroy(ftd_handle* h);
 
 /* TdmaBackendGPU::solve (tdma_backend_gpu.cu:35-46):
  * FILTERED -> solve_filtered_v1, FILTERED_V2 -> solve_filtered_v2,
- * PASCAL -> PaScaLTDMACUDA::solve; partitions == 1 -> plain Thomas, or above
- * 32 rows PaScaL over the engine's own partitions (exact to rounding). */
+ * PASCAL -> PaScaLTDMACUDA::solve; partitions == 1 -> exact.
+ *
+ * The exact solve's partitions are the caller's where partitions > 1 and a
+ * kernel holds them (at most 64 rows each; 16 of them, 32 of up to 32 rows).
+ * Otherwise the engine chooses, to rounding the same:
+ *   - one partition of up to 32 rows: plain Thomas; of 33 to 64 rows too if the
+ *     solve is periodic or complex, or the batch is large (131072 systems, or
+ *     from 49152 on some whole multiples of 16);
+ *   - up to 4096 rows (one system alone: 1024): PaScaL over partitions of 16
+ *     to 64 rows, also where the caller's (> 1) are longer than 64 rows;
+ *   - above: plain Thomas, or PaScaL over the caller's partitions, in place.
+ * Which partitions depends on n_row and n_sys, so a system can have other last
+ * bits in a batch of another n_sys. They depend on n_row alone after
+ * ftd_set_tuning with rows_per_lane and max_threads given (e.g. 32, 512, 0, 0 up
+ * to 1024 rows), at some cost in speed; ftd_last_path names them (Q=).
+ * PaScaL eliminates each partition by itself without pivoting, as the
+ * reference's ranks do: diagonally dominant systems always pass, a system
+ * that only the whole's Thomas elimination carries (a zero on the diagonal, for
+ * instance) may not. With one partition ftd_set_tuning(h, -1, 0, 0, 0) keeps
+ * plain Thomas for every n_row. */
 ftd_status ftd_solve(ftd_handle* h, double* A, double* B, double* C, double* D);
 
 /* PaScaLTDMACUDA::solve(A, B, C, D, n_sys, n_row) (pascal_tdma_cuda.hpp:28-29):
