@@ -468,7 +468,7 @@ ftd_status solve_filtered(ftd_handle* h, double* A, double* B, double* C, double
                                                    h->eps_value, h->eps_direct, nullptr, 0,
                                                    g ? nullptr : h->rho, st));
             FTD_LAUNCH(ftd::launch_compute_J((double*)h->partial.p, tiles, P, n_row, h->rho,
-                                             h->eps_value, h->eps_direct, csh, Jp, st));
+                                             h->eps_value, h->eps_direct, csh, Jp, st, true));
             FTD_LAUNCH(ftd::launch_filtered_stream(Ms, P, 1, 2, A, B, C, D, n_sys, n_row, cyclic, Jp,
                                                    (double*)h->xbuf.p, (double*)h->partial.p, ev,
                                                    ed, Js, g, nullptr, st));
@@ -515,7 +515,7 @@ ftd_status solve_filtered(ftd_handle* h, double* A, double* B, double* C, double
                                                   h->eps_direct, nullptr, 0, g ? nullptr : h->rho,
                                                   st));
             FTD_LAUNCH(ftd::launch_compute_J((double*)h->partial.p, tiles, P, n_row, h->rho,
-                                             h->eps_value, h->eps_direct, csh, Jp, st));
+                                             h->eps_value, h->eps_direct, csh, Jp, st, true));
             FTD_LAUNCH(ftd::launch_filtered_fused(fs.M, fs.T, 1, 2, A, B, C, D, n_sys, n_row, P, fs.S,
                                                   cyclic, csh, Jp, (double*)h->xbuf.p,
                                                   (double*)h->partial.p, ev, ed, Js, g, nullptr,

@@ -17,8 +17,10 @@ hipError_t launch_set_rho(const double* A, const double* B, const double* C, int
 // n_sys / 2 columns, and J is kept per parity (J[p], J[P + p])
 hipError_t launch_boundary_maxabs(const double* D, int n_sys, int n_row, int P, int csh,
                                   double* partial, int* n_tiles, hipStream_t st);
+// stored: the maxima are of a first pass given rho (launch_filtered_stream)
 hipError_t launch_compute_J(const double* partial, int n_tiles, int P, int n_row, const double* rho,
-                            double eps_value, int eps_direct, int csh, int* J, hipStream_t st);
+                            double eps_value, int eps_direct, int csh, int* J, hipStream_t st,
+                            bool stored = false);
 
 int pascal_fused_supported(int M, int maxt);
 size_t pascal_fused_lds(int Q, int S, int cyclic);

@@ -163,7 +163,9 @@ __global__ __launch_bounds__(256) void k_boundary_maxabs(const double* __restric
 }
 
 // J_p from rho (column-0 bounds of the partition's rows 1..m_p-1), the
-// reduced max_b and eps_p; one block per partition
+// reduced max_b and eps_p; one block per partition. STORED: maxima of a first
+// pass that may have stored tiles, with J = m - 1 and a negative maximum
+template <bool STORED>
 __global__ __launch_bounds__(256) void k_compute_J(const double* __restrict__ partial, int n_tiles,
                                                    int P, int n_row,
                                                    const double* __restrict__ A_rho,
@@ -171,34 +173,37 @@ __global__ __launch_bounds__(256) void k_compute_J(const double* __restrict__ pa
                                                    double eps_value, int eps_direct,
                                                    int* __restrict__ J_out) {
     __shared__ double red_b[4], red_r[4];
+    __shared__ int red_s[4];
     // block p + k * P: partition p of parity k (complex right-hand sides)
     const int p = blockIdx.x % P;
     const double* part = partial + (size_t)(blockIdx.x / P) * n_tiles * P;
     int s, m;
     part_of(n_row, P, p, s, m);
     double vb = 0.0, vr = 0.0;
-    // (a negative maximum: the first pass stored that tile with J = m - 1)
     bool stored = false;
     for (int t = threadIdx.x; t < n_tiles; t += 256) {
         const double v = part[(size_t)t * P + p];
-        stored |= __builtin_signbit(v);
-        vb = fmax(vb, fabs(v));
+        if (STORED) stored |= __builtin_signbit(v);
+        vb = fmax(vb, STORED ? fabs(v) : v);
     }
     for (int k = 1 + threadIdx.x; k < m; k += 256)
         vr = fmax(vr, fmax(fabs(A_rho[s + k]), fabs(C_rho[s + k])));
     vb = group_max(vb, 64);
     vr = group_max(vr, 64);
+    const int any = STORED ? __ballot(stored) != 0 : 0;
     if ((threadIdx.x & 63) == 0) {
         red_b[threadIdx.x >> 6] = vb;
         red_r[threadIdx.x >> 6] = vr;
+        if (STORED) red_s[threadIdx.x >> 6] = any;
     }
-    stored = __syncthreads_or(stored) != 0;
+    __syncthreads();
     if (threadIdx.x == 0) {
         double mb = fmax(fmax(red_b[0], red_b[1]), fmax(red_b[2], red_b[3]));
         double rho = fmax(fmax(red_r[0], red_r[1]), fmax(red_r[2], red_r[3]));
         double Nl = (double)(m * P);
         double eps = eps_direct ? eps_value : eps_value / (Nl * Nl);
-        J_out[blockIdx.x] = stored ? m - 1 : cal_J_gpu(rho, mb, eps, m);
+        const bool full = STORED && (red_s[0] | red_s[1] | red_s[2] | red_s[3]);
+        J_out[blockIdx.x] = full ? m - 1 : cal_J_gpu(rho, mb, eps, m);
     }
 }
 
@@ -2651,9 +2656,14 @@ hipError_t launch_boundary_maxabs(const double* D, int n_sys, int n_row, int P, 
 }
 
 hipError_t launch_compute_J(const double* partial, int n_tiles, int P, int n_row, const double* rho,
-                            double eps_value, int eps_direct, int csh, int* J, hipStream_t st) {
-    hipLaunchKernelGGL(k_compute_J, dim3(P << csh), dim3(256), 0, st, partial, n_tiles, P, n_row,
-                       rho, rho + (n_row + 1), eps_value, eps_direct, J);
+                            double eps_value, int eps_direct, int csh, int* J, hipStream_t st,
+                            bool stored) {
+    if (stored)
+        hipLaunchKernelGGL(k_compute_J<true>, dim3(P << csh), dim3(256), 0, st, partial, n_tiles,
+                           P, n_row, rho, rho + (n_row + 1), eps_value, eps_direct, J);
+    else
+        hipLaunchKernelGGL(k_compute_J<false>, dim3(P << csh), dim3(256), 0, st, partial, n_tiles,
+                           P, n_row, rho, rho + (n_row + 1), eps_value, eps_direct, J);
     return hipGetLastError();
 }
 
