@@ -236,8 +236,9 @@ bool thomas_pays(int n_sys, int n_row) {
 //  * above, 32-system tiles where rows are whole lines and the tiles fill the
 //    CUs (32768 x 512: 146 against 163), else 16 (66049 x 257: 170 against
 //    193; 2048 x 300: 12.7 against 15.8).
-//    Periodic ones of whole lines keep 64-row lanes, half the periodic reduced
-//    rows (100000 x 300: 296 against 304; 16384 x 448: 65.4, 67.2).
+//    Periodic ones of whole lines take 64-row lanes, half the periodic reduced
+//    rows, from 24576 systems on (100000 x 300: 296 against 304; 24576 x 400:
+//    88.7, 90.9; 11136 x 330: 46.4 against 45.4).
 //  * 449..512 rows of whole 32-system tiles keep 8 partitions, which the
 //    streamed kernel runs (262144 x 512: 980 against 1018).
 //  * above 512 rows the streamed long-system kernel (66049 x 768: 562 against
@@ -259,7 +260,7 @@ bool own_shape(int n_sys, int n_row, int cyclic, FusedShape& out) {
     if (n_row > 448 && n_sys % 32 == 0) return shape_for(64, 256, 8, n_row, 32, out);
     if (n_row <= 256 && n_sys <= 8192)
         return shape_for(16, 512, (n_row + 15) / 16, n_row, n_sys <= 4096 ? 16 : 32, out);
-    if (cyclic && n_row > 256 && lines && n_sys >= 8192)
+    if (cyclic && n_row > 256 && lines && n_sys >= 24576)
         return shape_for(64, 256, (n_row + 63) / 64, n_row, 32, out);
     const int Q = (n_row + 31) / 32;
     const int S = n_row > 256         ? (lines && n_sys >= 8192 ? 32 : 16)
